@@ -409,6 +409,54 @@ int hattn_hstate_step(float* states, int* counts, const void* q, const void* k, 
                       int dtype_v, int dtype_l, int dtype_beta, void* stream);
 
 /*
+ * Plans the cascades of up to n token inserts on the level counts counts [L]
+ * (host memory, advanced in place): cascades[t] is what hattn_hstate_step takes
+ * as `cascade` for token t (HState.cascade_weak / cascade_strong,
+ * recurrent.py:42-74).  Returns the number of tokens planned: fewer than n where
+ * a weak insert finds every level full or a level above its capacity (counts is
+ * then as before that insert).  Runs on the host only.
+ */
+int hattn_hstate_plan(int* counts, int L, int htype, int n, unsigned char* cascades);
+
+/*
+ * n decode steps in one launch: tokens t0 .. t0 + n - 1 of operands with a token
+ * axis, q, k [B, T, G, K], v, o [B, T, H, V], beta, g [B, T, H], l [B, T, H, L].
+ *
+ * Replaces the token loops around step_state / step_output
+ * (hattention/recurrent.py:169-216, kernel.py:555-570).  The state is read and
+ * written once.  cascades [n] and final_counts [L] (host memory) come from
+ * hattn_hstate_plan; final_counts are stored to counts (device) if that is not
+ * NULL.  o is written only with output != 0 (q, l, o may be NULL otherwise).
+ *
+ * Constraints: those of hattn_hstate_step, 1 <= n <= 256.
+ */
+int hattn_hstate_steps(float* states, int* counts, const void* q, const void* k, const void* v,
+                       const void* beta, const float* g, const void* l, void* o, int B, int T,
+                       int t0, int n, int G, int H, int K, int V, int L, int hstruct, int htype,
+                       const unsigned char* cascades, const int* final_counts, int output,
+                       int l2norm_qk, float scale, int dtype_qk, int dtype_v, int dtype_l,
+                       int dtype_beta, void* stream);
+
+/*
+ * What turns the final states of a chunkwise prefill of T tokens (T % 64 == 0)
+ * into an HState: levels 0 .. nlo - 1 rebuilt from the last chunk, the levels
+ * above that hold no token set to zero, and the level counts stored to counts
+ * (device, or NULL).
+ *
+ * Replaces hattention/kernel.py:378-465 `postprocess_prefill_hstate_`: MAMBA2 as
+ * hattn_mamba2_prefill_levels, GDELTA the recurrent form over the last 64 tokens
+ * from an empty state of nlo levels (:438-449) in one launch.
+ *
+ * k [B, T, G, K], v [B, T, H, V], beta (GDELTA), g [B, T, H]; constraints as for
+ * hattn_hstate_step and hattn_mamba2_prefill_levels.
+ */
+int hattn_hstate_prefill_levels(float* states, int* counts, const void* k, const void* v,
+                                const void* beta, const float* g, int B, int T, int G, int H,
+                                int K, int V, int L, int nlo, int hstruct, int htype,
+                                int l2norm_qk, int dtype_k, int dtype_v, int dtype_beta,
+                                void* stream);
+
+/*
  * Levels 0 .. nlo - 1 of the HState after a chunkwise prefill of T tokens
  * (T % 64 == 0), MAMBA2.
  *

@@ -12,6 +12,7 @@
 #include <cstring>
 #include <initializer_list>
 
+#include "hstate.h"
 #include "../../include/hattn.h"
 
 hipError_t hattn_mamba2_fwd_launch(const void* q, const void* k, const void* v, const float* g,
@@ -94,15 +95,12 @@ void hattn_mamba2_fwd_ws_summaries(void* ws, int B, int T, int H, int V, const f
 void hattn_mamba2_fwd_set_lookback(int spin_limit, int publish);
 const unsigned int* hattn_mamba2_fwd_status_word(const void* ws, int B, int T, int H, int V);
 
-hipError_t hattn_hstate_step_launch(float* states, int* counts, const void* q, const void* k,
-                                    const void* v, const void* beta, const float* g,
-                                    const void* l, void* o, int B, int G, int H, int K, int V,
-                                    int L, int gdn, int cascade, int strong, int update, int output,
-                                    int norm_qk, float scale, int dt_qk, int dt_v, int dt_l,
-                                    int dt_b, hipStream_t stream, int* unsupported);
+hipError_t hattn_hstate_steps_launch(HsArgs a, int B, int gdn, hipStream_t stream,
+                                     int* unsupported);
 hipError_t hattn_mamba2_prefill_levels_launch(float* states, const void* k, const void* v,
                                               const float* g, int B, int T, int G, int H, int K,
                                               int V, int L, int nlo, int dt_k, int dt_v,
+                                              unsigned int clear, const HsCounts& counts,
                                               hipStream_t stream, int* unsupported);
 
 size_t hattn_mamba2_layer_bwd_ws_bytes(int B, int T, int H, int L);
@@ -736,40 +734,201 @@ int hattn_gdn_chunkwise_bwd_fwd_ws(const void* q, const void* k, const void* v, 
                       fwd_workspace_bytes, true, stream);
 }
 
-int hattn_hstate_step(float* states, int* counts, const void* q, const void* k, const void* v,
-                      const void* beta, const float* g, const void* l, void* o, int B, int G,
-                      int H, int K, int V, int L, int hstruct, int htype, int cascade, int update,
-                      int output, int l2norm_qk, float scale, int dtype_qk, int dtype_v,
-                      int dtype_l, int dtype_beta, void* stream) {
+namespace {
+
+int hs_check(int B, int G, int H, int K, int V, int L, int hstruct, int htype) {
   if (B <= 0 || G <= 0 || H <= 0 || K <= 0 || V <= 0 || L <= 0)
     return fail(HATTN_ERR_VALUE, "non-positive dimension");
   if (H % G != 0) return fail(HATTN_ERR_VALUE, "G=%d does not divide H=%d", G, H);
   if (hstruct != HATTN_HSTRUCT_MAMBA2 && hstruct != HATTN_HSTRUCT_GDELTA)
     return fail(HATTN_ERR_NOT_IMPLEMENTED, "hstruct=%d", hstruct);
-  if (K > 256 || V % 16 != 0 || L > 32)
+  if (K > 256 || V % 16 != 0 || L > kHsMaxLevels)
     return fail(HATTN_ERR_NOT_IMPLEMENTED,
                 "K=%d V=%d L=%d (K <= 256, V a multiple of 16, L <= 32)", K, V, L);
   if (htype != HATTN_HTYPE_WEAK && htype != HATTN_HTYPE_STRONG)
     return fail(HATTN_ERR_VALUE, "htype=%d", htype);
+  return HATTN_OK;
+}
+
+int hs_cascade_check(int cascade, int L, int htype, int update) {
   if (htype == HATTN_HTYPE_WEAK && (cascade < 0 || cascade >= L))
     return fail(HATTN_ERR_VALUE, "cascade depth %d with %d levels (level overflow)", cascade, L);
   if (htype == HATTN_HTYPE_STRONG && update && (cascade < 1 || cascade > L))
     return fail(HATTN_ERR_VALUE, "strong cascade merge level %d with %d levels", cascade, L);
+  return HATTN_OK;
+}
+
+// The kernel's arguments for n tokens of operands [B, T, ...] from token t0 on.
+HsArgs hs_args(float* states, int* counts, const void* q, const void* k, const void* v,
+               const void* beta, const float* g, const void* l, void* o, int T, int t0, int n,
+               int G, int H, int K, int V, int L) {
+  HsArgs a{};
+  a.states = states;
+  a.counts = counts;
+  a.G = G; a.H = H; a.K = K; a.V = V; a.L = L; a.LA = L; a.T = n;
+  a.q_t = (long long)G * K; a.s_t = H; a.v_t = a.o_t = (long long)H * V; a.l_t = (long long)H * L;
+  a.q_b = T * a.q_t; a.s_b = T * a.s_t; a.v_b = a.o_b = T * a.v_t; a.l_b = T * a.l_t;
+  a.q = q; a.k = k; a.v = v; a.beta = beta; a.l = l; a.g = g; a.o = o;
+  a.t0 = t0;
+  a.scale = 1.f;
+  a.dt_qk = a.dt_v = a.dt_l = a.dt_b = HATTN_FP32;
+  return a;
+}
+
+int hs_launch(const HsArgs& a, int B, int hstruct, hipStream_t stream, const char* what) {
+  int unsupported = 0;
+  hipError_t e = hattn_hstate_steps_launch(a, B, hstruct == HATTN_HSTRUCT_GDELTA ? 1 : 0, stream,
+                                           &unsupported);
+  if (unsupported)
+    return fail(HATTN_ERR_NOT_IMPLEMENTED, "dtype codes qk=%d v=%d l=%d beta=%d", a.dt_qk, a.dt_v,
+                a.dt_l, a.dt_b);
+  return check_hip(e, what);
+}
+
+// The level counts after a prefill of T tokens (kernel.py:451-462): one token at
+// level 0, 2^(e-1) at level e >= 1 where bit e - 1 of T - 1 is set.
+void hs_prefill_counts(int T, int L, int nlo, int* counts, unsigned int* clear) {
+  *clear = 0;
+  for (int e = 0; e < L; ++e) {
+    counts[e] = e == 0 ? 1 : ((T - 1) >> (e - 1) & 1) ? 1 << (e - 1) : 0;
+    if (e >= nlo && counts[e] == 0) *clear |= 1u << e;
+  }
+}
+
+}  // namespace
+
+int hattn_hstate_step(float* states, int* counts, const void* q, const void* k, const void* v,
+                      const void* beta, const float* g, const void* l, void* o, int B, int G,
+                      int H, int K, int V, int L, int hstruct, int htype, int cascade, int update,
+                      int output, int l2norm_qk, float scale, int dtype_qk, int dtype_v,
+                      int dtype_l, int dtype_beta, void* stream) {
+  if (int st = hs_check(B, G, H, K, V, L, hstruct, htype)) return st;
+  if (int st = hs_cascade_check(cascade, L, htype, update)) return st;
   if (!states || (output && (!q || !l || !o)) ||
       (update && (!k || !v || !g || (hstruct == HATTN_HSTRUCT_GDELTA && !beta))))
     return fail(HATTN_ERR_VALUE, "null tensor pointer");
-  int unsupported = 0;
-  hipError_t e = hattn_hstate_step_launch(
-      states, counts, q, k, v, beta, g, l, o, B, G, H, K, V, L,
-      hstruct == HATTN_HSTRUCT_GDELTA ? 1 : 0, update ? cascade : 0,
-      (htype == HATTN_HTYPE_STRONG && update) ? 1 : 0,
-      update ? 1 : 0, output ? 1 : 0,
-      l2norm_qk ? 1 : 0, scale, dtype_qk, dtype_v, dtype_l, dtype_beta, (hipStream_t)stream,
-      &unsupported);
-  if (unsupported)
-    return fail(HATTN_ERR_NOT_IMPLEMENTED, "dtype codes qk=%d v=%d l=%d beta=%d", dtype_qk,
-                dtype_v, dtype_l, dtype_beta);
-  return check_hip(e, "hattn_hstate_step launch");
+  HsArgs a = hs_args(states, counts, q, k, v, beta, g, l, o, 1, 0, 1, G, H, K, V, L);
+  a.strong = htype == HATTN_HTYPE_STRONG;
+  a.update = update != 0;
+  a.output = output != 0;
+  a.norm = l2norm_qk != 0;
+  a.scale = scale;
+  a.casc[0] = (unsigned char)(update ? cascade : 0);
+  a.dt_qk = dtype_qk; a.dt_v = dtype_v; a.dt_l = dtype_l; a.dt_b = dtype_beta;
+  return hs_launch(a, B, hstruct, (hipStream_t)stream, "hattn_hstate_step launch");
+}
+
+int hattn_hstate_plan(int* counts, int L, int htype, int n, unsigned char* cascades) {
+  if (!counts || !cascades || L <= 0 || L > kHsMaxLevels) return 0;
+  for (int t = 0; t < n; ++t) {
+    long long c[kHsMaxLevels];
+    for (int e = 0; e < L; ++e) c[e] = counts[e];
+    int at = L;
+    bool stop = false;
+    if (htype == HATTN_HTYPE_STRONG) {
+      long long carry = 0;
+      for (int e = 0; e < L; ++e) {
+        const long long cap = 1LL << (e > 0 ? e - 1 : 0);
+        if (c[e] + carry > cap || e == 0) {
+          const long long x = c[e];
+          c[e] = carry;
+          carry = x;
+        } else {
+          c[e] += carry;
+          at = e;
+          break;
+        }
+      }
+    } else {
+      for (int e = 0; e < L && at == L && !stop; ++e) {
+        const long long cap = 1LL << e;
+        if (c[e] == cap) {
+          if (e + 1 >= L) stop = true;     // every level is full
+          else {
+            c[e + 1] += c[e];
+            c[e] = 0;
+          }
+        } else if (c[e] < cap) {
+          at = e;
+        } else {
+          stop = true;                     // a level above its capacity
+        }
+      }
+    }
+    if (stop) return t;
+    c[0] += 1;
+    for (int e = 0; e < L; ++e) counts[e] = (int)c[e];
+    cascades[t] = (unsigned char)at;
+  }
+  return n;
+}
+
+int hattn_hstate_steps(float* states, int* counts, const void* q, const void* k, const void* v,
+                       const void* beta, const float* g, const void* l, void* o, int B, int T,
+                       int t0, int n, int G, int H, int K, int V, int L, int hstruct, int htype,
+                       const unsigned char* cascades, const int* final_counts, int output,
+                       int l2norm_qk, float scale, int dtype_qk, int dtype_v, int dtype_l,
+                       int dtype_beta, void* stream) {
+  if (int st = hs_check(B, G, H, K, V, L, hstruct, htype)) return st;
+  if (t0 < 0 || n < 1 || T < n || t0 > T - n || n > kHsMaxTokens)
+    return fail(HATTN_ERR_VALUE, "tokens %d .. %d + %d of %d (at most %d at a time)", t0, t0, n, T,
+                kHsMaxTokens);
+  if (!states || !cascades || !final_counts || !k || !v || !g || (output && (!q || !l || !o)) ||
+      (hstruct == HATTN_HSTRUCT_GDELTA && !beta))
+    return fail(HATTN_ERR_VALUE, "null tensor pointer");
+  HsArgs a = hs_args(states, counts, q, k, v, beta, g, l, o, T, t0, n, G, H, K, V, L);
+  for (int t = 0; t < n; ++t) {
+    if (int st = hs_cascade_check(cascades[t], L, htype, 1)) return st;
+    a.casc[t] = cascades[t];
+  }
+  for (int e = 0; e < L; ++e) a.final_counts[e] = final_counts[e];
+  a.set_counts = 1;
+  a.strong = htype == HATTN_HTYPE_STRONG;
+  a.update = 1;
+  a.output = output != 0;
+  a.norm = l2norm_qk != 0;
+  a.scale = scale;
+  a.dt_qk = dtype_qk; a.dt_v = dtype_v; a.dt_l = dtype_l; a.dt_b = dtype_beta;
+  return hs_launch(a, B, hstruct, (hipStream_t)stream, "hattn_hstate_steps launch");
+}
+
+int hattn_hstate_prefill_levels(float* states, int* counts, const void* k, const void* v,
+                                const void* beta, const float* g, int B, int T, int G, int H,
+                                int K, int V, int L, int nlo, int hstruct, int htype,
+                                int l2norm_qk, int dtype_k, int dtype_v, int dtype_beta,
+                                void* stream) {
+  if (int st = hs_check(B, G, H, K, V, L, hstruct, htype)) return st;
+  if (T < 64 || T % 64 != 0) return fail(HATTN_ERR_VALUE, "T=%d is not a positive multiple of 64", T);
+  if (nlo < 1 || nlo > 7 || nlo > L) return fail(HATTN_ERR_VALUE, "nlo=%d with L=%d", nlo, L);
+  if (!states || !k || !v || !g || (hstruct == HATTN_HSTRUCT_GDELTA && !beta))
+    return fail(HATTN_ERR_VALUE, "null tensor pointer");
+  if (hstruct == HATTN_HSTRUCT_MAMBA2) {
+    HsCounts c{counts, {}};
+    unsigned int clear = 0;
+    hs_prefill_counts(T, L, nlo, c.v, &clear);
+    int unsupported = 0;
+    hipError_t e = hattn_mamba2_prefill_levels_launch(states, k, v, g, B, T, G, H, K, V, L, nlo,
+                                                      dtype_k, dtype_v, clear, c,
+                                                      (hipStream_t)stream, &unsupported);
+    if (unsupported)
+      return fail(HATTN_ERR_NOT_IMPLEMENTED, "dtype codes k=%d v=%d", dtype_k, dtype_v);
+    return check_hip(e, "hattn_hstate_prefill_levels launch");
+  }
+  // GDELTA: the recurrent form over the last chunk from an empty state (kernel.py:438-449)
+  HsArgs a = hs_args(states, counts, nullptr, k, v, beta, g, nullptr, nullptr, T, T - 64, 64, G, H,
+                     K, V, L);
+  int c[kHsMaxLevels] = {};
+  if (hattn_hstate_plan(c, nlo, htype, 64, a.casc) != 64)
+    return fail(HATTN_ERR_VALUE, "%d levels do not hold a chunk", nlo);
+  hs_prefill_counts(T, L, nlo, a.final_counts, &a.clear);
+  a.LA = nlo;
+  a.zero = 1;
+  a.set_counts = 1;
+  a.strong = htype == HATTN_HTYPE_STRONG;
+  a.update = 1;
+  a.norm = l2norm_qk != 0;
+  a.dt_qk = dtype_k; a.dt_v = dtype_v; a.dt_b = dtype_beta;
+  return hs_launch(a, B, hstruct, (hipStream_t)stream, "hattn_hstate_prefill_levels launch");
 }
 
 int hattn_mamba2_prefill_levels(float* states, const void* k, const void* v, const float* g,
@@ -785,8 +944,8 @@ int hattn_mamba2_prefill_levels(float* states, const void* k, const void* v, con
   if (!states || !k || !v || !g) return fail(HATTN_ERR_VALUE, "null tensor pointer");
   int unsupported = 0;
   hipError_t e = hattn_mamba2_prefill_levels_launch(states, k, v, g, B, T, G, H, K, V, L, nlo,
-                                                    dtype_k, dtype_v, (hipStream_t)stream,
-                                                    &unsupported);
+                                                    dtype_k, dtype_v, 0, HsCounts{nullptr, {}},
+                                                    (hipStream_t)stream, &unsupported);
   if (unsupported)
     return fail(HATTN_ERR_NOT_IMPLEMENTED, "dtype codes k=%d v=%d", dtype_k, dtype_v);
   return check_hip(e, "hattn_mamba2_prefill_levels launch");

@@ -1,20 +1,17 @@
-// Recurrent (decode) path of log-linear attention for gfx950: one token step of
-// the Fenwick level state HState and the prefill of its low levels.
+// Recurrent (decode) path of log-linear attention for gfx950: token steps of the
+// Fenwick level state HState and the prefill of its low levels.
 //
 // Replaces hattention_step / step_state / step_output (hattention/kernel.py:577-633,
-// recurrent.py:9-166) and the MAMBA2 fast path of postprocess_prefill_hstate_
-// (kernel.py:378-465).  The reference runs a torch einsum per level and a
-// Python loop over levels that reads device counts back to the host at every
-// level (recurrent.py:42-54); here the weak cascade is planned on the host from
-// a host copy of the counts (the counts depend only on the step number) and the
-// whole step, including GDELTA's l2norm of q and k, is one launch.
+// recurrent.py:9-166), the token loops around them (hattention_recurrent, the tail
+// and the low levels of a prefill, kernel.py:438-449, 555-570) and the MAMBA2 fast
+// path of postprocess_prefill_hstate_ (kernel.py:378-465).  The reference runs a
+// torch einsum per level and a Python loop over levels that reads device counts
+// back to the host at every level (recurrent.py:42-54); here the cascades are
+// planned on the host from a host copy of the counts (the counts depend only on
+// the step number) and any number of tokens, including GDELTA's l2norm of q and k
+// and the Mamba-2 layer's pre- and post-processing, is one launch.
 //
 // States: fp32 [B, H, K, V, L] (level innermost), the reference's HState layout.
-// Grid (B * H, V / 16): a workgroup owns 16 value columns of one (b, h) and all
-// K rows.  Every quantity of the step is per value column (the state update,
-// GDELTA's k^T S and the output's sum over k), so the column slices need no
-// exchange.  Thread t owns column v0 + t % 16 and rows t / 16 + 16 i, all L
-// levels of each (k, v) in registers.
 //
 // A step with cascade depth c (levels 0 .. c-1 are full and cascade upwards,
 // recurrent.py:42-54) is, per (k, v):
@@ -25,26 +22,17 @@
 //   o[v] = sum_k q[k] sum_l lambda[l] S[k][v][l]              (step_output, :159-166)
 #include <hip/hip_runtime.h>
 
+#include <numeric>
+#include <type_traits>
+
 #include "common.h"
+#include "hstate.h"
+#include "layer_math.h"
 
 namespace hattn {
 
-constexpr int kHsMaxL = 32;   // levels held in registers per (k, v)
-constexpr int kHsCols = 16;   // value columns per workgroup
+constexpr int kHsCols = 16;   // value columns per workgroup of the prefill levels
 constexpr int kHsRowGroups = 256 / kHsCols;
-
-template <typename T>
-__device__ __forceinline__ float ld(const T* p, size_t i) { return to_f32<T>(p[i]); }
-
-// Sum of x over the 256 threads of the workgroup (every thread gets the sum).
-__device__ __forceinline__ float block_sum256(float x, float* scratch4) {
-#pragma unroll
-  for (int d = 32; d >= 1; d >>= 1) x += __shfl_xor(x, d, 64);
-  __syncthreads();
-  if ((threadIdx.x & 63) == 0) scratch4[threadIdx.x >> 6] = x;
-  __syncthreads();
-  return scratch4[0] + scratch4[1] + scratch4[2] + scratch4[3];
-}
 
 // The level counts (shared by all rows) after the step: the cascade (weak: levels
 // 0 .. c-1 merge into level c; strong: levels 0 .. m-1 move up one level, m - 1
@@ -68,355 +56,341 @@ __device__ inline void cascade_counts(int* counts, int L, int cascade, int stron
   counts[0] += 1;
 }
 
-template <typename TQ, typename TV, typename TL, typename TB, bool GDN>
-__global__ __launch_bounds__(256) void hstate_step_kernel(
-    float* __restrict__ states, int* __restrict__ counts, const TQ* __restrict__ q,
-    const TQ* __restrict__ k, const TV* __restrict__ v, const TB* __restrict__ beta,
-    const float* __restrict__ g, const TL* __restrict__ l, TV* __restrict__ o, int G, int H,
-    int K, int V, int L, int cascade, int strong, int update, int output, int norm_qk, float scale) {
-  __shared__ float sq[256], sk[256], sv[kHsCols], sl[kHsMaxL], snorm[8];
-  __shared__ float red[256 * 4];   // [row group][column][4]: k^T S per level, then o
-  const int tid = threadIdx.x;
-  const int v0 = blockIdx.y * kHsCols, bh = blockIdx.x, b = bh / H, h = bh % H;
-  const int gq = h / (H / G);
-  const int vv = tid % kHsCols, kg = tid / kHsCols;
-
-  // q, k (l2-normalised for GDELTA: q / |q| * scale, k / |k|, kernel.py:20-23,
-  // 626-629 with the eps of fla's l2norm), v columns, lambda
-  // (q, lambda are read only for the output, k, v only for the update)
-  float qx = 0.f, kx = 0.f;
-  if (output && tid < K) qx = ld(q, ((size_t)b * G + gq) * K + tid);
-  if (update && tid < K) kx = ld(k, ((size_t)b * G + gq) * K + tid);
-  if (norm_qk) {
-    const float nq = block_sum256(qx * qx, snorm);
-    const float nk = block_sum256(kx * kx, snorm + 4);
-    // rounded to the input dtype after the norm and after the scale, as the
-    // reference's l2norm_fwd / l2norm_and_scale_fwd store their outputs
-    qx = to_f32<TQ>(from_f32<TQ>(to_f32<TQ>(from_f32<TQ>(qx * rsqrtf(nq + 1e-6f))) * scale));
-    kx = to_f32<TQ>(from_f32<TQ>(kx * rsqrtf(nk + 1e-6f)));
-  }
-  if (tid < K) {
-    sq[tid] = qx;
-    sk[tid] = kx;
-  }
-  if (update && tid < kHsCols) sv[tid] = ld(v, (size_t)bh * V + v0 + tid);
-  if (output && tid < L) sl[tid] = ld(l, (size_t)bh * L + tid);
-  __syncthreads();
-  const float a = update ? __expf(g[bh]) : 0.f;
-  const float bt = GDN && update ? ld(beta, (size_t)bh) : 1.f;
-  float* sbase = states + (size_t)bh * K * V * L;
-
-  auto load_cascaded = [&](int kk, float (&s)[kHsMaxL]) {
-    const float* p = sbase + ((size_t)kk * V + v0 + vv) * L;
-#pragma unroll
-    for (int e = 0; e < kHsMaxL; ++e) s[e] = e < L ? p[e] : 0.f;
-    if (strong) {
-      // cascade_strong (recurrent.py:56-74) with merge level m = cascade: levels
-      // 0 .. m-1 move up one level, level m - 1 merging into level m (m = L: the
-      // top level's content leaves the state); level 0 ends empty
-      float prev = 0.f;
-#pragma unroll
-      for (int e = 0; e < kHsMaxL; ++e) {
-        const float cur = s[e];
-        s[e] = e == 0 ? 0.f : (e < cascade ? prev : (e == cascade ? cur + prev : cur));
-        prev = cur;
-      }
-    } else if (cascade > 0) {
-      float acc = 0.f;
-#pragma unroll
-      for (int e = 0; e < kHsMaxL; ++e)
-        if (e < cascade) {
-          acc += s[e];
-          s[e] = 0.f;
-        }
-#pragma unroll
-      for (int e = 0; e < kHsMaxL; ++e)
-        if (e == cascade) s[e] += acc;
-    }
-  };
-
-  // GDELTA: u[l] = sum_k k[k] S_cascaded[k][v][l], reduced over the row groups
-  float u[kHsMaxL];
-#pragma unroll
-  for (int e = 0; e < kHsMaxL; ++e) u[e] = 0.f;
-  if (GDN && update) {
-    for (int kk = kg; kk < K; kk += kHsRowGroups) {
-      float s[kHsMaxL];
-      load_cascaded(kk, s);
-#pragma unroll
-      for (int e = 0; e < kHsMaxL; ++e) u[e] += sk[kk] * s[e];
-    }
-    for (int e0 = 0; e0 < L; e0 += 4) {
-      __syncthreads();
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        float x = 0.f;
-#pragma unroll
-        for (int e = 0; e < kHsMaxL; ++e)
-          if (e == e0 + j) x = u[e];
-        red[(kg * kHsCols + vv) * 4 + j] = x;
-      }
-      __syncthreads();
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        float x = 0.f;
-        for (int gi = 0; gi < kHsRowGroups; ++gi) x += red[(gi * kHsCols + vv) * 4 + j];
-#pragma unroll
-        for (int e = 0; e < kHsMaxL; ++e)
-          if (e == e0 + j) u[e] = x;
-      }
-    }
-  }
-
-  float oacc = 0.f;
-  for (int kk = kg; kk < K; kk += kHsRowGroups) {
-    float s[kHsMaxL];
-    float* p = sbase + ((size_t)kk * V + v0 + vv) * L;
-    if (update) {
-      load_cascaded(kk, s);
-      const float bk = bt * sk[kk];
-#pragma unroll
-      for (int e = 0; e < kHsMaxL; ++e) s[e] = GDN ? a * (s[e] - bk * u[e]) : a * s[e];
-      s[0] = bk * sv[vv];
-#pragma unroll
-      for (int e = 0; e < kHsMaxL; ++e)
-        if (e < L) p[e] = s[e];
-    } else {
-#pragma unroll
-      for (int e = 0; e < kHsMaxL; ++e) s[e] = e < L ? p[e] : 0.f;
-    }
-    if (output) {
-      float w = 0.f;
-#pragma unroll
-      for (int e = 0; e < kHsMaxL; ++e)
-        if (e < L) w += sl[e] * s[e];
-      oacc += sq[kk] * w;
-    }
-  }
-  if (output) {
-    __syncthreads();
-    red[kg * kHsCols + vv] = oacc;
-    __syncthreads();
-    if (kg == 0) {
-      float x = 0.f;
-      for (int gi = 0; gi < kHsRowGroups; ++gi) x += red[gi * kHsCols + vv];
-      o[(size_t)bh * V + v0 + vv] = from_f32<TV>(x);
-    }
-  }
-  // counts (shared by all rows): the same cascade, then one more token at level 0
-  if (update && counts != nullptr && blockIdx.y == 0 && bh == 0 && tid == 0)
-    cascade_counts(counts, L, cascade, strong);
+// Element u + i, i < n, of a tensor with dtype code dt (0 bf16, 2 fp32); p, u and dt
+// are uniform.  Through a buffer descriptor: a lane keeps a 32-bit offset and no
+// address, and reads 0 from n on.
+__device__ __forceinline__ float hs_ld(const void* p, long long u, unsigned int i, int dt,
+                                       int n = 1) {
+  const int es = dt == 0 ? 2 : 4;
+  const rsrc_t r = make_rsrc((const char*)p + u * es, (size_t)n * es);
+  return dt == 0 ? (float)buf_load<__bf16>(r, 2 * i, 0) : buf_load<float>(r, 4 * i, 0);
 }
+__device__ __forceinline__ void hs_st(void* p, long long u, unsigned int i, float x, int dt) {
+  if (dt == 0) ((__bf16*)p + u)[i] = (__bf16)x;
+  else ((float*)p + u)[i] = x;
+}
+__device__ __forceinline__ float hs_round(float x, int dt) { return dt == 0 ? (float)(__bf16)x : x; }
 
-// Sum over the lanes of one wave that share lane % VB (VB a power of two <= 32):
-// butterfly over the lane bits above log2(VB).
-__device__ __forceinline__ float wave_sum_same_col(float x, int VB) {
-  for (int d = 32; d >= VB; d >>= 1) x += __shfl_xor(x, d, 64);
+__device__ __forceinline__ float wave_sum(float x) {
+  x = row_sum16(x);
+  x += __shfl_xor(x, 16, 64);
+  x += __shfl_xor(x, 32, 64);
   return x;
 }
+// lane i gets lane i - 1's value, lane 0 gets 0 (wave_shr:1)
+__device__ __forceinline__ float lane_before(float x) { return dpp_f32<0x138, 0xf, true>(0.f, x); }
+__device__ __forceinline__ float lane_value(float x, int lane) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), lane));
+}
 
-// The same step as hstate_step_kernel with the workgroup's state slab staged
-// in LDS: the slab (K rows of VB * L contiguous floats, row stride V * L) moves
-// between HBM and LDS in 16-byte pieces, all of a thread's loads issued before
-// the first is consumed, and the per-(k, v) work reads the slab from LDS with
-// each (k, v) group of L levels padded to an odd stride (conflict-free reads).
-// Grid (B * H, V / VB); VB in {4, 8, 16} is chosen by the host so that the slab
-// fits in LDS; NL (16 or 32) bounds the levels held in registers.  Dynamic
-// LDS: K * VB * (L | 1) floats.
-constexpr int kHsBatch = 8;    // 16-byte pieces in flight per thread
+// Token steps with the state in registers.
+//
+// A workgroup owns VB value columns of one (b, h): for every row k the VB * LA
+// contiguous floats [v][level].  Lane n of each wave holds the NV elements from
+// NV n on, of the wave's R rows (blockDim = 64 ceil(K / R)), from one load per row
+// to one store per row, however many tokens are stepped in between; so the state
+// moves through HBM once, in whole lines, with R loads in flight per lane.  (Staged
+// through LDS and one launch a token, this took 109 us for a GDELTA step of B 4, H
+// 16, K = V = 128, L 18, and 14 us for each of the 64 tokens that rebuild the low
+// levels after a prefill.)
+//   cascade   S[c] += S[0 .. c-1] is a sum over the c elements before S[c] in the
+//             flat [v][level] order: a shift along the lanes.
+//   u = k^T S, w = q^T S   sums over a wave's rows in registers (k, q of a row are
+//             wave-uniform: readlane), then over the waves through LDS, double
+//             buffered, so one barrier a token.
+//   update    S = a S - k (a beta u), level 0 = k (beta v)
+//   output    q^T S after the update = a (w - beta (q . k) u) per level, and
+//             (q . k) beta v at level 0; the first wave weights and sums the levels.
+// The next token's operands are loaded before the current token is computed.
+// (STRONG is an instance of its own: the two cascades in one kernel cost 70 spilled
+// registers.)  NV (elements per lane) sets the number of workgroups: the host takes the widest
+// that still fills the chip.
+template <int KIND, int NV, int R, bool STRONG, int KMAX>
+__global__ __launch_bounds__(64 * KMAX / R) void hstate_steps_kernel(const HsArgs p) {
+  extern __shared__ float red[];     // [2][u, w][wave][64 NV]
+  __shared__ float part[64 * NV];    // weighted levels of the output, first wave only
+  typedef float vecN __attribute__((ext_vector_type(NV)));
+  constexpr bool GDN = KIND == kHsGdelta, LAYER = KIND == kHsLayer;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), nw = blockDim.x >> 6;
+  const int bh = blockIdx.x, b = bh / p.H, h = bh - b * p.H, gq = h / (p.H / p.G);
+  const int K = p.K, V = p.V, L = p.L, LA = p.LA;
+  const int v0 = blockIdx.y * p.VB, vbc = p.VB < V - v0 ? p.VB : V - v0;
+  const bool act = lane * NV < vbc * LA;
+  const int e0 = act ? lane * NV : 0;
+  const int vv0 = e0 / LA, ll0 = e0 - vv0 * LA;
+  int ll[NV];
+  int vi = v0 + vv0;   // column of this lane's level-0 element, if it has one
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    ll[i] = ll0 + i >= LA ? ll0 + i - LA : ll0 + i;
+    if (i > 0 && ll[i] == 0) ++vi;
+  }
+  if (vi >= V) vi = V - 1;   // a lane at the end that has none
+  // elements are contiguous unless only the first LA of L levels are stepped
+  // (NV = 1 then)
+  const unsigned int at0 = LA == L ? e0 : vv0 * L + ll0;
+  const int row0 = wave * R, klane = row0 & 63;
+  // (a uniform row address and a 32-bit lane offset: no address registers per row)
+  float* base = p.states + (((size_t)bh * K + row0) * V + v0) * L;
+  const int rstride = V * L;
 
-template <typename TQ, typename TV, typename TL, typename TB, bool GDN, int NL>
-__global__ __launch_bounds__(256) void hstate_step_lds_kernel(
-    float* __restrict__ states, int* __restrict__ counts, const TQ* __restrict__ q,
-    const TQ* __restrict__ k, const TV* __restrict__ v, const TB* __restrict__ beta,
-    const float* __restrict__ g, const TL* __restrict__ l, TV* __restrict__ o, int G, int H,
-    int K, int V, int L, int VB, int cascade, int strong, int update, int output, int norm_qk,
-    float scale) {
-  extern __shared__ float slab[];
-  __shared__ float sq[256], sk[256], sv[kHsCols], sl[NL], snorm[8];
-  __shared__ float red[4 * kHsCols * NL];   // [wave][column][level]
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int v0 = blockIdx.y * VB, bh = blockIdx.x, b = bh / H, h = bh % H;
-  const int gq = h / (H / G);
-  const int Lp = L | 1, W = VB * L, W4 = W >> 2, n4 = K * W4;
-  float* src = states + (size_t)bh * K * V * L + (size_t)v0 * L;
-  const size_t rstride = (size_t)V * L;
-  // piece f = tid + 256 i sits at (row, off) = divmod(f, W4); advanced without
-  // dividing: 256 = dq * W4 + dr
-  const int dq = 256 / W4, dr = 256 - dq * W4;
-  int row = tid / W4, off = tid - (tid / W4) * W4;
-  floatx4 x[kHsBatch];
-  int brow = row, boff = off;   // (row, off) of the batch's first piece
-  auto advance = [&](int& r, int& c) {
-    r += dq;
-    c += dr;
-    if (c >= W4) {
-      c -= W4;
-      ++r;
+  float s[R][NV];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    vecN x{};
+    if (!p.zero && row0 + r < K) x = *(const vecN*)(base + r * rstride + at0);
+    if constexpr (NV == 1) s[r][0] = x[0];
+    else
+#pragma unroll
+      for (int i = 0; i < NV; ++i) s[r][i] = x[i];
+  }
+
+  struct Token {
+    float k[4], q[4], g, beta, v, lam[NV], x;
+  };
+  const HsLayer& y = p.layer;
+  auto fetch = [&](int i0) {
+    Token n;
+    const int t = p.t0 + i0;
+    const long long qo = b * p.q_b + t * p.q_t + gq * K, so = b * p.s_b + t * p.s_t + h;
+    const long long vo = b * p.v_b + t * p.v_t + h * V, lo = b * p.l_b + t * p.l_t + h * L;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int i = lane + 64 * j;
+      n.k[j] = p.update && 64 * j < K ? hs_ld(p.k, qo, i, p.dt_qk, K) : 0.f;
+      n.q[j] = p.output && 64 * j < K ? hs_ld(p.q, qo, i, p.dt_qk, K) : 0.f;
     }
-  };
-  auto load_batch = [&]() {
-    brow = row;
-    boff = off;
+    n.beta = GDN && p.update ? hs_ld(p.beta, so, 0, p.dt_b) : 1.f;
+    n.x = 0.f;
+    n.v = p.update ? hs_ld(p.v, vo, vi, LAYER ? y.dt_x : p.dt_v, V) : 0.f;
 #pragma unroll
-    for (int i = 0; i < kHsBatch; ++i) {
-      if (row < K) x[i] = *(const floatx4*)(src + row * rstride + 4 * off);
-      advance(row, off);
+    for (int i = 0; i < NV; ++i) n.lam[i] = p.output ? hs_ld(p.l, lo, ll[i], p.dt_l, L) : 0.f;
+    if (LAYER) {
+      // the Mamba-2 layer's inputs: v = x dt', g = A dt', lambda of (L, dl), each
+      // rounded to its dtype as the separate layer kernels do
+      const float d = layer_dtp(hs_ld(y.dt, so, 0, y.dt_dt),
+                                y.bias ? hs_ld(y.bias, h, 0, y.dt_bias) : 0.f, y.softplus);
+      n.g = layer_g(hs_ld(y.A, h, 0, y.dt_A), d);
+      n.v = hs_round(n.v * d, p.dt_v);
+#pragma unroll
+      for (int i = 0; i < NV; ++i)
+        n.lam[i] = hs_round(lambda_of(hs_ld(y.Lp, h * L, ll[i], y.dt_Lp, L), n.lam[i], y.mode), y.dt_lam);
+      if (y.D) n.x = hs_ld(p.v, vo, v0 + lane, y.dt_x, V);
+    } else {
+      n.g = p.update ? p.g[so] : 0.f;
     }
+    return n;
   };
-  // padded LDS offset of element w of a row: group w / L, level w % L (the
-  // quotient by a float reciprocal: exact for w < 2^16, L <= 32, as (w + 0.5) / L
-  // is at least 1 / (2L) away from an integer)
-  const float invL = 1.f / (float)L;
-  auto pad = [&](int w) {
-    const int grp = (int)((float)w * invL + 0.5f * invL);
-    return grp * Lp + (w - grp * L);
-  };
-  auto store_batch_lds = [&]() {
-    int r = brow, c = boff;
+
+  Token nx = fetch(0);
+  for (int t = 0; t < p.T; ++t) {
+    Token tk = nx;
+    if (t + 1 < p.T) nx = fetch(t + 1);
+    if (p.norm) {
+      // q / |q| * scale, k / |k| (kernel.py:20-23, 626-629 with the eps of fla's
+      // l2norm), rounded to the input dtype after the norm and after the scale, as
+      // the reference's l2norm_fwd / l2norm_and_scale_fwd store their outputs
+      float nq = 0.f, nk = 0.f;
 #pragma unroll
-    for (int i = 0; i < kHsBatch; ++i) {
-      if (r < K) {
-        float* d = slab + r * VB * Lp;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) d[pad(4 * c + j)] = x[i][j];
+      for (int j = 0; j < 4; ++j) {
+        nq += tk.q[j] * tk.q[j];
+        nk += tk.k[j] * tk.k[j];
       }
-      advance(r, c);
-    }
-  };
-
-  // ---- HBM -> LDS: the first batch of state loads goes out before the small
-  // operands are read, so their latencies overlap
-  load_batch();
-  float qx = 0.f, kx = 0.f;
-  if (output && tid < K) qx = ld(q, ((size_t)b * G + gq) * K + tid);
-  if (update && tid < K) kx = ld(k, ((size_t)b * G + gq) * K + tid);
-  const float a = update ? __expf(g[bh]) : 0.f;
-  const float bt = GDN && update ? ld(beta, (size_t)bh) : 1.f;
-  if (update && tid < VB) sv[tid] = ld(v, (size_t)bh * V + v0 + tid);
-  if (output && tid < L) sl[tid] = ld(l, (size_t)bh * L + tid);
-  if (norm_qk) {
-    const float nq = block_sum256(qx * qx, snorm);
-    const float nk = block_sum256(kx * kx, snorm + 4);
-    qx = to_f32<TQ>(from_f32<TQ>(to_f32<TQ>(from_f32<TQ>(qx * rsqrtf(nq + 1e-6f))) * scale));
-    kx = to_f32<TQ>(from_f32<TQ>(kx * rsqrtf(nk + 1e-6f)));
-  }
-  if (tid < K) {
-    sq[tid] = qx;
-    sk[tid] = kx;
-  }
-  store_batch_lds();
-  for (int f0 = 256 * kHsBatch; f0 < n4; f0 += 256 * kHsBatch) {
-    load_batch();
-    store_batch_lds();
-  }
-  __syncthreads();
-
-  // ---- per (k, v) work: thread owns column vv = tid % VB, rows tid / VB + (256 / VB) i
-  const int vv = tid & (VB - 1), kg = tid / VB, nkg = 256 / VB;
-  auto load_cascaded = [&](int kk, float (&s)[NL]) {
-    const float* p = slab + (kk * VB + vv) * Lp;
+      const float rq = rsqrtf(wave_sum(nq) + 1e-6f), rk = rsqrtf(wave_sum(nk) + 1e-6f);
 #pragma unroll
-    for (int e = 0; e < NL; ++e) s[e] = e < L ? p[e] : 0.f;
-    if (strong) {
-      float prev = 0.f;   // cascade_strong, as in hstate_step_kernel
-#pragma unroll
-      for (int e = 0; e < NL; ++e) {
-        const float cur = s[e];
-        s[e] = e == 0 ? 0.f : (e < cascade ? prev : (e == cascade ? cur + prev : cur));
-        prev = cur;
+      for (int j = 0; j < 4; ++j) {
+        tk.q[j] = hs_round(hs_round(tk.q[j] * rq, p.dt_qk) * p.scale, p.dt_qk);
+        tk.k[j] = hs_round(tk.k[j] * rk, p.dt_qk);
       }
-    } else if (cascade > 0) {
-      float acc = 0.f;
+    }
+    float qk = 0.f;
+    if (p.output && p.update) {
 #pragma unroll
-      for (int e = 0; e < NL; ++e)
-        if (e < cascade) {
-          acc += s[e];
-          s[e] = 0.f;
+      for (int j = 0; j < 4; ++j) qk += tk.q[j] * tk.k[j];
+      qk = wave_sum(qk);
+    }
+    const int kj = row0 >> 6;
+    const float kr = kj == 0 ? tk.k[0] : kj == 1 ? tk.k[1] : kj == 2 ? tk.k[2] : tk.k[3];
+    const float qr = kj == 0 ? tk.q[0] : kj == 1 ? tk.q[1] : kj == 2 ? tk.q[2] : tk.q[3];
+
+    if (p.update) {
+      const int c = p.casc[t];
+      bool keep[NV], into[NV];
+      if (STRONG) {
+        // cascade_strong (recurrent.py:56-74) with merge level c: levels 0 .. c-1
+        // move up one level, c - 1 merging into c (c = L: the top level's content
+        // leaves the state); level 0 ends empty
+#pragma unroll
+        for (int i = 0; i < NV; ++i) {
+          keep[i] = ll[i] >= c && ll[i] > 0;
+          into[i] = ll[i] <= c && ll[i] > 0;
         }
 #pragma unroll
-      for (int e = 0; e < NL; ++e)
-        if (e == cascade) s[e] += acc;
-    }
-  };
-
-  float u[NL];
+        for (int r = 0; r < R; ++r) {
+          const float before = lane_before(s[r][NV - 1]);
 #pragma unroll
-  for (int e = 0; e < NL; ++e) u[e] = 0.f;
-  if (GDN && update) {
-    for (int kk = kg; kk < K; kk += nkg) {
-      float s[NL];
-      load_cascaded(kk, s);
+          for (int i = NV - 1; i >= 0; --i)
+            s[r][i] = (keep[i] ? s[r][i] : 0.f) + (into[i] ? (i > 0 ? s[r][i > 0 ? i - 1 : 0] : before) : 0.f);
+        }
+      } else {
+        // cascade_weak: level 0 ends empty too (at c = 0 the insert overwrites it)
+        int at = c - ll0;           // this lane's element of level c, if it has one
+        if (at < 0) at += LA;
+        const bool has = at < NV;
+        const int lim = has ? c - at : -(1 << 20);
+        bool own[NV];
 #pragma unroll
-      for (int e = 0; e < NL; ++e) u[e] += sk[kk] * s[e];
-    }
+        for (int i = 0; i < NV; ++i) {
+          keep[i] = ll[i] >= c && ll[i] > 0;
+          into[i] = i == at;
+          own[i] = has && i < at && at - i <= c;
+        }
+        const int far = (c + NV - 1) / NV;   // lanes before that hold levels below c
 #pragma unroll
-    for (int e = 0; e < NL; ++e)
-      if (e < L) {
-        const float x = wave_sum_same_col(u[e], VB);
-        if (lane < VB) red[(wave * kHsCols + vv) * NL + e] = x;
+        for (int r = 0; r < R; ++r) {
+          float sum = 0.f, cur[NV];
+#pragma unroll
+          for (int i = 0; i < NV; ++i) {
+            sum += own[i] ? s[r][i] : 0.f;
+            cur[i] = s[r][i];
+          }
+          for (int d = 1; d <= far; ++d)
+#pragma unroll
+            for (int i = 0; i < NV; ++i) {
+              cur[i] = lane_before(cur[i]);
+              sum += NV * d - i <= lim ? cur[i] : 0.f;
+            }
+#pragma unroll
+          for (int i = 0; i < NV; ++i)
+            s[r][i] = (keep[i] ? s[r][i] : 0.f) + (into[i] && c > 0 ? sum : 0.f);
+        }
       }
-    __syncthreads();
-#pragma unroll
-    for (int e = 0; e < NL; ++e)
-      if (e < L)
-        u[e] = red[(0 * kHsCols + vv) * NL + e] + red[(1 * kHsCols + vv) * NL + e] +
-               red[(2 * kHsCols + vv) * NL + e] + red[(3 * kHsCols + vv) * NL + e];
-  }
-
-  float oacc = 0.f;
-  for (int kk = kg; kk < K; kk += nkg) {
-    float s[NL];
-    float* p = slab + (kk * VB + vv) * Lp;
-    if (update) {
-      load_cascaded(kk, s);
-      const float bk = bt * sk[kk];
-#pragma unroll
-      for (int e = 0; e < NL; ++e) s[e] = GDN ? a * (s[e] - bk * u[e]) : a * s[e];
-      s[0] = bk * sv[vv];
-#pragma unroll
-      for (int e = 0; e < NL; ++e)
-        if (e < L) p[e] = s[e];
-    } else {
-#pragma unroll
-      for (int e = 0; e < NL; ++e) s[e] = e < L ? p[e] : 0.f;
     }
-    if (output) {
-      float w = 0.f;
-#pragma unroll
-      for (int e = 0; e < NL; ++e)
-        if (e < L) w += sl[e] * s[e];
-      oacc += sq[kk] * w;
-    }
-  }
-  if (output) {
-    oacc = wave_sum_same_col(oacc, VB);
-    __syncthreads();   // red is reused
-    if (lane < VB) red[wave * kHsCols + vv] = oacc;
-    __syncthreads();
-    if (tid < VB)
-      o[(size_t)bh * V + v0 + tid] =
-          from_f32<TV>(red[tid] + red[kHsCols + tid] + red[2 * kHsCols + tid] +
-                       red[3 * kHsCols + tid]);
-  }
 
-  // ---- LDS -> HBM
-  if (update) {
-    __syncthreads();
-    row = tid / W4;
-    off = tid - row * W4;
-    for (int f0 = 0; f0 < n4; f0 += 256) {
-      if (row < K) {
-        const float* d = slab + row * VB * Lp;
-        floatx4 x;
+    float u[NV], w[NV];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) x[j] = d[pad(4 * off + j)];
-        *(floatx4*)(src + row * rstride + 4 * off) = x;
+    for (int i = 0; i < NV; ++i) u[i] = w[i] = 0.f;
+    const bool need_u = GDN && p.update;
+    if (need_u)
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const float kk = lane_value(kr, klane + r);
+#pragma unroll
+        for (int i = 0; i < NV; ++i) u[i] += kk * s[r][i];
       }
-      advance(row, off);
+    if (p.output)
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const float qq = lane_value(qr, klane + r);
+#pragma unroll
+        for (int i = 0; i < NV; ++i) w[i] += qq * s[r][i];
+      }
+    float* ru = red + (size_t)(t & 1) * 2 * nw * 64 * NV;
+    float* rw = ru + nw * 64 * NV;
+    if (need_u || p.output) {
+      vecN x;
+      if (need_u) {
+        if constexpr (NV == 1) x = u[0];
+        else
+#pragma unroll
+          for (int i = 0; i < NV; ++i) x[i] = u[i];
+        *(vecN*)(ru + (wave * 64 + lane) * NV) = x;
+      }
+      if (p.output) {
+        if constexpr (NV == 1) x = w[0];
+        else
+#pragma unroll
+          for (int i = 0; i < NV; ++i) x[i] = w[i];
+        *(vecN*)(rw + (wave * 64 + lane) * NV) = x;
+      }
+      __syncthreads();
+      if (need_u) {
+        vecN acc{};
+        for (int j = 0; j < nw; ++j) acc += *(const vecN*)(ru + (j * 64 + lane) * NV);
+        if constexpr (NV == 1) u[0] = acc[0];
+        else
+#pragma unroll
+          for (int i = 0; i < NV; ++i) u[i] = acc[i];
+      }
     }
-    if (counts != nullptr && blockIdx.y == 0 && bh == 0 && tid == 0)
-      cascade_counts(counts, L, cascade, strong);
+
+    const float a = p.update ? __expf(tk.g) : 1.f;
+    if (p.output && wave == 0) {
+      vecN acc{};
+      for (int j = 0; j < nw; ++j) acc += *(const vecN*)(rw + (j * 64 + lane) * NV);
+      if constexpr (NV == 1) w[0] = acc[0];
+      else
+#pragma unroll
+        for (int i = 0; i < NV; ++i) w[i] = acc[i];
+#pragma unroll
+      for (int i = 0; i < NV; ++i) {
+        float z = w[i];
+        if (p.update) {
+          z = GDN ? a * (z - tk.beta * qk * u[i]) : a * z;
+          if (ll[i] == 0) z = qk * (tk.beta * tk.v);
+        }
+        if (act) part[e0 + i] = tk.lam[i] * z;
+      }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      if (lane < vbc) {
+        float z = 0.f;
+        for (int e = 0; e < LA; ++e) z += part[lane * LA + e];
+        const long long oo = b * p.o_b + (p.t0 + t) * p.o_t + h * V + v0;
+        if (LAYER) {
+          z = hs_round(z, p.dt_v);
+          if (y.D) z = layer_out(z, tk.x, hs_ld(y.D, h, 0, y.dt_D));
+        }
+        hs_st(p.o, oo, lane, z, LAYER ? y.dt_out : p.dt_v);
+      }
+      __builtin_amdgcn_wave_barrier();
+    }
+
+    if (p.update) {
+      float m[NV], kr2 = kr;
+      asm("" : "+v"(kr2));   // read the rows' k again instead of holding R scalars
+#pragma unroll
+      for (int i = 0; i < NV; ++i) m[i] = ll[i] == 0 ? tk.beta * tk.v : -(a * tk.beta) * u[i];
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const float kk = lane_value(kr2, klane + r);
+#pragma unroll
+        for (int i = 0; i < NV; ++i) {
+          if (GDN) s[r][i] = __builtin_fmaf(kk, m[i], a * s[r][i]);
+          else s[r][i] = ll[i] == 0 ? kk * m[i] : a * s[r][i];
+        }
+      }
+    }
+  }
+
+  if (p.update && act)
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+      if (row0 + r < K) {
+        vecN x;
+        if constexpr (NV == 1) x = s[r][0];
+        else
+#pragma unroll
+          for (int i = 0; i < NV; ++i) x[i] = s[r][i];
+        *(vecN*)(base + r * rstride + at0) = x;
+      }
+  // levels above the stepped ones that end empty
+  if (p.clear)
+    for (int i = tid; i < K * vbc; i += blockDim.x) {
+      const int kk = i / vbc;
+      float* d = p.states + (((size_t)bh * K + kk) * V + v0 + (i - kk * vbc)) * L;
+      for (int e = LA; e < L; ++e)
+        if (p.clear >> e & 1) d[e] = 0.f;
+    }
+  // counts (shared by all rows)
+  if (p.counts != nullptr && blockIdx.y == 0 && bh == 0) {
+    if (p.set_counts) {
+      if (tid < L) p.counts[tid] = p.final_counts[tid];
+    } else if (p.update && tid == 0) {
+      cascade_counts(p.counts, L, p.casc[0], STRONG);
+    }
   }
 }
 
@@ -426,11 +400,13 @@ __global__ __launch_bounds__(256) void hstate_step_lds_kernel(
 // < e, i.e. chunk offsets [64 - 2^e, 64 - 2^(e-1)) of the last chunk, each token
 // s weighted by exp(sum_{u = s+1}^{T-1} g_u) (the reverse chunk-local cumsum
 // gr[s + 1] of :420).  Grid (B * H, V / 16); the last chunk's k rows and its
-// weighted v columns are staged in LDS as fp32.
+// weighted v columns are staged in LDS as fp32.  Levels in the bit mask `clear`
+// (those above that hold no token) are set to zero, and the level counts stored.
 template <typename TK, typename TV>
 __global__ __launch_bounds__(256) void mamba2_prefill_levels_kernel(
     float* __restrict__ states, const TK* __restrict__ k, const TV* __restrict__ v,
-    const float* __restrict__ g, int T, int G, int H, int K, int V, int L, int nlo) {
+    const float* __restrict__ g, int T, int G, int H, int K, int V, int L, int nlo,
+    unsigned int clear, HsCounts counts) {
   __shared__ float sk[64 * 256];      // [token][k]
   __shared__ float sv[64 * kHsCols];  // [token][column], weighted
   __shared__ float sw[64];            // sw[j]: weight of chunk offset j
@@ -471,7 +447,10 @@ __global__ __launch_bounds__(256) void mamba2_prefill_levels_kernel(
         acc += sk[j * 256 + kk] * sv[j * kHsCols + vv];
       p[e] = acc;
     }
+    for (int e = nlo; e < L; ++e)
+      if (clear >> e & 1) p[e] = 0.f;
   }
+  if (counts.out != nullptr && blockIdx.y == 0 && bh == 0 && tid < L) counts.out[tid] = counts.v[tid];
 }
 
 }  // namespace hattn
@@ -495,94 +474,69 @@ bool with_type(int dt, F&& f) {
   return false;
 }
 
+bool known_type(int dt) { return dt == HS_BF16 || dt == HS_FP32; }
+
+template <int KIND, int NV, int R, bool STRONG = false, int KMAX = 256>
+hipError_t launch_steps(const HsArgs& a, int B, int nblk, hipStream_t stream) {
+  const int nw = (a.K + R - 1) / R;
+  const size_t smem = (size_t)2 * 2 * nw * 64 * NV * sizeof(float);
+  hipLaunchKernelGGL((hattn::hstate_steps_kernel<KIND, NV, R, STRONG, KMAX>), dim3(B * a.H, nblk), dim3(64 * nw),
+                     smem, stream, a);
+  return hipGetLastError();
+}
+
 }  // namespace
 
-hipError_t hattn_hstate_step_launch(float* states, int* counts, const void* q, const void* k,
-                                    const void* v, const void* beta, const float* g,
-                                    const void* l, void* o, int B, int G, int H, int K, int V,
-                                    int L, int gdn, int cascade, int strong, int update,
-                                    int output, int norm_qk, float scale, int dt_qk, int dt_v,
-                                    int dt_l, int dt_b, hipStream_t stream, int* unsupported) {
-  using namespace hattn;
-  const bool known = (dt_qk == HS_BF16 || dt_qk == HS_FP32) &&
-                     (dt_v == HS_BF16 || dt_v == HS_FP32) &&
-                     (dt_l == HS_BF16 || dt_l == HS_FP32) &&
-                     (!gdn || dt_b == HS_BF16 || dt_b == HS_FP32);
+hipError_t hattn_hstate_steps_launch(HsArgs a, int B, int gdn, hipStream_t stream,
+                                     int* unsupported) {
+  const HsLayer& y = a.layer;
+  bool known = known_type(a.dt_qk) && known_type(a.dt_v) && known_type(a.dt_l) &&
+               (!gdn || known_type(a.dt_b));
+  if (y.on)
+    for (int dt : {y.dt_x, y.dt_dt, y.dt_A, y.dt_bias, y.dt_Lp, y.dt_D, y.dt_lam, y.dt_out})
+      known = known && known_type(dt);
   *unsupported = known ? 0 : 1;
   if (!known) return hipSuccess;
-  // LDS-staged kernel when the slab of VB columns fits (VB = 16, halved while
-  // the grid has fewer than 1024 workgroups or the slab exceeds 40 KB, so that
-  // several workgroups share a CU and their load / compute / store phases
-  // overlap); the register kernel otherwise (large K * L) or when the state
-  // pointer is not 16-byte aligned
-  const int Lp = L | 1;
-  int VB = 16;
-  auto slab_bytes = [&](int vb) { return (size_t)K * vb * Lp * sizeof(float); };
-  while (VB > 4 && ((long)B * H * (V / VB) < 1024 || slab_bytes(VB) > 40 * 1024)) VB >>= 1;
-  const bool use_lds = slab_bytes(VB) <= 144 * 1024 && ((uintptr_t)states & 15) == 0;
-  const int smem = (int)slab_bytes(VB);
-  hipError_t err = hipSuccess;
-  auto launch = [&](auto kern_lds, auto kern_reg, auto tq, auto tv, auto tl, auto tb) {
-    using TQ = decltype(tq);
-    using TV = decltype(tv);
-    using TL = decltype(tl);
-    using TB = decltype(tb);
-    if (use_lds) {
-      if ((err = hipFuncSetAttribute((const void*)kern_lds,
-                                     hipFuncAttributeMaxDynamicSharedMemorySize, smem)) !=
-          hipSuccess)
-        return;
-      hipLaunchKernelGGL(kern_lds, dim3(B * H, V / VB), dim3(256), smem, stream, states, counts,
-                         (const TQ*)q, (const TQ*)k, (const TV*)v, (const TB*)beta, g,
-                         (const TL*)l, (TV*)o, G, H, K, V, L, VB, cascade, strong, update, output,
-                         norm_qk, scale);
-    } else {
-      hipLaunchKernelGGL(kern_reg, dim3(B * H, V / kHsCols), dim3(256), 0, stream, states,
-                         counts, (const TQ*)q, (const TQ*)k, (const TV*)v, (const TB*)beta, g,
-                         (const TL*)l, (TV*)o, G, H, K, V, L, cascade, strong, update, output, norm_qk,
-                         scale);
-    }
+  // Columns per workgroup: as many as fit 64 NV elements of whole [level] groups, in
+  // steps that keep every column block NV-aligned, evened out over the blocks.
+  auto columns = [&](int nv, int* nblk) {
+    const int step = nv / std::gcd(nv, a.LA), most = 64 * nv / a.LA / step * step;
+    if (most == 0) return 0;
+    *nblk = (a.V + most - 1) / most;
+    const int vb = ((a.V + *nblk - 1) / *nblk + step - 1) / step * step;
+    *nblk = (a.V + vb - 1) / vb;
+    return vb;
   };
-  with_type(dt_qk, [&](auto tq) {
-    using TQ = decltype(tq);
-    with_type(dt_v, [&](auto tv) {
-      using TV = decltype(tv);
-      with_type(dt_l, [&](auto tl) {
-        using TL = decltype(tl);
-        if (!gdn) {
-          if (L <= 16)
-            launch(hstate_step_lds_kernel<TQ, TV, TL, float, false, 16>,
-                   hstate_step_kernel<TQ, TV, TL, float, false>, tq, tv, tl, float{});
-          else
-            launch(hstate_step_lds_kernel<TQ, TV, TL, float, false, 32>,
-                   hstate_step_kernel<TQ, TV, TL, float, false>, tq, tv, tl, float{});
-          return;
-        }
-        with_type(dt_b, [&](auto tb) {
-          using TB = decltype(tb);
-          if (L <= 16)
-            launch(hstate_step_lds_kernel<TQ, TV, TL, TB, true, 16>,
-                   hstate_step_kernel<TQ, TV, TL, TB, true>, tq, tv, tl, tb);
-          else
-            launch(hstate_step_lds_kernel<TQ, TV, TL, TB, true, 32>,
-                   hstate_step_kernel<TQ, TV, TL, TB, true>, tq, tv, tl, tb);
-        });
-      });
-    });
-  });
-  if (err != hipSuccess) return err;
-  return hipGetLastError();
+  // The widest lane load that still gives two workgroups per CU; a single element
+  // per lane where the levels stepped are not contiguous, the state is not
+  // aligned, or a lane's elements would span more than two columns.
+  int nv = 4, nblk = 0;
+  for (; nv > 1; nv >>= 1) {
+    const bool fits = a.LA == a.L && !a.strong && a.LA >= nv && ((uintptr_t)a.states & (4 * nv - 1)) == 0;
+    if (fits && (a.VB = columns(nv, &nblk)) != 0 && (long)B * a.H * nblk >= kHsBlocks) break;
+  }
+  if (nv == 1) a.VB = columns(1, &nblk);
+  auto pick = [&](auto kind) {
+    constexpr int KIND = decltype(kind)::value;
+    if (a.strong) return launch_steps<KIND, 1, 16, true>(a, B, nblk, stream);
+    if (nv == 4) return a.K > 64 ? launch_steps<KIND, 4, 32>(a, B, nblk, stream)
+                                 : launch_steps<KIND, 4, 16, false, 64>(a, B, nblk, stream);
+    if (nv == 2) return launch_steps<KIND, 2, 16>(a, B, nblk, stream);
+    return launch_steps<KIND, 1, 16>(a, B, nblk, stream);
+  };
+  if (gdn) return pick(std::integral_constant<int, kHsGdelta>{});
+  return pick(std::integral_constant<int, kHsMamba2>{});
 }
 
 hipError_t hattn_mamba2_prefill_levels_launch(float* states, const void* k, const void* v,
                                               const float* g, int B, int T, int G, int H, int K,
                                               int V, int L, int nlo, int dt_k, int dt_v,
+                                              unsigned int clear, const HsCounts& counts,
                                               hipStream_t stream, int* unsupported) {
   using namespace hattn;
   const dim3 grid(B * H, V / kHsCols), block(256);
   *unsupported = 0;
-  const bool known = (dt_k == HS_BF16 || dt_k == HS_FP32) && (dt_v == HS_BF16 || dt_v == HS_FP32);
-  if (!known) {
+  if (!known_type(dt_k) || !known_type(dt_v)) {
     *unsupported = 1;
     return hipSuccess;
   }
@@ -591,7 +545,7 @@ hipError_t hattn_mamba2_prefill_levels_launch(float* states, const void* k, cons
     with_type(dt_v, [&](auto tv) {
       using TV = decltype(tv);
       hipLaunchKernelGGL((mamba2_prefill_levels_kernel<TK, TV>), grid, block, 0, stream, states,
-                         (const TK*)k, (const TV*)v, g, T, G, H, K, V, L, nlo);
+                         (const TK*)k, (const TV*)v, g, T, G, H, K, V, L, nlo, clear, counts);
     });
   });
   return hipGetLastError();

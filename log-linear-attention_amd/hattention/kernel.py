@@ -230,9 +230,9 @@ def postprocess_prefill_hstate_(hstate, q, k, v, b, g, l, scale, head_first, lev
     (7 for 64-token chunks) in ``hstate.states``; rebuild the levels below from
     the last chunk, then set the counts and clear the empty levels.
 
-    MAMBA2: one ``hattn_mamba2_prefill_levels`` launch (the einsums of
-    :418-436).  GDELTA: the recurrent form over the last chunk from a zero state
-    (:438-449), one ``hattn_hstate_step`` launch per token."""
+    One ``hattn_hstate_prefill_levels`` launch: for MAMBA2 the einsums of :418-436,
+    for GDELTA the recurrent form over the last chunk from a zero state
+    (:438-449)."""
     from hattention.base import get_num_levels
     from hattention import _lib
     from hattention import recurrent as _rec
@@ -255,28 +255,18 @@ def postprocess_prefill_hstate_(hstate, q, k, v, b, g, l, scale, head_first, lev
         raise ValueError("shape mismatch between the HState and q, k, v, g, l")
     if L < level_chunk:
         raise ValueError(f"{L} levels, the prefill needs at least {level_chunk}")
-    if hstruct == HStruct.MAMBA2:
-        k, v, g = k.contiguous(), v.contiguous(), g.float().contiguous()
-        dev = _lib.require_device(hstate.states, k, v, g)
-        _lib.check(_lib.load().hattn_mamba2_prefill_levels(
-            _lib.ptr(hstate.states), _lib.ptr(k), _lib.ptr(v), _lib.ptr(g), B, T, G, H, K, V,
-            L, level_chunk, _lib.dtype_code(k), _lib.dtype_code(v), _lib.stream_handle(dev)))
-    else:
-        if b is None:
-            raise ValueError
-        tmp = _rec.HState(base=level_base, htype=htype, hstruct=hstruct,
-                          shape=(B, H, K, V, level_chunk), dtype=hstate.dtype,
-                          device=hstate.device)
-        tm = lambda x: x[:, -chunk_size:].transpose(0, 1).contiguous()
-        k_t, v_t, b_t, g_t = tm(k), tm(v), tm(b), tm(g.float())
-        for t in range(chunk_size):
-            _rec.launch_step(tmp, k=k_t[t], v=v_t[t], beta=b_t[t], g=g_t[t], update=True,
-                             output=False, l2norm_qk=use_qk_l2norm_in_kernel, scale=scale)
-        hstate.states[..., :level_chunk] = tmp.states
-    counts, empty = _prefill_counts(T, L, level_base)
-    if empty:
-        hstate.states[..., empty] = 0
-    hstate.set_counts(counts)
+    if hstruct != HStruct.MAMBA2 and b is None:
+        raise ValueError
+    k, v, g = k.contiguous(), v.contiguous(), g.float().contiguous()
+    b = b.contiguous() if hstruct != HStruct.MAMBA2 else None
+    counts, _ = _prefill_counts(T, L, level_base)
+    dev = _lib.require_device(hstate.states, k, v, g, b)
+    _lib.check(_lib.load().hattn_hstate_prefill_levels(
+        _lib.ptr(hstate.states), _lib.ptr(hstate.counts), _lib.ptr(k), _lib.ptr(v), _lib.ptr(b),
+        _lib.ptr(g), B, T, G, H, K, V, L, level_chunk, hstruct.value, htype.value,
+        int(use_qk_l2norm_in_kernel), _lib.dtype_code(k), _lib.dtype_code(v),
+        _lib.dtype_code(b) if b is not None else 2, _lib.stream_handle(dev)))
+    hstate.host_counts = counts
     return hstate
 
 
@@ -284,8 +274,8 @@ def postprocess_prefill_hstate_(hstate, q, k, v, b, g, l, scale, head_first, lev
 def hattention_prefill(q, k, v, b, g, l, scale, head_first, level_base, htype, hstruct,
                        chunk_size=None, use_qk_l2norm_in_kernel=False):
     """kernel.py:467-574: chunkwise forward over the whole 64-token chunks with
-    the final level states, the low levels rebuilt from the last chunk, then one
-    decode step per remaining token.  Returns (o, hstate)."""
+    the final level states, the low levels rebuilt from the last chunk, then the
+    decode steps of the remaining tokens.  Returns (o, hstate)."""
     from hattention import recurrent as _rec
     if chunk_size is None:
         chunk_size = 64
@@ -295,7 +285,7 @@ def hattention_prefill(q, k, v, b, g, l, scale, head_first, level_base, htype, h
     _, _, H, V = v.shape
     _, _, _, L = l.shape
     T0 = T - (T % chunk_size) if htype == HType.WEAK else 0
-    o = torch.zeros_like(v)
+    o = torch.empty_like(v)
     hstate = _rec.HState(base=level_base, htype=htype, hstruct=hstruct, shape=(B, H, K, V, L),
                          dtype=g.dtype, device=g.device)
     if T0 != 0:
@@ -312,15 +302,12 @@ def hattention_prefill(q, k, v, b, g, l, scale, head_first, level_base, htype, h
         _check_step_args(hstate, q[:, T0], k[:, T0], v[:, T0],
                          b[:, T0] if b is not None else None, g[:, T0], l[:, T0], level_base,
                          htype, hstruct, use_qk_l2norm_in_kernel, scale)
-        tm = lambda x: x[:, T0:].transpose(0, 1).contiguous() if x is not None else None
-        q_t, k_t, v_t, b_t, g_t, l_t = tm(q), tm(k), tm(v), tm(b), tm(g), tm(l)
-        o_t = torch.empty_like(v_t)
-        for t in range(T - T0):
-            _rec.launch_step(hstate, q=q_t[t], k=k_t[t], v=v_t[t],
-                             beta=b_t[t] if b_t is not None else None, g=g_t[t], l=l_t[t],
-                             o=o_t[t], update=True, output=True,
-                             l2norm_qk=use_qk_l2norm_in_kernel, scale=scale)
-        o[:, T0:] = o_t.transpose(0, 1)
+        con = lambda x: x.contiguous() if x is not None else None
+        oc = con(o)
+        _rec.launch_steps(hstate, T0, T, q=con(q), k=con(k), v=con(v), beta=con(b), g=con(g),
+                          l=con(l), o=oc, l2norm_qk=use_qk_l2norm_in_kernel, scale=scale)
+        if oc is not o:
+            o.copy_(oc)
     return o, hstate
 
 

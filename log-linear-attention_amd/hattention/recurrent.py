@@ -7,8 +7,9 @@ Mirrors hattention/recurrent.py:9-216:
 * ``hattention_recurrent`` -- :169-216 (the token loop)
 
 The state lives in HBM in the reference's layout and is advanced in place by
-one ``hattn_hstate_step`` launch per token (libhattn_hip.so): cascade, gate,
-insert, and for ``hattention_step`` also the output.  The cascades (weak,
+one ``hattn_hstate_step`` launch per decoded token, or one ``hattn_hstate_steps``
+launch for a run of known tokens (libhattn_hip.so): cascade, gate, insert, and
+for ``hattention_step`` also the output.  The cascades (weak,
 :42-54, and strong, :56-74) depend only on the level counts, which depend only
 on the number of tokens inserted, so they are planned here on a host copy of
 the counts (``plan_cascade_weak`` / ``plan_cascade_strong``); the device
@@ -17,6 +18,7 @@ from the device.  Level base 2 only (other bases raise NotImplementedError, as
 the reference's strong check does); states are fp32, the dtype the reference
 gives them (state dtype = g.dtype, :185, kernel.py:505).
 """
+import ctypes
 from typing import List, Optional, Tuple
 
 import torch
@@ -220,6 +222,62 @@ def launch_step(S: HState, *, q=None, k=None, v=None, beta=None, g=None, l=None,
         _lib.check(status)
 
 
+MAX_TOKENS = 256   # tokens per hattn_hstate_steps launch
+
+
+def launch_steps(S: HState, t0: int, t1: int, *, q=None, k=None, v=None, beta=None, g=None,
+                 l=None, o=None, l2norm_qk: bool = False, scale: Optional[float] = None) -> None:
+    """Tokens t0 .. t1 - 1 of operands with a token axis (q, k [B, T, G, K]; v, o
+    [B, T, H, V]; beta, g [B, T, H]; l [B, T, H, L]; contiguous, on the state's
+    device), state update and, with ``o``, output: what ``launch_step`` does one
+    token at a time, up to MAX_TOKENS of them per ``hattn_hstate_steps`` launch.
+    Where a token's cascade cannot be planned (a level overflow), the tokens
+    before it are stepped and the error of ``plan_cascade`` is raised."""
+    _check_state(S)
+    st = S.states
+    if not st.is_cuda:
+        raise RuntimeError("hattention (MI355X) runs only on HIP device tensors; the HState "
+                           f"is on {st.device}")
+    B, H, K, V, L = S.shape
+    if k is None or v is None or g is None or (o is not None and (q is None or l is None)):
+        raise ValueError("missing operand for the step")
+    G, T = k.shape[2], k.shape[1]
+    for name, t, shape in (("q", q, (B, T, G, K)), ("k", k, (B, T, G, K)), ("v", v, (B, T, H, V)),
+                           ("beta", beta, (B, T, H)), ("g", g, (B, T, H)), ("l", l, (B, T, H, L)),
+                           ("o", o, (B, T, H, V))):
+        if t is not None and (t.shape != shape or not t.is_contiguous() or
+                              t.get_device() != st.get_device()):
+            raise _operand_error(name, t, shape, st.device)
+    if G <= 0 or H % G != 0:
+        raise ValueError(f"G={G} does not divide H={H}")
+    if g.dtype is not torch.float32:
+        raise TypeError("g must be float32")
+    if q is not None and q.dtype != k.dtype:
+        raise TypeError("q and k must share a dtype")
+    if o is not None and v.dtype != o.dtype:
+        raise TypeError("o must have v's dtype")
+    codes = (_lib.dtype_code(k), _lib.dtype_code(v), _lib.dtype_code(l) if l is not None else _FP32,
+             _lib.dtype_code(beta) if beta is not None else _FP32)
+    lib = _lib.load()
+    counts = (ctypes.c_int * L)(*S.host_counts)
+    cascades = (ctypes.c_ubyte * MAX_TOKENS)()
+    while t0 < t1:
+        want = min(t1 - t0, MAX_TOKENS)
+        n = lib.hattn_hstate_plan(counts, L, S.htype.value, want, cascades)
+        if n:
+            _lib.check(lib.hattn_hstate_steps(
+                st.data_ptr(), S.counts.data_ptr(), _lib.ptr(q), _lib.ptr(k), _lib.ptr(v),
+                _lib.ptr(beta), _lib.ptr(g), _lib.ptr(l), _lib.ptr(o), B, T, t0, n, G, H, K, V, L,
+                S.hstruct.value, S.htype.value, cascades, counts, int(o is not None),
+                int(l2norm_qk), float(scale if scale is not None else 1.0), *codes,
+                _lib.stream_handle(st.device)))
+            S.host_counts = list(counts)
+        if n < want:
+            S.plan_cascade()
+            raise ValueError("level count above capacity")
+        t0 += n
+
+
 def step_state(S: HState, k: torch.Tensor, v: torch.Tensor, a: torch.Tensor,
                b: Optional[torch.Tensor] = None) -> HState:
     """recurrent.py:134-156: k [B, H, K], v [B, H, V], gate a [B, H] (linear,
@@ -250,8 +308,8 @@ def step_output(S: HState, q: torch.Tensor, l: torch.Tensor,
 def hattention_recurrent(Q, K, V, A, B, L, base: int, htype: HType,
                          hstruct: HStruct) -> Tuple[torch.Tensor, HState]:
     """recurrent.py:169-216: Q, K [B, T, H, K]; V [B, T, H, V]; A [B, T, H] the
-    gate (linear, fp32); B [B, T, H] (GDELTA) or None; L [B, T, H, L].  One
-    fused step (update + output) per token."""
+    gate (linear, fp32); B [B, T, H] (GDELTA) or None; L [B, T, H, L].  The fused
+    steps (update + output) of up to MAX_TOKENS tokens per launch."""
     if not all([Q.shape == K.shape, Q.shape[:-1] == V.shape[:-1], Q.shape[:-1] == A.shape,
                 Q.shape[:-1] == L.shape[:-1], A.dtype == torch.float32, Q.dtype == K.dtype,
                 Q.dtype == V.dtype, Q.dtype == L.dtype]):
@@ -261,11 +319,8 @@ def hattention_recurrent(Q, K, V, A, B, L, base: int, htype: HType,
     Bsz, T, H, Kd = Q.shape
     S = HState(base=base, htype=htype, hstruct=hstruct,
                shape=(Bsz, H, Kd, V.shape[3], L.shape[-1]), dtype=A.dtype, device=Q.device)
-    tm = lambda x: x.transpose(0, 1).contiguous() if x is not None else None
-    q_t, k_t, v_t, l_t, b_t = tm(Q), tm(K), tm(V), tm(L), tm(B)
-    g_t = tm(torch.log(A))
-    o_t = torch.empty(T, Bsz, H, V.shape[3], dtype=V.dtype, device=V.device)
-    for t in range(T):
-        launch_step(S, q=q_t[t], k=k_t[t], v=v_t[t], beta=b_t[t] if b_t is not None else None,
-                    g=g_t[t], l=l_t[t], o=o_t[t], update=True, output=True)
-    return o_t.transpose(0, 1).contiguous(), S
+    con = lambda x: x.contiguous() if x is not None else None
+    o = torch.empty(Bsz, T, H, V.shape[3], dtype=V.dtype, device=V.device)
+    launch_steps(S, 0, T, q=con(Q), k=con(K), v=con(V), beta=con(B), g=torch.log(A).contiguous(),
+                 l=con(L), o=o)
+    return o, S
