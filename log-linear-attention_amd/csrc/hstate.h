@@ -8,7 +8,7 @@
 constexpr int kHsMaxLevels = 32;    // levels of a state
 constexpr int kHsMaxTokens = 256;   // tokens per launch: their cascades travel in the arguments
 enum { kHsMamba2 = 0, kHsGdelta = 1, kHsLayer = 2 };   // what a step is
-constexpr int kHsBlocks = 512;      // workgroups below which narrower column blocks are taken
+constexpr int kHsBlocks = 256;      // workgroups below which narrower column blocks are taken
 
 // The Mamba-2 layer's decode step (hselective_state_update): the kernel forms v, g
 // and lambda from the layer's inputs and adds the D residual.  HsArgs::v is x then,
@@ -30,6 +30,7 @@ struct HsArgs {
   int G, H, K, V, L;
   int LA;        // levels stepped: the first LA of the L
   int VB;        // value columns per workgroup (set by the launch)
+  int batch;     // tokens whose operands are in LDS at a time (set by the launch)
   int T, t0;     // tokens, the first one's index in the operands
   int strong, update, output, norm;
   int zero;      // start from an empty state instead of reading it

@@ -33,6 +33,7 @@ namespace hattn {
 
 constexpr int kHsCols = 16;   // value columns per workgroup of the prefill levels
 constexpr int kHsRowGroups = 256 / kHsCols;
+constexpr int kHsBatch = 8;   // tokens whose operands are in LDS at a time
 
 // The level counts (shared by all rows) after the step: the cascade (weak: levels
 // 0 .. c-1 merge into level c; strong: levels 0 .. m-1 move up one level, m - 1
@@ -58,12 +59,19 @@ __device__ inline void cascade_counts(int* counts, int L, int cascade, int stron
 
 // Element u + i, i < n, of a tensor with dtype code dt (0 bf16, 2 fp32); p, u and dt
 // are uniform.  Through a buffer descriptor: a lane keeps a 32-bit offset and no
-// address, and reads 0 from n on.
-__device__ __forceinline__ float hs_ld(const void* p, long long u, unsigned int i, int dt,
-                                       int n = 1) {
+// address, and reads 0 from n on.  hs_raw leaves the bits as loaded and hs_val makes
+// them a float, apart, so that a token's loads are all under way before the first
+// is waited for (converted within the branch on dt, each load was waited for on the
+// spot: 2 us a token).
+__device__ __forceinline__ unsigned int hs_raw(const void* p, long long u, unsigned int i, int dt,
+                                               int n = 1) {
   const int es = dt == 0 ? 2 : 4;
   const rsrc_t r = make_rsrc((const char*)p + u * es, (size_t)n * es);
-  return dt == 0 ? (float)buf_load<__bf16>(r, 2 * i, 0) : buf_load<float>(r, 4 * i, 0);
+  if (dt == 0) return __builtin_amdgcn_raw_buffer_load_b16(r, 2 * i, 0, 0);
+  return __builtin_amdgcn_raw_buffer_load_b32(r, 4 * i, 0, 0);
+}
+__device__ __forceinline__ float hs_val(unsigned int raw, int dt) {
+  return __builtin_bit_cast(float, raw << (dt == 0 ? 16 : 0));
 }
 __device__ __forceinline__ void hs_st(void* p, long long u, unsigned int i, float x, int dt) {
   if (dt == 0) ((__bf16*)p + u)[i] = (__bf16)x;
@@ -79,9 +87,6 @@ __device__ __forceinline__ float wave_sum(float x) {
 }
 // lane i gets lane i - 1's value, lane 0 gets 0 (wave_shr:1)
 __device__ __forceinline__ float lane_before(float x) { return dpp_f32<0x138, 0xf, true>(0.f, x); }
-__device__ __forceinline__ float lane_value(float x, int lane) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), lane));
-}
 
 // Token steps with the state in registers.
 //
@@ -93,26 +98,64 @@ __device__ __forceinline__ float lane_value(float x, int lane) {
 // through LDS and one launch a token, this took 109 us for a GDELTA step of B 4, H
 // 16, K = V = 128, L 18, and 14 us for each of the 64 tokens that rebuild the low
 // levels after a prefill.)
+//   operands  of a batch of tokens at a time in LDS, each token prepared by one
+//             wave (l2norm, the layer's v, g and lambda, q . k); the rows' k and q
+//             are then broadcast reads.  With every wave preparing every token for
+//             itself the 37 tokens after a GDELTA prefill took 6 us each.
 //   cascade   S[c] += S[0 .. c-1] is a sum over the c elements before S[c] in the
 //             flat [v][level] order: a shift along the lanes.
-//   u = k^T S, w = q^T S   sums over a wave's rows in registers (k, q of a row are
-//             wave-uniform: readlane), then over the waves through LDS, double
-//             buffered, so one barrier a token.
+//   u = k^T S, w = q^T S   sums over a wave's rows in registers, then over the
+//             waves through LDS: u at once (one barrier a token, GDELTA only), w
+//             at the end of the batch.
 //   update    S = a S - k (a beta u), level 0 = k (beta v)
 //   output    q^T S after the update = a (w - beta (q . k) u) per level, and
-//             (q . k) beta v at level 0; the first wave weights and sums the levels.
-// The next token's operands are loaded before the current token is computed.
+//             (q . k) beta v at level 0; weighted and summed over the levels at the
+//             end of the batch, one wave a token.
 // (STRONG is an instance of its own: the two cascades in one kernel cost 70 spilled
-// registers.)  NV (elements per lane) sets the number of workgroups: the host takes the widest
-// that still fills the chip.
+// registers.)  NV (elements per lane) sets the number of workgroups: the host takes
+// the widest that still fills the chip.  Measured: one GDELTA step of B 4, H 16, K =
+// V = 128, L 18 in 39 us (3.9 TB/s of the 4.8 that a copy reaches), 40 tokens at B
+// 1, H 16, K = V = 64 / 128 in 64 / 160 us: there the cascade's shifts and the
+// barrier of u bound a token.
+template <int NV>
+struct HsVec {
+  typedef float type __attribute__((ext_vector_type(NV)));
+};
+template <>
+struct HsVec<1> {
+  typedef float type;
+};
+template <int NV>
+__device__ __forceinline__ float hs_get(const typename HsVec<NV>::type& x, int i) {
+  if constexpr (NV == 1) return x;
+  else return x[i];
+}
+template <int NV>
+__device__ __forceinline__ void hs_set(typename HsVec<NV>::type& x, int i, float y) {
+  if constexpr (NV == 1) x = y;
+  else x[i] = y;
+}
+
 template <int KIND, int NV, int R, bool STRONG, int KMAX>
 __global__ __launch_bounds__(64 * KMAX / R) void hstate_steps_kernel(const HsArgs p) {
-  extern __shared__ float red[];     // [2][u, w][wave][64 NV]
-  __shared__ float part[64 * NV];    // weighted levels of the output, first wave only
-  typedef float vecN __attribute__((ext_vector_type(NV)));
+  typedef typename HsVec<NV>::type vecN;
   constexpr bool GDN = KIND == kHsGdelta, LAYER = KIND == kHsLayer;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), nw = blockDim.x >> 6;
+  const int KP = nw * R;
+  // dynamic LDS, nb tokens a batch: their k and q [nb][KP], the waves' w
+  // [nb][wave][64 NV], u summed over the waves [nb][64 NV], the waves' u
+  // [2][wave][64 NV]
+  extern __shared__ floatx4 dyn[];
+  const int nb = p.batch;
+  float* tok_k = (float*)dyn;
+  float* tok_q = tok_k + nb * KP;
+  float* red_w = tok_q + nb * KP;
+  float* sum_u = red_w + nb * nw * 64 * NV;
+  float* red_u = sum_u + nb * 64 * NV;
+  __shared__ float tok_l[kHsBatch][kHsMaxLevels], tok_v[kHsBatch][64], tok_x[LAYER ? kHsBatch : 1][64];
+  __shared__ float tok_s[kHsBatch][4];   // exp(g), beta, q . k
+
   const int bh = blockIdx.x, b = bh / p.H, h = bh - b * p.H, gq = h / (p.H / p.G);
   const int K = p.K, V = p.V, L = p.L, LA = p.LA;
   const int v0 = blockIdx.y * p.VB, vbc = p.VB < V - v0 ? p.VB : V - v0;
@@ -120,99 +163,119 @@ __global__ __launch_bounds__(64 * KMAX / R) void hstate_steps_kernel(const HsArg
   const int e0 = act ? lane * NV : 0;
   const int vv0 = e0 / LA, ll0 = e0 - vv0 * LA;
   int ll[NV];
-  int vi = v0 + vv0;   // column of this lane's level-0 element, if it has one
+  int vi = vv0;   // column of this lane's level-0 element, if it has one
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
     ll[i] = ll0 + i >= LA ? ll0 + i - LA : ll0 + i;
     if (i > 0 && ll[i] == 0) ++vi;
   }
-  if (vi >= V) vi = V - 1;   // a lane at the end that has none
-  // elements are contiguous unless only the first LA of L levels are stepped
-  // (NV = 1 then)
-  const unsigned int at0 = LA == L ? e0 : vv0 * L + ll0;
-  const int row0 = wave * R, klane = row0 & 63;
+  vi &= 63;       // (a lane at the end that has none)
+  // a lane's elements are contiguous unless only the first LA of L levels are stepped
+  const bool whole = LA == L;
+  const unsigned int at0 = whole ? e0 : vv0 * L + ll0;
+  const int row0 = wave * R;
   // (a uniform row address and a 32-bit lane offset: no address registers per row)
   float* base = p.states + (((size_t)bh * K + row0) * V + v0) * L;
   const int rstride = V * L;
+  auto at = [&](int i) { return at0 + i + (ll0 + i >= LA ? L - LA : 0); };
 
   float s[R][NV];
 #pragma unroll
   for (int r = 0; r < R; ++r) {
     vecN x{};
     if (!p.zero && row0 + r < K) x = *(const vecN*)(base + r * rstride + at0);
-    if constexpr (NV == 1) s[r][0] = x[0];
-    else
 #pragma unroll
-      for (int i = 0; i < NV; ++i) s[r][i] = x[i];
+    for (int i = 0; i < NV; ++i) s[r][i] = hs_get<NV>(x, i);
   }
 
-  struct Token {
-    float k[4], q[4], g, beta, v, lam[NV], x;
-  };
   const HsLayer& y = p.layer;
-  auto fetch = [&](int i0) {
-    Token n;
-    const int t = p.t0 + i0;
+  // token t0 + i0 + j of the batch at i0, prepared by one wave
+  auto prepare = [&](int i0, int j) {
+    const int t = p.t0 + i0 + j;
     const long long qo = b * p.q_b + t * p.q_t + gq * K, so = b * p.s_b + t * p.s_t + h;
     const long long vo = b * p.v_b + t * p.v_t + h * V, lo = b * p.l_b + t * p.l_t + h * L;
+    unsigned int kraw[4], qraw[4];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int i = lane + 64 * j;
-      n.k[j] = p.update && 64 * j < K ? hs_ld(p.k, qo, i, p.dt_qk, K) : 0.f;
-      n.q[j] = p.output && 64 * j < K ? hs_ld(p.q, qo, i, p.dt_qk, K) : 0.f;
+    for (int c = 0; c < 4; ++c) {
+      const int i = lane + 64 * c;
+      kraw[c] = p.update && 64 * c < K ? hs_raw(p.k, qo, i, p.dt_qk, K) : 0;
+      qraw[c] = p.output && 64 * c < K ? hs_raw(p.q, qo, i, p.dt_qk, K) : 0;
     }
-    n.beta = GDN && p.update ? hs_ld(p.beta, so, 0, p.dt_b) : 1.f;
-    n.x = 0.f;
-    n.v = p.update ? hs_ld(p.v, vo, vi, LAYER ? y.dt_x : p.dt_v, V) : 0.f;
+    const int dt_x = LAYER ? y.dt_x : p.dt_v;
+    const unsigned int graw = p.update && !LAYER ? hs_raw(p.g, so, 0, 2) : 0;
+    const unsigned int braw = GDN && p.update ? hs_raw(p.beta, so, 0, p.dt_b) : 0;
+    const unsigned int vraw = p.update ? hs_raw(p.v, vo, v0 + lane, dt_x, V) : 0;
+    const unsigned int lraw = p.output ? hs_raw(p.l, lo, lane, p.dt_l, L) : 0;
+    unsigned int draw = 0, biasraw = 0, araw = 0, lpraw = 0;
+    if (LAYER) {
+      draw = hs_raw(y.dt, so, 0, y.dt_dt);
+      if (y.bias) biasraw = hs_raw(y.bias, h, 0, y.dt_bias);
+      araw = hs_raw(y.A, h, 0, y.dt_A);
+      lpraw = hs_raw(y.Lp, h * L, lane, y.dt_Lp, L);
+    }
+    float kx[4], qx[4];
 #pragma unroll
-    for (int i = 0; i < NV; ++i) n.lam[i] = p.output ? hs_ld(p.l, lo, ll[i], p.dt_l, L) : 0.f;
+    for (int c = 0; c < 4; ++c) {
+      kx[c] = hs_val(kraw[c], p.dt_qk);
+      qx[c] = hs_val(qraw[c], p.dt_qk);
+    }
+    const float beta = GDN && p.update ? hs_val(braw, p.dt_b) : 1.f, xv = hs_val(vraw, dt_x);
+    float g = hs_val(graw, 2), vx = xv, lx = hs_val(lraw, p.dt_l);
     if (LAYER) {
       // the Mamba-2 layer's inputs: v = x dt', g = A dt', lambda of (L, dl), each
       // rounded to its dtype as the separate layer kernels do
-      const float d = layer_dtp(hs_ld(y.dt, so, 0, y.dt_dt),
-                                y.bias ? hs_ld(y.bias, h, 0, y.dt_bias) : 0.f, y.softplus);
-      n.g = layer_g(hs_ld(y.A, h, 0, y.dt_A), d);
-      n.v = hs_round(n.v * d, p.dt_v);
-#pragma unroll
-      for (int i = 0; i < NV; ++i)
-        n.lam[i] = hs_round(lambda_of(hs_ld(y.Lp, h * L, ll[i], y.dt_Lp, L), n.lam[i], y.mode), y.dt_lam);
-      if (y.D) n.x = hs_ld(p.v, vo, v0 + lane, y.dt_x, V);
-    } else {
-      n.g = p.update ? p.g[so] : 0.f;
+      const float d = layer_dtp(hs_val(draw, y.dt_dt), hs_val(biasraw, y.dt_bias), y.softplus);
+      g = layer_g(hs_val(araw, y.dt_A), d);
+      vx = hs_round(xv * d, p.dt_v);
+      lx = hs_round(lambda_of(hs_val(lpraw, y.dt_Lp), lx, y.mode), y.dt_lam);
+      tok_x[j][lane] = xv;
     }
-    return n;
-  };
-
-  Token nx = fetch(0);
-  for (int t = 0; t < p.T; ++t) {
-    Token tk = nx;
-    if (t + 1 < p.T) nx = fetch(t + 1);
     if (p.norm) {
       // q / |q| * scale, k / |k| (kernel.py:20-23, 626-629 with the eps of fla's
       // l2norm), rounded to the input dtype after the norm and after the scale, as
       // the reference's l2norm_fwd / l2norm_and_scale_fwd store their outputs
       float nq = 0.f, nk = 0.f;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        nq += tk.q[j] * tk.q[j];
-        nk += tk.k[j] * tk.k[j];
+      for (int c = 0; c < 4; ++c) {
+        nq += qx[c] * qx[c];
+        nk += kx[c] * kx[c];
       }
       const float rq = rsqrtf(wave_sum(nq) + 1e-6f), rk = rsqrtf(wave_sum(nk) + 1e-6f);
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        tk.q[j] = hs_round(hs_round(tk.q[j] * rq, p.dt_qk) * p.scale, p.dt_qk);
-        tk.k[j] = hs_round(tk.k[j] * rk, p.dt_qk);
+      for (int c = 0; c < 4; ++c) {
+        qx[c] = hs_round(hs_round(qx[c] * rq, p.dt_qk) * p.scale, p.dt_qk);
+        kx[c] = hs_round(kx[c] * rk, p.dt_qk);
       }
     }
     float qk = 0.f;
-    if (p.output && p.update) {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) qk += tk.q[j] * tk.k[j];
-      qk = wave_sum(qk);
+    for (int c = 0; c < 4; ++c) qk += qx[c] * kx[c];
+    qk = wave_sum(qk);
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+      if (lane + 64 * c < KP) {
+        tok_k[j * KP + lane + 64 * c] = kx[c];
+        tok_q[j * KP + lane + 64 * c] = qx[c];
+      }
+    tok_v[j][lane] = vx;
+    if (lane < kHsMaxLevels) tok_l[j][lane] = lx;
+    if (lane == 0) {
+      tok_s[j][0] = p.update ? __expf(g) : 1.f;
+      tok_s[j][1] = beta;
+      tok_s[j][2] = qk;
     }
-    const int kj = row0 >> 6;
-    const float kr = kj == 0 ? tk.k[0] : kj == 1 ? tk.k[1] : kj == 2 ? tk.k[2] : tk.k[3];
-    const float qr = kj == 0 ? tk.q[0] : kj == 1 ? tk.q[1] : kj == 2 ? tk.q[2] : tk.q[3];
+  };
+
+  for (int t = 0; t < p.T; ++t) {
+    const int j = t & (nb - 1);
+    if (j == 0) {
+      if (t > 0) __syncthreads();   // the last batch's output reads
+      for (int i = wave; i < nb && t + i < p.T; i += nw) prepare(t, i);
+      __syncthreads();
+    }
+    const float a = tok_s[j][0], beta = tok_s[j][1], qk = tok_s[j][2];
+    const floatx4* kr = (const floatx4*)(tok_k + j * KP + row0);
+    const floatx4* qr = (const floatx4*)(tok_q + j * KP + row0);
 
     if (p.update) {
       const int c = p.casc[t];
@@ -235,35 +298,63 @@ __global__ __launch_bounds__(64 * KMAX / R) void hstate_steps_kernel(const HsArg
         }
       } else {
         // cascade_weak: level 0 ends empty too (at c = 0 the insert overwrites it)
-        int at = c - ll0;           // this lane's element of level c, if it has one
-        if (at < 0) at += LA;
-        const bool has = at < NV;
-        const int lim = has ? c - at : -(1 << 20);
+        int own_c = c - ll0;        // this lane's element of level c, if it has one
+        if (own_c < 0) own_c += LA;
+        const bool has = own_c < NV;
+        const int lim = has ? c - own_c : -(1 << 20);
         bool own[NV];
 #pragma unroll
         for (int i = 0; i < NV; ++i) {
           keep[i] = ll[i] >= c && ll[i] > 0;
-          into[i] = i == at;
-          own[i] = has && i < at && at - i <= c;
+          into[i] = i == own_c && c > 0;
+          own[i] = has && i < own_c && own_c - i <= c;
         }
         const int far = (c + NV - 1) / NV;   // lanes before that hold levels below c
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-          float sum = 0.f, cur[NV];
+        auto hop = [&](int d, float (&cur)[NV], float& sum) {
 #pragma unroll
           for (int i = 0; i < NV; ++i) {
-            sum += own[i] ? s[r][i] : 0.f;
-            cur[i] = s[r][i];
+            cur[i] = lane_before(cur[i]);
+            sum += NV * d - i <= lim ? cur[i] : 0.f;
+          }
+        };
+        if constexpr (NV < 4) {
+          // the hops outside, the rows inside: straight code for a hop (a loop per row
+          // was half of a token)
+          float sum[R], cur[R][NV];
+#pragma unroll
+          for (int r = 0; r < R; ++r) {
+            sum[r] = 0.f;
+#pragma unroll
+            for (int i = 0; i < NV; ++i) {
+              sum[r] += own[i] ? s[r][i] : 0.f;
+              cur[r][i] = s[r][i];
+            }
           }
           for (int d = 1; d <= far; ++d)
 #pragma unroll
-            for (int i = 0; i < NV; ++i) {
-              cur[i] = lane_before(cur[i]);
-              sum += NV * d - i <= lim ? cur[i] : 0.f;
-            }
+            for (int r = 0; r < R; ++r) hop(d, cur[r], sum[r]);
 #pragma unroll
-          for (int i = 0; i < NV; ++i)
-            s[r][i] = (keep[i] ? s[r][i] : 0.f) + (into[i] && c > 0 ? sum : 0.f);
+          for (int r = 0; r < R; ++r)
+#pragma unroll
+            for (int i = 0; i < NV; ++i)
+              s[r][i] = (keep[i] ? s[r][i] : 0.f) + (into[i] ? sum[r] : 0.f);
+        } else {
+          // one hop reaches all levels below c <= NV; no registers to hold the hops of
+          // every row
+#pragma unroll
+          for (int r = 0; r < R; ++r) {
+            float sum = 0.f, cur[NV];
+#pragma unroll
+            for (int i = 0; i < NV; ++i) {
+              sum += own[i] ? s[r][i] : 0.f;
+              cur[i] = s[r][i];
+            }
+            hop(1, cur, sum);
+            for (int d = 2; d <= far; ++d) hop(d, cur, sum);
+#pragma unroll
+            for (int i = 0; i < NV; ++i)
+              s[r][i] = (keep[i] ? s[r][i] : 0.f) + (into[i] ? sum : 0.f);
+          }
         }
       }
     }
@@ -274,92 +365,93 @@ __global__ __launch_bounds__(64 * KMAX / R) void hstate_steps_kernel(const HsArg
     const bool need_u = GDN && p.update;
     if (need_u)
 #pragma unroll
-      for (int r = 0; r < R; ++r) {
-        const float kk = lane_value(kr, klane + r);
+      for (int r = 0; r < R; r += 4) {
+        const floatx4 kk = kr[r / 4];
 #pragma unroll
-        for (int i = 0; i < NV; ++i) u[i] += kk * s[r][i];
+        for (int m = 0; m < 4; ++m)
+#pragma unroll
+          for (int i = 0; i < NV; ++i) u[i] += kk[m] * s[r + m][i];
       }
     if (p.output)
 #pragma unroll
-      for (int r = 0; r < R; ++r) {
-        const float qq = lane_value(qr, klane + r);
+      for (int r = 0; r < R; r += 4) {
+        const floatx4 qq = qr[r / 4];
 #pragma unroll
-        for (int i = 0; i < NV; ++i) w[i] += qq * s[r][i];
-      }
-    float* ru = red + (size_t)(t & 1) * 2 * nw * 64 * NV;
-    float* rw = ru + nw * 64 * NV;
-    if (need_u || p.output) {
-      vecN x;
-      if (need_u) {
-        if constexpr (NV == 1) x = u[0];
-        else
+        for (int m = 0; m < 4; ++m)
 #pragma unroll
-          for (int i = 0; i < NV; ++i) x[i] = u[i];
-        *(vecN*)(ru + (wave * 64 + lane) * NV) = x;
+          for (int i = 0; i < NV; ++i) w[i] += qq[m] * s[r + m][i];
       }
-      if (p.output) {
-        if constexpr (NV == 1) x = w[0];
-        else
+    vecN x;
+    if (p.output) {
 #pragma unroll
-          for (int i = 0; i < NV; ++i) x[i] = w[i];
-        *(vecN*)(rw + (wave * 64 + lane) * NV) = x;
-      }
-      __syncthreads();
-      if (need_u) {
-        vecN acc{};
-        for (int j = 0; j < nw; ++j) acc += *(const vecN*)(ru + (j * 64 + lane) * NV);
-        if constexpr (NV == 1) u[0] = acc[0];
-        else
-#pragma unroll
-          for (int i = 0; i < NV; ++i) u[i] = acc[i];
-      }
+      for (int i = 0; i < NV; ++i) hs_set<NV>(x, i, w[i]);
+      *(vecN*)(red_w + ((j * nw + wave) * 64 + lane) * NV) = x;
     }
-
-    const float a = p.update ? __expf(tk.g) : 1.f;
-    if (p.output && wave == 0) {
+    if (need_u) {
+      float* ru = red_u + (t & 1) * nw * 64 * NV;
+#pragma unroll
+      for (int i = 0; i < NV; ++i) hs_set<NV>(x, i, u[i]);
+      *(vecN*)(ru + (wave * 64 + lane) * NV) = x;
+      __syncthreads();
       vecN acc{};
-      for (int j = 0; j < nw; ++j) acc += *(const vecN*)(rw + (j * 64 + lane) * NV);
-      if constexpr (NV == 1) w[0] = acc[0];
-      else
+      for (int i = 0; i < nw; ++i) acc += *(const vecN*)(ru + (i * 64 + lane) * NV);
 #pragma unroll
-        for (int i = 0; i < NV; ++i) w[i] = acc[i];
-#pragma unroll
-      for (int i = 0; i < NV; ++i) {
-        float z = w[i];
-        if (p.update) {
-          z = GDN ? a * (z - tk.beta * qk * u[i]) : a * z;
-          if (ll[i] == 0) z = qk * (tk.beta * tk.v);
-        }
-        if (act) part[e0 + i] = tk.lam[i] * z;
-      }
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-      if (lane < vbc) {
-        float z = 0.f;
-        for (int e = 0; e < LA; ++e) z += part[lane * LA + e];
-        const long long oo = b * p.o_b + (p.t0 + t) * p.o_t + h * V + v0;
-        if (LAYER) {
-          z = hs_round(z, p.dt_v);
-          if (y.D) z = layer_out(z, tk.x, hs_ld(y.D, h, 0, y.dt_D));
-        }
-        hs_st(p.o, oo, lane, z, LAYER ? y.dt_out : p.dt_v);
-      }
-      __builtin_amdgcn_wave_barrier();
+      for (int i = 0; i < NV; ++i) u[i] = hs_get<NV>(acc, i);
+      if (p.output && wave == 0) *(vecN*)(sum_u + (j * 64 + lane) * NV) = acc;
     }
 
     if (p.update) {
-      float m[NV], kr2 = kr;
-      asm("" : "+v"(kr2));   // read the rows' k again instead of holding R scalars
+      float m[NV];
+      const float vx = beta * tok_v[j][vi];
 #pragma unroll
-      for (int i = 0; i < NV; ++i) m[i] = ll[i] == 0 ? tk.beta * tk.v : -(a * tk.beta) * u[i];
+      for (int i = 0; i < NV; ++i) m[i] = ll[i] == 0 ? vx : -(a * beta) * u[i];
 #pragma unroll
-      for (int r = 0; r < R; ++r) {
-        const float kk = lane_value(kr2, klane + r);
+      for (int r = 0; r < R; r += 4) {
+        const floatx4 kk = kr[r / 4];
+#pragma unroll
+        for (int n = 0; n < 4; ++n)
+#pragma unroll
+          for (int i = 0; i < NV; ++i) {
+            float& z = s[r + n][i];
+            if (GDN) z = __builtin_fmaf(kk[n], m[i], a * z);
+            else z = ll[i] == 0 ? kk[n] * m[i] : a * z;
+          }
+      }
+    }
+
+    if (p.output && (j == nb - 1 || t + 1 == p.T)) {
+      __syncthreads();
+      for (int n = wave; n <= j; n += nw) {
+        const float an = tok_s[n][0], bn = tok_s[n][1], qkn = tok_s[n][2];
+        float* rw = red_w + (n * nw * 64 + lane) * NV;
+        vecN acc{}, un{};
+        for (int i = 0; i < nw; ++i) acc += *(const vecN*)(rw + i * 64 * NV);
+        if (need_u) un = *(const vecN*)(sum_u + (n * 64 + lane) * NV);
 #pragma unroll
         for (int i = 0; i < NV; ++i) {
-          if (GDN) s[r][i] = __builtin_fmaf(kk, m[i], a * s[r][i]);
-          else s[r][i] = ll[i] == 0 ? kk * m[i] : a * s[r][i];
+          float z = hs_get<NV>(acc, i);
+          if (p.update) {
+            z = GDN ? an * (z - bn * qkn * hs_get<NV>(un, i)) : an * z;
+            if (ll[i] == 0) z = qkn * (bn * tok_v[n][vi]);
+          }
+          hs_set<NV>(acc, i, tok_l[n][ll[i]] * z);
+        }
+        // this wave alone reads and writes token n's sums
+        *(vecN*)rw = acc;
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        if (lane < vbc) {
+          const float* part = red_w + n * nw * 64 * NV + lane * LA;
+          float z = 0.f;
+#pragma unroll 8
+          for (int e = 0; e < LA; ++e) z += part[e];
+          const long long oo = b * p.o_b + (p.t0 + t - j + n) * p.o_t + h * V + v0;
+          if (LAYER) {
+            z = hs_round(z, p.dt_v);
+            if (y.D) z = layer_out(z, tok_x[n][lane], hs_val(hs_raw(y.D, h, 0, y.dt_D), y.dt_D));
+          }
+          hs_st(p.o, oo, lane, z, LAYER ? y.dt_out : p.dt_v);
         }
       }
     }
@@ -369,12 +461,15 @@ __global__ __launch_bounds__(64 * KMAX / R) void hstate_steps_kernel(const HsArg
 #pragma unroll
     for (int r = 0; r < R; ++r)
       if (row0 + r < K) {
-        vecN x;
-        if constexpr (NV == 1) x = s[r][0];
-        else
+        if (whole) {
+          vecN x;
 #pragma unroll
-          for (int i = 0; i < NV; ++i) x[i] = s[r][i];
-        *(vecN*)(base + r * rstride + at0) = x;
+          for (int i = 0; i < NV; ++i) hs_set<NV>(x, i, s[r][i]);
+          *(vecN*)(base + r * rstride + at0) = x;
+        } else {
+#pragma unroll
+          for (int i = 0; i < NV; ++i) base[r * rstride + at(i)] = s[r][i];
+        }
       }
   // levels above the stepped ones that end empty
   if (p.clear)
@@ -477,9 +572,13 @@ bool with_type(int dt, F&& f) {
 bool known_type(int dt) { return dt == HS_BF16 || dt == HS_FP32; }
 
 template <int KIND, int NV, int R, bool STRONG = false, int KMAX = 256>
-hipError_t launch_steps(const HsArgs& a, int B, int nblk, hipStream_t stream) {
+hipError_t launch_steps(HsArgs a, int B, int nblk, hipStream_t stream) {
   const int nw = (a.K + R - 1) / R;
-  const size_t smem = (size_t)2 * 2 * nw * 64 * NV * sizeof(float);
+  // (a power of two; four tokens at K > 128, where eight would leave one workgroup
+  // per CU)
+  a.batch = a.T == 1 ? 1 : a.K > 128 ? 4 : hattn::kHsBatch;
+  const size_t smem =
+      (size_t)(a.batch * (2 * nw * R + (nw + 1) * 64 * NV) + 2 * nw * 64 * NV) * sizeof(float);
   hipLaunchKernelGGL((hattn::hstate_steps_kernel<KIND, NV, R, STRONG, KMAX>), dim3(B * a.H, nblk), dim3(64 * nw),
                      smem, stream, a);
   return hipGetLastError();
@@ -507,12 +606,12 @@ hipError_t hattn_hstate_steps_launch(HsArgs a, int B, int gdn, hipStream_t strea
     *nblk = (a.V + vb - 1) / vb;
     return vb;
   };
-  // The widest lane load that still gives two workgroups per CU; a single element
-  // per lane where the levels stepped are not contiguous, the state is not
-  // aligned, or a lane's elements would span more than two columns.
+  // The widest lane load that still gives kHsBlocks workgroups; narrower where the
+  // state is not aligned or a lane's elements would span more than two columns.
   int nv = 4, nblk = 0;
   for (; nv > 1; nv >>= 1) {
-    const bool fits = a.LA == a.L && !a.strong && a.LA >= nv && ((uintptr_t)a.states & (4 * nv - 1)) == 0;
+    const bool fits = !a.strong && a.LA >= nv &&
+                      (a.LA == a.L ? ((uintptr_t)a.states & (4 * nv - 1)) == 0 : a.zero != 0);
     if (fits && (a.VB = columns(nv, &nblk)) != 0 && (long)B * a.H * nblk >= kHsBlocks) break;
   }
   if (nv == 1) a.VB = columns(1, &nblk);

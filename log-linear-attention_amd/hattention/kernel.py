@@ -289,13 +289,14 @@ def hattention_prefill(q, k, v, b, g, l, scale, head_first, level_base, htype, h
     hstate = _rec.HState(base=level_base, htype=htype, hstruct=hstruct, shape=(B, H, K, V, L),
                          dtype=g.dtype, device=g.device)
     if T0 != 0:
+        # the whole chunks of every operand, copied (where they are a part) once
+        qc, kc, vc, bc, gc, lc = (x[:, :T0].contiguous() if x is not None else None
+                                  for x in (q, k, v, b, g, l))
         o[:, :T0], hstate.states = HAttentionPrefillFunction.apply(
-            q[:, :T0], k[:, :T0], v[:, :T0], b[:, :T0] if b is not None else None, g[:, :T0],
-            l[:, :T0], scale, head_first, level_base, htype, hstruct, chunk_size,
+            qc, kc, vc, bc, gc, lc, scale, head_first, level_base, htype, hstruct, chunk_size,
             use_qk_l2norm_in_kernel)
         postprocess_prefill_hstate_(
-            hstate=hstate, q=q[:, :T0], k=k[:, :T0], v=v[:, :T0],
-            b=b[:, :T0] if b is not None else None, g=g[:, :T0], l=l[:, :T0], scale=scale,
+            hstate=hstate, q=qc, k=kc, v=vc, b=bc, g=gc, l=lc, scale=scale,
             head_first=head_first, level_base=level_base, htype=htype, hstruct=hstruct,
             chunk_size=chunk_size, use_qk_l2norm_in_kernel=use_qk_l2norm_in_kernel)
     if T0 < T:
