@@ -438,6 +438,26 @@ int hattn_hstate_steps(float* states, int* counts, const void* q, const void* k,
                        int dtype_beta, void* stream);
 
 /*
+ * One decode step of the Mamba-2 layer in one launch.
+ *
+ * Replaces hattention/mamba_apis.py:407-566 `hselective_state_update`: the layer
+ * pre-processing of one token (as hattn_mamba2_layer_prologue: d = dt + dt_bias,
+ * softplus(d) if dt_softplus; v = x d; g = A[h] d; lam = compute_lambda(Lp[h], dl)),
+ * hattn_hstate_step with q = C, k = B, and out = o + x D[h] (out = o without D).
+ *
+ * x, out [B, H, P]; dt [B, H]; A, dt_bias (or NULL), D (or NULL) [H]; Bm, Cm
+ * [B, G, N] in one dtype; dl [B, H, L]; Lp [H, L].  dtypes: the codes (BF16 or FP32)
+ * of x, dt, A, dt_bias, Bm and Cm, dl, Lp, D, v, lam, out, in this order; v, o and
+ * lam are rounded to theirs.  Constraints: those of hattn_hstate_step (K = N,
+ * V = P), P a multiple of 4 with P / 4 a power of two <= 64.
+ */
+int hattn_mamba2_layer_step(float* states, int* counts, const void* x, const void* dt,
+                            const void* A, const void* dt_bias, const void* Bm, const void* Cm,
+                            const void* dl, const void* Lp, const void* D, void* out, int B,
+                            int G, int H, int P, int N, int L, int htype, int cascade,
+                            int dt_softplus, int lambda_mode, const int* dtypes, void* stream);
+
+/*
  * What turns the final states of a chunkwise prefill of T tokens (T % 64 == 0)
  * into an HState: levels 0 .. nlo - 1 rebuilt from the last chunk, the levels
  * above that hold no token set to zero, and the level counts stored to counts

@@ -969,6 +969,36 @@ int layer_dims_check(int B, int T, int H, int P, int L) {
 }
 }  // namespace
 
+int hattn_mamba2_layer_step(float* states, int* counts, const void* x, const void* dt,
+                            const void* A, const void* dt_bias, const void* Bm, const void* Cm,
+                            const void* dl, const void* Lp, const void* D, void* out, int B,
+                            int G, int H, int P, int N, int L, int htype, int cascade,
+                            int dt_softplus, int lambda_mode, const int* dtypes, void* stream) {
+  if (int st = layer_dims_check(B, 1, H, P, L)) return st;
+  if (int st = hs_check(B, G, H, N, P, L, HATTN_HSTRUCT_MAMBA2, htype)) return st;
+  if (int st = hs_cascade_check(cascade, L, htype, 1)) return st;
+  if (lambda_mode < 0 || lambda_mode > 2) return fail(HATTN_ERR_VALUE, "lambda_mode=%d", lambda_mode);
+  if (!states || !x || !dt || !A || !Bm || !Cm || !dl || !Lp || !out || !dtypes)
+    return fail(HATTN_ERR_VALUE, "null tensor pointer");
+  for (int i = 0; i < 11; ++i)
+    if (bf_flag(dtypes[i]) < 0) return fail(HATTN_ERR_NOT_IMPLEMENTED, "dtype code (bf16 or fp32 only)");
+  HsArgs a = hs_args(states, counts, Cm, Bm, x, nullptr, nullptr, dl, out, 1, 0, 1, G, H, N, P, L);
+  a.strong = htype == HATTN_HTYPE_STRONG;
+  a.update = a.output = 1;
+  a.casc[0] = (unsigned char)cascade;
+  a.dt_qk = dtypes[4];
+  a.dt_l = dtypes[5];
+  a.dt_v = dtypes[8];
+  HsLayer& y = a.layer;
+  y.on = 1;
+  y.dt = dt; y.A = A; y.bias = dt_bias; y.Lp = Lp; y.D = D;
+  y.softplus = dt_softplus != 0;
+  y.mode = lambda_mode;
+  y.dt_x = dtypes[0]; y.dt_dt = dtypes[1]; y.dt_A = dtypes[2]; y.dt_bias = dtypes[3];
+  y.dt_Lp = dtypes[6]; y.dt_D = dtypes[7]; y.dt_lam = dtypes[9]; y.dt_out = dtypes[10];
+  return hs_launch(a, B, HATTN_HSTRUCT_MAMBA2, (hipStream_t)stream, "hattn_mamba2_layer_step launch");
+}
+
 int hattn_mamba2_layer_prologue(const void* x, const void* dt, const float* A,
                                 const float* dt_bias, const void* dl, const void* Lp, void* v,
                                 float* g, void* lam, int B, int T, int H, int P, int L,

@@ -624,6 +624,7 @@ hipError_t hattn_hstate_steps_launch(HsArgs a, int B, int gdn, hipStream_t strea
     return launch_steps<KIND, 1, 16>(a, B, nblk, stream);
   };
   if (gdn) return pick(std::integral_constant<int, kHsGdelta>{});
+  if (y.on) return pick(std::integral_constant<int, kHsLayer>{});
   return pick(std::integral_constant<int, kHsMamba2>{});
 }
 

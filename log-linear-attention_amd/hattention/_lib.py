@@ -57,6 +57,7 @@ SIGNATURES = [
     ("hattn_hstate_plan", _I, [_P, _I, _I, _I, _P]),
     ("hattn_hstate_steps", _I,
      [_P] * 9 + [_I] * 11 + [_P, _P, _I, _I, ctypes.c_float] + [_I] * 4 + [_P]),
+    ("hattn_mamba2_layer_step", _I, [_P] * 12 + [_I] * 10 + [_P, _P]),
     ("hattn_hstate_prefill_levels", _I, [_P] * 6 + [_I] * 14 + [_P]),
     ("hattn_mamba2_prefill_levels", _I, [_P] * 4 + [_I] * 10 + [_P]),
     ("hattn_mamba2_layer_prologue", _I, [_P] * 9 + [_I] * 13 + [_P]),

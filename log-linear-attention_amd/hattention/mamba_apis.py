@@ -333,10 +333,10 @@ def hselective_state_update(
 
     x [B,H,P], dt [B,H], A [H], B/C [B,G,N], dl [B,H,L], L [H,L], D [H].
     Returns (out [B,H,P], state advanced in place).  The dt / A / lambda
-    pre-processing is elementwise torch on the device; the state step is one
-    ``hattn_hstate_step`` launch (q = C, k = B, v = x * dt, g = A * dt).
+    pre-processing, the state step (q = C, k = B, v = x * dt, g = A * dt) and the D
+    residual are one ``hattn_mamba2_layer_step`` launch.
     """
-    from hattention.recurrent import launch_step
+    from hattention.recurrent import launch_layer_step
     if state_batch_indices is not None:
         raise NotImplementedError
     if z is not None:
@@ -384,13 +384,7 @@ def hselective_state_update(
                 state.base == lambda_level_base, state.htype == lambda_htype,
                 state.hstruct == lambda_hstruct]):
         raise TypeError
-    # one token: the layer prologue on [B, 1, H, .] views, one step launch, the epilogue
-    v, g, lam = layer_prologue(x.unsqueeze(1), dt.unsqueeze(1), A, dt_bias, dl.unsqueeze(1), L,
-                               dt_softplus, lambda_mode)
-    v, g, lam = v.squeeze(1), g.squeeze(1), lam.squeeze(1)
-    out = torch.empty_like(v)
-    launch_step(state, q=C.contiguous(), k=B.contiguous(), v=v, g=g, l=lam, o=out, update=True,
-                output=True)
-    if D is not None:
-        out = layer_epilogue(out.unsqueeze(1), x.unsqueeze(1), D).squeeze(1)
-    return out, state
+    # one launch: v = x dt', g = A dt' and lambda from the layer's inputs, the state
+    # step, and the D residual
+    return launch_layer_step(state, x, dt, A, dt_bias, B, C, dl, L, D, dt_softplus, lambda_mode,
+                             x_dtype, lam_dtype), state

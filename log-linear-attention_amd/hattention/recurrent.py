@@ -222,6 +222,57 @@ def launch_step(S: HState, *, q=None, k=None, v=None, beta=None, g=None, l=None,
         _lib.check(status)
 
 
+def launch_layer_step(S: HState, x, dt, A, dt_bias, Bm, Cm, dl, Lp, D, dt_softplus: bool,
+                      lambda_mode: Optional[str], v_dtype: torch.dtype,
+                      lam_dtype: torch.dtype) -> torch.Tensor:
+    """One ``hattn_mamba2_layer_step`` launch: the decode step of the Mamba-2 layer
+    on checked operands (x [B, H, P], dt [B, H], A, dt_bias, D [H], Bm, Cm [B, G, N],
+    dl [B, H, L], Lp [H, L]); returns out [B, H, P].  ``v_dtype`` and ``lam_dtype``
+    are those of v = x dt' and of lambda."""
+    from hattention.mamba_layer import lambda_mode_code
+    mode = lambda_mode_code(lambda_mode)
+    _check_state(S)
+    st = S.states
+    if not st.is_cuda:
+        raise RuntimeError("hattention (MI355X) runs only on HIP device tensors; the HState "
+                           f"is on {st.device}")
+    B, H, N, P, L = S.shape
+    didx = st.get_device()
+    ops = []
+    for name, t in (("x", x), ("dt", dt), ("A", A), ("dt_bias", dt_bias), ("B", Bm), ("C", Cm),
+                    ("dl", dl), ("L", Lp), ("D", D)):
+        if t is not None:
+            if t.get_device() != didx:
+                raise _operand_error(name, t, tuple(t.shape), st.device)
+            t = t.contiguous()
+        ops.append(t)
+    x, dt, A, dt_bias, Bm, Cm, dl, Lp, D = ops
+    if x.shape != (B, H, P) or Bm.shape[0] != B or Bm.shape[2] != N or dl.shape != (B, H, L):
+        raise ValueError(f"the state {tuple(S.shape)} does not fit the operands")
+    out_dtype = v_dtype if D is None else \
+        torch.promote_types(v_dtype, torch.promote_types(x.dtype, D.dtype))
+    out = torch.empty(B, H, P, dtype=out_dtype, device=st.device)
+    dc = _lib.DTYPE_CODES
+    try:
+        codes = (ctypes.c_int * 11)(
+            dc[x.dtype], dc[dt.dtype], dc[A.dtype], dc[dt_bias.dtype] if dt_bias is not None else _FP32,
+            dc[Bm.dtype], dc[dl.dtype], dc[Lp.dtype], dc[D.dtype] if D is not None else _FP32,
+            dc[v_dtype], dc[lam_dtype], dc[out_dtype])
+    except KeyError as e:
+        raise NotImplementedError(f"unsupported dtype {e}") from None
+    saved = S.host_counts
+    cascade = S.plan_cascade()
+    status = _lib.load().hattn_mamba2_layer_step(
+        st.data_ptr(), S.counts.data_ptr(), x.data_ptr(), dt.data_ptr(), A.data_ptr(),
+        _lib.ptr(dt_bias), Bm.data_ptr(), Cm.data_ptr(), dl.data_ptr(), Lp.data_ptr(), _lib.ptr(D),
+        out.data_ptr(), B, Bm.shape[1], H, P, N, L, S.htype.value, cascade, int(bool(dt_softplus)),
+        mode, codes, _lib.stream_handle(st.device))
+    if status:
+        S.host_counts = saved
+        _lib.check(status)
+    return out
+
+
 MAX_TOKENS = 256   # tokens per hattn_hstate_steps launch
 
 
