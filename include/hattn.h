@@ -372,6 +372,31 @@ int hattn_gdn_chunkwise_bwd_fwd_ws(const void* q, const void* k, const void* v, 
 size_t hattn_gdn_chunkwise_bwd_fwd_ws_workspace(int B, int T, int H, int K, int V, int L);
 
 /*
+ * hattn_gdn_chunkwise_fwd_keep and the backward for V any multiple of 64 in one call
+ * (the level sums and the chunk-local products run over all of V).  With
+ * fwd_workspace (from the keeping forward on the same inputs) the backward takes
+ * q_new, W_new, K_new, U and the level states from it, with NULL it recomputes them.
+ * Workspaces: hattn_gdn_chunkwise_fwd_keep_workspace;
+ * hattn_gdn_chunkwise_bwd_fwd_ws_workspace with a forward workspace, else
+ * hattn_gdn_chunkwise_bwd_workspace.  No counterpart in the reference.
+ */
+int hattn_gdn_chunkwise_fwd_keep_any_v(const void* q, const void* k, const void* v,
+                                       const void* beta, const float* g, const void* l, void* o,
+                                       float* g_cumsum, void* Aw, void* Au, float* ht, int B,
+                                       int T, int H, int K, int V, int L, int dtype_qkv,
+                                       int dtype_beta, int dtype_l, int dtype_o, int level_base,
+                                       int htype, int chunk_size, int l2norm_qk, float qk_scale,
+                                       void* workspace, size_t workspace_bytes, void* stream);
+int hattn_gdn_chunkwise_bwd_any_v(const void* q, const void* k, const void* v, const void* beta,
+                                  const float* g_cumsum, const void* l, const void* do_, void* dq,
+                                  void* dk, void* dv, void* db, float* dg, float* dl, int B, int T,
+                                  int H, int K, int V, int L, int dtype_qkv, int dtype_beta,
+                                  int dtype_l, int dtype_do, int level_base, int htype,
+                                  int chunk_size, int l2norm_qk, float qk_scale, void* workspace,
+                                  size_t workspace_bytes, const void* fwd_workspace,
+                                  size_t fwd_workspace_bytes, void* stream);
+
+/*
  * One decode step of the Fenwick level state (HState) for every (b, h).
  *
  * Replaces hattention/kernel.py:577-633 `hattention_step(hstate, q, k, v, b, g, l,

@@ -18,18 +18,24 @@
 // (rd / wr: bit e of c set / clear; nr: c is not the last chunk of an aligned
 // 2^(e+1) block).
 //
-// Four launches:
+// Launches:
 //   1. prep recompute (gdn_fwd.hip, from g_cumsum): q_new, K_new, W_new, U;
-//   2. forward scan recompute: every level's state at every chunk start, bf16;
-//   3. gdn_bwd_scan_kernel, one workgroup per (row, 32 columns of V), walks the
-//      chunks backwards with every level's dh [K x 32] in fp32 registers:
-//        dV_new = K_new dh_{c+1},   dU += wr dV_new,
-//        dq_new += rd lambda_e o (dO h_c^T),  dlambda_e = rd rowsum(dO o q_new h_c),
-//        dW_new -= nr dV_new h_c^T,  dK_new += V_new dh_{c+1}^T,
-//        d exp(Gc_last) += nr <h_c, dh_{c+1}>,
+//   2. forward scan recompute: the state of every level that a chunk reads, at the
+//      chunk's start, bf16 (both skipped where the forward kept their results);
+//   3. gdn_dh_scan_kernel walks the chunks backwards and stores dh_{c+1} of every level:
+//        dV_new = K_new dh_{c+1},
 //        dh_c = nr (exp(Gc_last) dh_{c+1} - W_new^T dV_new) + rd q_new^T (lambda_e o dO);
-//      the contractions over V give per-slice partials (bf16), summed in fp32 by kernel 4;
-//   4. gdn_bwd_chunk_kernel, one workgroup per chunk, backpropagates through
+//   4. gdn_bwd_level_kernel, one workgroup per chunk, sums the rest over the levels:
+//        dU = sum_e wr K_new dh_{c+1},
+//        dq_new = sum_e rd lambda_e o (dO h_c^T),   dlambda_e = rd rowdot(q_new, dO h_c^T),
+//        Z = sum_e nr h_c dh_{c+1}^T  [K x K],      d exp(Gc_last) = trace Z,
+//        dW_new = -K_new Z^T,   dK_new = U (sum_e wr dh_{c+1})^T - W_new Z.
+//      A level with bit e clear (wr) is in the first half of its block, whose chunks
+//      so far are the blocks of the set bits j below e: h_e = sum_{j < e, j set} h_j.
+//      So only the states of set bits are stored and
+//        Z = sum_{j set} h_j (nr dh_j + sum_{e > j, e clear} dh_e)^T;
+//      a strong chunk's read of a clear level is one of each of those h_j as well;
+//   5. gdn_bwd_chunk_kernel, one workgroup per chunk, backpropagates through
 //      the chunk-local algebra.  With X = e o dq_new and E = dP - (X K^T) o beta_s,
 //        dM = tril(E Aw^T),  dAw = M^T E + ((e o dW_new) K^T + (dU V^T) o Gamma) o beta_s,
 //        dA = -strict-tril(Aw^T dAw Aw^T),
@@ -40,7 +46,7 @@
 //      dg = reverse chunk-local cumsum of dGc (chunkwise_hgdn.py:1219).  The
 //      64 x 64 products with fp32 operands run as bf16x3 (three MFMAs); the
 //      inverse is recomputed in fp32, so the Aw / Au of the forward are not read.
-#include "gdn_common.h"
+#include "gdn_bwd.h"
 
 hipError_t hattn_gdn_recompute_launch(const void* q, const void* k, const void* v,
                                       const void* beta, const float* gcum, const void* l,
@@ -52,325 +58,7 @@ hipError_t hattn_gdn_recompute_launch(const void* q, const void* k, const void* 
 namespace hattn {
 
 // ---------------------------------------------------------------------------
-// Kernel 3: reverse level scan
-// ---------------------------------------------------------------------------
-template <int KD>
-struct GdnBscanSmem {
-  static constexpr int LK = KD + 8, LVS = kBVs + 8;
-  __bf16 qn[kGC * LK];
-  __bf16 wn[kGC * LK];
-  __bf16 kn[kGC * LK];
-  __bf16 u[kGC * LVS];       // U[t][v] slice
-  __bf16 dO[kGC * LVS];      // dO[t][v] slice
-  __bf16 ldo[kGC * LVS];     // lambda[t, 7 + e] dO[t][v] of the current level e
-  __bf16 hs[kBVs * LK];      // h_e at the chunk start, [v][k]
-  __bf16 dhs[kBVs * LK];     // dh_e after the chunk, [v][k]
-  __bf16 dvn[kBVs * kLd64];  // dV_new_e, [v][t]
-  __bf16 vn[kBVs * kLd64];   // V_new_e, [v][t]
-  float lam[kGBwdMaxLev][kGC];  // lambda[t, 7 + e]
-  float dlr[2][kGC];         // dlambda row sums of the two 16-column halves
-  float red[8];
-};
-
-// NW = 8 waves (the wave-count parameter keeps the tile map general).  With
-// VTW = 8 / NW, wave w owns: dh tiles (k-tile, v-tile) = ((w TPW + j) >> 1,
-// (w TPW + j) & 1), TPW = VTW K / 64; the [64 x 32] products of step (i) at
-// (t-tile w & 3, v-tile (w >> 2) VTW + x), x < VTW; the [64 x K] accumulators at
-// t-tile w & 3, k-tiles ((w >> 2) VTW + x) APW + j, APW = K / 32.  At K = 192
-// every level's dh (96 registers) and the three accumulators (72) leave too
-// few registers for the products and some values spill.
-template <int KD>
-constexpr int gdn_bscan_waves() { return 8; }
-
-// E: the 16-bit format of q_new, W_new, K_new, U, dO and the saved states (bf16,
-// or fp16 for fp16 inputs; fp16 MFMA).  The per-V-slice partial gradients are
-// bf16 either way (summed in fp32 by the chunk kernel).
-template <int KD, typename TL, typename E = __bf16>
-__global__ __launch_bounds__(64 * gdn_bscan_waves<KD>(), 1) void gdn_bwd_scan_kernel(
-    const __bf16* __restrict__ qn, const __bf16* __restrict__ wn, const __bf16* __restrict__ kn,
-    const __bf16* __restrict__ un, const __bf16* __restrict__ dO, const float* __restrict__ gcum,
-    const TL* __restrict__ l, const __bf16* __restrict__ hsave, __bf16* __restrict__ dq_p,
-    __bf16* __restrict__ dw_p, __bf16* __restrict__ dk_p, float* __restrict__ du,
-    float* __restrict__ dl_p, float* __restrict__ del_p, int B, int T, int H, int V, int L,
-    int nlev, int strong) {
-  using Sm = GdnBscanSmem<KD>;
-  extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
-  Sm& s = *(Sm*)smem_raw;
-  constexpr int NW = gdn_bscan_waves<KD>(), NTH = 64 * NW, VTW = 8 / NW;
-  constexpr int LK = Sm::LK, LVS = Sm::LVS, TPW = VTW * KD / 64, APW = KD / 32;
-  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int lq = lane >> 4, ln = lane & 15;
-  const int tt = w & 3, vt0 = (w >> 2) * VTW;   // step (i) tiles; tt is also the accumulators' t-tile
-  const int nvb = V / kBVs;
-  const int vb = blockIdx.x % nvb;
-  const int row = blockIdx.x / nvb;
-  const int b = row / H, h = row % H;
-  const int NT = T / kGC;
-  const size_t hk = (size_t)H * KD, hv = (size_t)H * V;
-  const size_t BTH = (size_t)B * T * H;
-  const int v0 = vb * kBVs;
-
-  floatx4 dh[kGBwdMaxLev][TPW];
-#pragma unroll
-  for (int e = 0; e < kGBwdMaxLev; ++e)
-#pragma unroll
-    for (int j = 0; j < TPW; ++j) dh[e][j] = zero4();
-
-  // Register prefetch: the saved state of the next (chunk, level) pair is
-  // loaded while the current level computes (thread tid owns 16-byte unit tid
-  // of the [32 x K] slice), and the next chunk's q_new / W_new / K_new / U / dO
-  // tiles, lambda columns and last decay while the current chunk computes
-  // (K = 64 only: with K = 128 those registers would spill, and the tiles are
-  // loaded at the chunk start).  Every load is issued unconditionally, clamped
-  // to a valid address where its value is not used: a load under a condition
-  // makes the compiler merge its registers after the branch, which waits for
-  // the load right away.
-  constexpr bool kPrefTiles = KD <= 64;
-  constexpr int UPR = KD / 8, QU = kGC * UPR / NTH;   // units per row / per thread
-  constexpr int HU = (kBVs * UPR + NTH - 1) / NTH;     // units of the saved state per thread
-  static_assert(kGC * UPR % NTH == 0 && kGC * kBVs / 8 <= NTH, "units per thread");
-  const __bf16* hsrow = hsave + (size_t)row * NT * nlev * V * KD + (size_t)v0 * KD;
-  u32x4 ph[HU];
-  auto fetch_h = [&](int jc, int e) __attribute__((always_inline)) {
-#pragma unroll
-    for (int i = 0; i < HU; ++i) {
-      const int u = (tid + NTH * i) % (kBVs * UPR);
-      ph[i] = *(const u32x4*)(hsrow + ((size_t)jc * nlev + e) * V * KD + (size_t)(u / UPR) * KD +
-                              8 * (u % UPR));
-    }
-  };
-  u32x4 pq[QU], pw[QU], pk[QU], pu, pdo;
-  float plam, peL;
-  auto fetch_tiles = [&](int jc) __attribute__((always_inline)) {
-    const size_t t0 = (size_t)b * T + (size_t)jc * kGC;
-#pragma unroll
-    for (int i = 0; i < QU; ++i) {
-      const int u = tid + NTH * i, r = u / UPR, c = 8 * (u % UPR);
-      const size_t off = (t0 + r) * hk + (size_t)h * KD + c;
-      pq[i] = *(const u32x4*)(qn + off);
-      pw[i] = *(const u32x4*)(wn + off);
-      pk[i] = *(const u32x4*)(kn + off);
-    }
-    {
-      const int u = tid % (kGC * kBVs / 8);
-      const size_t off = (t0 + (u >> 2)) * hv + (size_t)h * V + v0 + 8 * (u & 3);
-      pu = *(const u32x4*)(un + off);
-      pdo = *(const u32x4*)(dO + off);
-    }
-    const int nl1 = nlev > 0 ? nlev : 1;   // T = 64 has no inter-chunk level
-    const int le = min(tid, nl1 * kGC - 1);
-    plam = to_f32<TL>(l[((t0 + le / nl1) * H + h) * L + min(7 + le % nl1, L - 1)]);
-    peL = gcum[(t0 + kGC - 1) * H + h];
-  };
-  if (kPrefTiles) fetch_tiles(NT - 1);
-  fetch_h(NT - 1, 0);
-  const rsrc_t rdl = make_rsrc(dl_p + ((size_t)vb * BTH + h) * nlev,
-                               w == 0 ? (size_t)B * T * H * nlev * 4 : 0);
-
-  for (int ic = NT - 1; ic >= 0; --ic) {
-    const size_t tok0 = (size_t)b * T + (size_t)ic * kGC;
-    if (!kPrefTiles) fetch_tiles(ic);
-#pragma unroll
-    for (int i = 0; i < QU; ++i) {
-      const int u = tid + NTH * i, r = u / UPR, c = 8 * (u % UPR);
-      *(u32x4*)(s.qn + r * LK + c) = pq[i];
-      *(u32x4*)(s.wn + r * LK + c) = pw[i];
-      *(u32x4*)(s.kn + r * LK + c) = pk[i];
-    }
-    if (tid < kGC * kBVs / 8) {
-      *(u32x4*)(s.u + (tid >> 2) * LVS + 8 * (tid & 3)) = pu;
-      *(u32x4*)(s.dO + (tid >> 2) * LVS + 8 * (tid & 3)) = pdo;
-    }
-    if (tid < nlev * kGC) s.lam[tid % nlev][tid / nlev] = plam;
-    const float eL = fexp(peL);
-    // the first level's barrier publishes the tiles; the prefetch registers are
-    // reloaded after it
-
-    floatx4 adq[VTW * APW], adw[VTW * APW], adk[VTW * APW], adu[VTW];
-#pragma unroll
-    for (int j = 0; j < VTW * APW; ++j) adq[j] = adw[j] = adk[j] = zero4();
-#pragma unroll
-    for (int x = 0; x < VTW; ++x) adu[x] = zero4();
-    float del = 0.f;
-
-    // the level loop stays rolled (an unrolled one holds every level's fragments
-    // at once); slot 0 of the dh array is the current level and the array
-    // rotates by one level per iteration (kGBwdMaxLev iterations, the levels
-    // >= nlev only rotating), so it is only indexed by constants.  The level's
-    // read / write / no-reset flags enter the products as 0 / 1 factors or
-    // operand selects, so that its LDS reads and MFMAs issue without a branch
-    // per product.
-#pragma unroll 1
-    for (int e = 0; e < kGBwdMaxLev; ++e) {
-      floatx4 cur[TPW];
-#pragma unroll
-      for (int j = 0; j < TPW; ++j) cur[j] = dh[0][j];
-      if (e < nlev) {
-        const int per = 2 << e;
-        const bool bit = (ic >> e) & 1;
-        // the forward's level read: bit e set; strong: every chunk reads every
-        // level >= 1 and none reads level 0 (the writes keep the weak masks)
-        const bool rd = strong ? e >= 1 : bit;
-        const bool nr = (ic & (per - 1)) != per - 1;
-        const float frd = rd ? 1.f : 0.f, fwr = bit ? 0.f : 1.f, fnr = nr ? 1.f : 0.f;
-#pragma unroll
-        for (int i = 0; i < HU; ++i) {
-          const int u = tid + NTH * i;
-          if (u < kBVs * UPR) *(u32x4*)(s.hs + (u / UPR) * LK + 8 * (u % UPR)) = ph[i];
-        }
-#pragma unroll
-        for (int j = 0; j < TPW; ++j) {
-          const int kt = (w * TPW + j) >> 1, vv = (w * TPW + j) & 1;
-          *(bf16x4*)(s.dhs + (16 * vv + ln) * LK + 16 * kt + 4 * lq) = cvt4e<E>(cur[j]);
-        }
-        __syncthreads();
-        {
-          const bool nxt = e + 1 < nlev;
-          fetch_h(nxt ? ic : max(ic - 1, 0), nxt ? e + 1 : 0);
-        }
-        if (kPrefTiles && e == 0) fetch_tiles(max(ic - 1, 0));
-        // lambda_e o dO, once per level for the products of steps (ii), (iii): written
-        // after the barrier that publishes the chunk's dO and lambda (and that
-        // orders it after the previous level's readers), read after the next one
-        for (int u = tid; u < kGC * kBVs / 4; u += NTH) {
-          const int t = u / (kBVs / 4), c = 4 * (u % (kBVs / 4));
-          const float la = s.lam[e][t];
-          const bf16x4 x = *(const bf16x4*)(s.dO + t * LVS + c);
-          *(bf16x4*)(s.ldo + t * LVS + c) =
-              bf16x4{to16<E>(from16<E>(x[0]) * la), to16<E>(from16<E>(x[1]) * la),
-                     to16<E>(from16<E>(x[2]) * la), to16<E>(from16<E>(x[3]) * la)};
-        }
-
-        // (i) dV_new = K_new dh, V_new = wr U - nr W_new h, q_new h (for dlambda)
-#pragma unroll
-        for (int x = 0; x < VTW; ++x) {
-          const int vt = vt0 + x;
-          floatx4 dv = zero4(), y = zero4(), z = zero4();
-#pragma unroll
-          for (int c = 0; c < KD / 32; ++c) {
-            // bound the operand loads in flight (registers) for the wide K
-            if (KD > 128) __builtin_amdgcn_sched_barrier(0);
-            const bf16x8 bd = *(const bf16x8*)(s.dhs + (16 * vt + ln) * LK + 32 * c + 8 * lq);
-            const bf16x8 bh = *(const bf16x8*)(s.hs + (16 * vt + ln) * LK + 32 * c + 8 * lq);
-            dv = mfma16<E>(*(const bf16x8*)(s.kn + (16 * tt + ln) * LK + 32 * c + 8 * lq), bd, dv);
-            y = mfma16<E>(*(const bf16x8*)(s.wn + (16 * tt + ln) * LK + 32 * c + 8 * lq), bh, y);
-            z = mfma16<E>(*(const bf16x8*)(s.qn + (16 * tt + ln) * LK + 32 * c + 8 * lq), bh, z);
-          }
-          bf16x4 dvb, vnb;
-          float dlr[4];
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const int t = 16 * tt + 4 * lq + i;
-            vnb[i] = to16<E>(fwr * from16<E>(s.u[t * LVS + 16 * vt + ln]) - fnr * y[i]);
-            dvb[i] = to16<E>(dv[i]);
-            adu[x][i] += fwr * dv[i];
-            dlr[i] = frd * from16<E>(s.dO[t * LVS + 16 * vt + ln]) * z[i];
-          }
-          *(bf16x4*)(s.dvn + (16 * vt + ln) * kLd64 + 16 * tt + 4 * lq) = dvb;
-          *(bf16x4*)(s.vn + (16 * vt + ln) * kLd64 + 16 * tt + 4 * lq) = vnb;
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const float xs = row_sum16(dlr[i]);
-            if (ln == 0) s.dlr[vt][16 * tt + 4 * lq + i] = xs;
-          }
-        }
-        __syncthreads();
-        // wave 0's lanes store the level's dlambda row sums; the other waves store
-        // through an empty range, so the store is unconditional and the memory
-        // waits of the walk count exactly
-        buf_store<float>(s.dlr[0][lane] + s.dlr[1][lane], rdl,
-                         (unsigned int)((lane * H) * nlev + e) * 4, (unsigned int)(tok0 * H * nlev * 4));
-
-        // (ii) contractions over this slice's 32 columns of V
-        {
-          // A operands with the level's factors in their rows (t = 16 tt + ln): the
-          // staged lambda_e o dO, and the read / no-reset flags as selects, so the
-          // three accumulators take plain MFMA accumulation
-          const bf16x8 ldo8 = *(const bf16x8*)(s.ldo + (16 * tt + ln) * LVS + 8 * lq);
-          const bf16x8 dvn8 = tr_frag(s.dvn, kLd64, 0, 16 * tt);   // dV_new[t][v]
-          const bf16x8 adO = rd ? ldo8 : bf16x8{};
-          const bf16x8 advn = nr ? dvn8 : bf16x8{};
-          const bf16x8 avn = tr_frag(s.vn, kLd64, 0, 16 * tt);     // V_new[t][v]
-#pragma unroll
-          for (int j = 0; j < VTW * APW; ++j) {
-            if (KD > 128 && (j & 1) == 0) __builtin_amdgcn_sched_barrier(0);
-            const int kt = vt0 * APW + j;
-            const bf16x8 bh = tr_frag(s.hs, LK, 0, 16 * kt);    // h^T[v][k]
-            const bf16x8 bd = tr_frag(s.dhs, LK, 0, 16 * kt);   // dh^T[v][k]
-            adq[j] = mfma16<E>(adO, bh, adq[j]);
-            adw[j] = mfma16<E>(advn, bh, adw[j]);
-            adk[j] = mfma16<E>(avn, bd, adk[j]);
-          }
-          float dd = 0.f;
-#pragma unroll
-          for (int j = 0; j < TPW; ++j) {
-            const int kt = (w * TPW + j) >> 1, vv = (w * TPW + j) & 1;
-            const bf16x4 hv4 = *(const bf16x4*)(s.hs + (16 * vv + ln) * LK + 16 * kt + 4 * lq);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) dd += from16<E>(hv4[i]) * cur[j][i];
-          }
-          del += fnr * dd;
-        }
-
-        // (iii) dh_e <- nr (eL dh_e - W_new^T dV_new) + rd q_new^T (lambda_e o dO)
-#pragma unroll
-        for (int j = 0; j < TPW; ++j) {
-          if (KD > 128) __builtin_amdgcn_sched_barrier(0);
-          const int kt = (w * TPW + j) >> 1, vv = (w * TPW + j) & 1;
-          floatx4 tw = zero4(), tq = zero4();
-#pragma unroll
-          for (int c = 0; c < 2; ++c) {
-            const bf16x8 bdv = *(const bf16x8*)(s.dvn + (16 * vv + ln) * kLd64 + 32 * c + 8 * lq);
-            tw = mfma16<E>(tr_frag(s.wn, LK, 32 * c, 16 * kt), bdv, tw);
-            const bf16x8 x = tr_frag(s.ldo, LVS, 32 * c, 16 * vv);   // (lambda_e o dO)[t][v]
-            tq = mfma16<E>(tr_frag(s.qn, LK, 32 * c, 16 * kt), x, tq);
-          }
-#pragma unroll
-          for (int i = 0; i < 4; ++i) cur[j][i] = fnr * (eL * cur[j][i] - tw[i]) + frd * tq[i];
-        }
-        __syncthreads();
-      }
-      // rotate: level e + 1 moves to slot 0; after all kGBwdMaxLev steps every
-      // level is back in its own slot
-#pragma unroll
-      for (int l = 0; l + 1 < kGBwdMaxLev; ++l)
-#pragma unroll
-        for (int j = 0; j < TPW; ++j) dh[l][j] = dh[l + 1][j];
-#pragma unroll
-      for (int j = 0; j < TPW; ++j) dh[kGBwdMaxLev - 1][j] = cur[j];
-    }
-
-    // ---- the chunk's outputs -----------------------------------------------------
-#pragma unroll
-    for (int j = 0; j < VTW * APW; ++j)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const size_t o = ((size_t)vb * BTH + (tok0 + 16 * tt + 4 * lq + i) * H + h) * KD +
-                         16 * (vt0 * APW + j) + ln;
-        dq_p[o] = (__bf16)adq[j][i];
-        dw_p[o] = (__bf16)-adw[j][i];
-        dk_p[o] = (__bf16)adk[j][i];
-      }
-#pragma unroll
-    for (int x = 0; x < VTW; ++x)
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        du[((tok0 + 16 * tt + 4 * lq + i) * H + h) * V + v0 + 16 * (vt0 + x) + ln] = adu[x][i];
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) del += __shfl_xor(del, off, 64);
-    if (lane == 0) s.red[w] = del;
-    __syncthreads();
-    if (tid == 0) {
-      float x = 0.f;
-#pragma unroll
-      for (int w2 = 0; w2 < NW; ++w2) x += s.red[w2];
-      del_p[(size_t)vb * B * H * NT + (size_t)row * NT + ic] = x;
-    }
-  }
-}
-
-// ---------------------------------------------------------------------------
-// Kernel 4: chunk-local backward
+// Kernel 5: chunk-local backward
 // ---------------------------------------------------------------------------
 // QG (K > 192): q is not staged in LDS (the tile would not fit next to the
 // fp32 matrices); its fragments come from global memory (L2) and each
@@ -589,21 +277,20 @@ __global__ __launch_bounds__(256, 1) void gdn_bwd_chunk_kernel(
     const __bf16* __restrict__ dk_p, const float* __restrict__ du, const float* __restrict__ dl_p,
     const float* __restrict__ del_p, __bf16* __restrict__ dq, __bf16* __restrict__ dk,
     __bf16* __restrict__ dv, TB* __restrict__ db, float* __restrict__ dg, float* __restrict__ dl,
-    int B, int T, int H, int L, int nlev, int norm_qk, float qk_scale) {
+    int B, int T, int H, int V, int L, int nlev, int norm_qk, float qk_scale) {
   using Sm = GdnBchunkSmem<KD, VD>;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
   Sm& s = *(Sm*)smem_raw;
   constexpr int LK = Sm::LK, LS = Sm::LS, LDB = Sm::LDB, NKT = KD / 16;
-  constexpr int NPV = VD / kBVs;   // V slices of the level scan = partials per entry
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lq = lane >> 4, ln = lane & 15;
   const int NT = T / kGC;
   const int ic = blockIdx.x % NT, row = blockIdx.x / NT;
   const int b = row / H, h = row % H;
   const size_t tok0 = (size_t)b * T + (size_t)ic * kGC;
-  const size_t hk = (size_t)H * KD, hv = (size_t)H * VD;
-  const size_t BTH = (size_t)B * T * H;
-  const size_t rowk = (tok0 * H + h) * KD, rowv = (tok0 * H + h) * VD;
+  const int VN = VD ? VD : V;   // columns of V
+  const size_t hk = (size_t)H * KD, hv = (size_t)H * VN;
+  const size_t rowk = (tok0 * H + h) * KD, rowv = (tok0 * H + h) * VN;
   float* S0 = s.m[0];
   float* S1 = s.m[1];
   float* S2 = s.m[2];
@@ -721,23 +408,33 @@ __global__ __launch_bounds__(256, 1) void gdn_bwd_chunk_kernel(
   __syncthreads();
 
   // step 5's fragments of X = e o dq_new (partials) are loaded while step 4 computes
-  FrgPf<NPV, __bf16> pfx[KD / 32];
+  FrgPf<1, __bf16> pfx[KD / 32];
 #pragma unroll
-  for (int c = 0; c < KD / 32; ++c) frg_load(pfx[c], dq_p + rowk, hk, BTH * KD, t16, 32 * c);
+  for (int c = 0; c < KD / 32; ++c) frg_load(pfx[c], dq_p + rowk, hk, 0, t16, 32 * c);
 
   // ---- 4: Z = dO V^T; Z o P o Gamma -> S0, dP = Z o Gamma o Lambda o beta_s -> S4 -----
   {
-    bf16x8 ad[VD / 32];
+    // (all of dO's fragments at once where V is a constant, two at a time elsewhere)
+    floatx4 zt[4];
 #pragma unroll
-    for (int c = 0; c < VD / 32; ++c) ad[c] = *(const bf16x8*)(dO + rowv + (size_t)(t16 + ln) * hv + 32 * c + 8 * lq);
+    for (int nt = 0; nt < 4; ++nt) zt[nt] = zero4();
+    constexpr int NF = VD ? VD / 32 : 2;
+    for (int c0 = 0; c0 < VN / 32; c0 += NF) {
+      bf16x8 ad[NF];
+#pragma unroll
+      for (int c = 0; c < NF; ++c)
+        ad[c] = *(const bf16x8*)(dO + rowv + (size_t)(t16 + ln) * hv + 32 * (c0 + c) + 8 * lq);
+#pragma unroll
+      for (int nt = 0; nt < 4; ++nt)
+        if (nt <= w) {
+#pragma unroll
+          for (int c = 0; c < NF; ++c)
+            zt[nt] = mfma16<E>(ad[c], *(const bf16x8*)(v + rowv + (size_t)(16 * nt + ln) * hv + 32 * (c0 + c) + 8 * lq), zt[nt]);
+        }
+    }
 #pragma unroll
     for (int nt = 0; nt < 4; ++nt) {
-      floatx4 z = zero4();
-      if (nt <= w) {
-#pragma unroll
-        for (int c = 0; c < VD / 32; ++c)
-          z = mfma16<E>(ad[c], *(const bf16x8*)(v + rowv + (size_t)(16 * nt + ln) * hv + 32 * c + 8 * lq), z);
-      }
+      const floatx4 z = zt[nt];
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int t = t16 + 4 * lq + i, sc = 16 * nt + ln;
@@ -819,12 +516,13 @@ __global__ __launch_bounds__(256, 1) void gdn_bwd_chunk_kernel(
   __syncthreads();
 
   // step 7's fragments of e o dW_new (partials) and dU are loaded while step 6 computes
-  FrgPf<NPV, __bf16> pfw[KD / 32];
-  FrgPf<1, float> pfu[VD / 32];
+  FrgPf<1, __bf16> pfw[KD / 32];
+  constexpr int NFU = VD ? VD / 32 : 1;
+  FrgPf<1, float> pfu[NFU];
 #pragma unroll
-  for (int c = 0; c < KD / 32; ++c) frg_load(pfw[c], dw_p + rowk, hk, BTH * KD, t16, 32 * c);
+  for (int c = 0; c < KD / 32; ++c) frg_load(pfw[c], dw_p + rowk, hk, 0, t16, 32 * c);
 #pragma unroll
-  for (int c = 0; c < VD / 32; ++c) frg_load(pfu[c], du + rowv, hv, 0, t16, 32 * c);
+  for (int c = 0; c < NFU; ++c) frg_load(pfu[c], du + rowv, hv, 0, t16, 32 * c);
 
   // ---- 6: H = (F1 beta) Aw^T, D = E Aw^T; dGc_t -= rowsum(M o H); dM = tril(D) -> S0 --
   {
@@ -868,21 +566,33 @@ __global__ __launch_bounds__(256, 1) void gdn_bwd_chunk_kernel(
   // ---- 7: F2 = (e o dW_new) K^T, F3 = dU V^T; (F2 + F3 o Gamma) o beta_s -> S5;
   //         dGc from the W_new factor e and the Gamma of Au --------------------------
   {
-    float a2[KD / 32][8], a3[VD / 32][8];
+    float a2[KD / 32][8];
 #pragma unroll
     for (int c = 0; c < KD / 32; ++c) frg_done(pfw[c], s.e[t16 + ln], a2[c]);
+    floatx4 f3t[4];
 #pragma unroll
-    for (int c = 0; c < VD / 32; ++c) frg_done(pfu[c], 1.f, a3[c]);
+    for (int nt = 0; nt < 4; ++nt) f3t[nt] = zero4();
+    for (int c0 = 0; c0 < VN / 32; c0 += NFU) {
+      float a3[NFU][8];
+#pragma unroll
+      for (int c = 0; c < NFU; ++c) frg_done(pfu[c], 1.f, a3[c]);
+      if (c0 + NFU < VN / 32)
+#pragma unroll
+        for (int c = 0; c < NFU; ++c) frg_load(pfu[c], du + rowv, hv, 0, t16, 32 * (c0 + NFU + c));
+#pragma unroll
+      for (int nt = 0; nt < 4; ++nt)
+#pragma unroll
+        for (int c = 0; c < NFU; ++c)
+          f3t[nt] = mma_fb<E>(a3[c], *(const bf16x8*)(v + rowv + (size_t)(16 * nt + ln) * hv + 32 * (c0 + c) + 8 * lq), f3t[nt]);
+    }
     float rs[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int nt = 0; nt < 4; ++nt) {
-      floatx4 f2 = zero4(), f3 = zero4();
+      floatx4 f2 = zero4();
+      const floatx4 f3 = f3t[nt];
 #pragma unroll
       for (int c = 0; c < KD / 32; ++c)
         f2 = mma_fb<E>(a2[c], *(const bf16x8*)(s.k + (16 * nt + ln) * LK + 32 * c + 8 * lq), f2);
-#pragma unroll
-      for (int c = 0; c < VD / 32; ++c)
-        f3 = mma_fb<E>(a3[c], *(const bf16x8*)(v + rowv + (size_t)(16 * nt + ln) * hv + 32 * c + 8 * lq), f3);
       float cs = 0.f;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
@@ -923,8 +633,8 @@ __global__ __launch_bounds__(256, 1) void gdn_bwd_chunk_kernel(
 
   // the kb loop's first partial block (X) is loaded while steps 9 compute
   constexpr bool PF = KD <= 128;   // partial blocks prefetched into registers
-  RowsPf<NPV> pf;
-  if constexpr (PF) rows_load<NPV>(pf, dq_p + rowk, hk, BTH * KD);
+  RowsPf<1> pf;
+  if constexpr (PF) rows_load<1>(pf, dq_p + rowk, hk, 0);
 
   // ---- 9: Y = dAw Aw^T -> S1; dA = -strict-tril(Aw^T Y) -> S1 --------------------------
   {
@@ -997,10 +707,10 @@ __global__ __launch_bounds__(256, 1) void gdn_bwd_chunk_kernel(
     // ---- 10: X -> ST; dQ = X + dM K; U2 = -P^T X; dGc += rowdot(X, Q) ----------------
     // (PF: each block's partial loads are issued one step before it is staged)
     if constexpr (PF) {
-      rows_store<LS, NPV>(ST, pf, s.e);
-      rows_load<NPV>(pf, dw_p + rowk + k0, hk, BTH * KD);
+      rows_store<LS, 1>(ST, pf, s.e);
+      rows_load<1>(pf, dw_p + rowk + k0, hk, 0);
     } else {
-      stage_rows<64, LS, NPV>(ST, dq_p + rowk + k0, hk, BTH * KD, s.e);
+      stage_rows<64, LS, 1>(ST, dq_p + rowk + k0, hk, 0, s.e);
     }
     __syncthreads();
     floatx4 u2[4];
@@ -1030,10 +740,10 @@ __global__ __launch_bounds__(256, 1) void gdn_bwd_chunk_kernel(
 
     // ---- 11: e o dW_new -> ST; U2 += Aw^T ST ---------------------------------------------
     if constexpr (PF) {
-      rows_store<LS, NPV>(ST, pf, s.e);
-      rows_load<NPV>(pf, dk_p + rowk + k0, hk, BTH * KD);
+      rows_store<LS, 1>(ST, pf, s.e);
+      rows_load<1>(pf, dk_p + rowk + k0, hk, 0);
     } else {
-      stage_rows<64, LS, NPV>(ST, dw_p + rowk + k0, hk, BTH * KD, s.e);
+      stage_rows<64, LS, 1>(ST, dw_p + rowk + k0, hk, 0, s.e);
     }
     __syncthreads();
 #pragma unroll
@@ -1071,10 +781,10 @@ __global__ __launch_bounds__(256, 1) void gdn_bwd_chunk_kernel(
 
     // ---- 13: dK_new -> ST; dK = U1 + beta o U2 + r o dK_new; dbeta, dGc of K_new -------
     if constexpr (PF) {
-      rows_store<LS, NPV>(ST, pf, nullptr);
-      if (kb + 1 < KD / 64) rows_load<NPV>(pf, dq_p + rowk + k0 + 64, hk, BTH * KD);
+      rows_store<LS, 1>(ST, pf, nullptr);
+      if (kb + 1 < KD / 64) rows_load<1>(pf, dq_p + rowk + k0 + 64, hk, 0);
     } else {
-      stage_rows<64, LS, NPV>(ST, dk_p + rowk + k0, hk, BTH * KD, nullptr);
+      stage_rows<64, LS, 1>(ST, dk_p + rowk + k0, hk, 0, nullptr);
     }
     __syncthreads();
 #pragma unroll
@@ -1131,8 +841,7 @@ __global__ __launch_bounds__(256, 1) void gdn_bwd_chunk_kernel(
       }
     }
     float rbv[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int vb = 0; vb < VD / 64; ++vb) {
+    for (int vb = 0; vb < VN / 64; ++vb) {
       const int v0 = 64 * vb;
       stage_rows<64, LS, 1>(ST, du + rowv + v0, hv, 0, nullptr);
       g2s_tile<64>(dO + rowv + v0, hv, SD, LDB);
@@ -1169,11 +878,9 @@ __global__ __launch_bounds__(256, 1) void gdn_bwd_chunk_kernel(
     const int t = lane;
     float x = s.dgr[t] + s.dgcol[0][t] + s.dgcol[1][t] + s.dgcol[2][t] + s.dgcol[3][t];
     if (t == kGC - 1) {
-      float lc = 0.f, de = 0.f;
+      float lc = 0.f;
       for (int u = 0; u < kGC; ++u) lc += s.lastc[u];
-#pragma unroll
-      for (int p = 0; p < NPV; ++p) de += del_p[(size_t)p * B * H * NT + (size_t)row * NT + ic];
-      x += lc + s.e[kGC - 1] * de;
+      x += lc + s.e[kGC - 1] * del_p[(size_t)row * NT + ic];
     }
 #pragma unroll
     for (int d = 1; d < 64; d <<= 1) {
@@ -1183,35 +890,24 @@ __global__ __launch_bounds__(256, 1) void gdn_bwd_chunk_kernel(
     dg[(tok0 + t) * H + h] = x;
     db[(tok0 + t) * H + h] = from_f32<TB>(s.dbr[t]);
   }
-  // four elements per thread and round: the partial loads of every slice and
-  // element of a round issue together (inter-chunk columns; clamped to column
-  // 7 elsewhere and to the last element past the end, and not used there;
-  // with no inter-chunk level (T = 64) the partial buffer is empty and nothing
-  // is loaded)
+  // four elements per thread and round, their loads issued together (inter-chunk
+  // columns; clamped to column 7 elsewhere and to the last element past the end, and
+  // not used there; with no inter-chunk level (T = 64) nothing is loaded)
   for (int u0 = 0; u0 < kGC * L; u0 += 4 * 256) {
-    float pl[4][NPV];
+    float pl[4];
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       const int u = min(u0 + tid + 256 * q, kGC * L - 1);
       const int t = u / L, c = u % L;
       const int ce = min(max(c, 7), 6 + nlev) - 7;
-#pragma unroll
-      for (int p = 0; p < NPV; ++p)
-        pl[q][p] = nlev > 0 ? dl_p[((size_t)p * BTH + (tok0 + t) * H + h) * nlev + ce] : 0.f;
+      pl[q] = nlev > 0 ? dl_p[((tok0 + t) * H + h) * nlev + ce] : 0.f;
     }
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       const int u = u0 + tid + 256 * q;
       if (u < kGC * L) {
         const int t = u / L, c = u % L;
-        float x = 0.f;
-        if (c < 7) {
-          x = s.dlam[c][t];
-        } else if (c < 7 + nlev) {
-#pragma unroll
-          for (int p = 0; p < NPV; ++p) x += pl[q][p];
-        }
-        dl[((tok0 + t) * H + h) * L + c] = x;
+        dl[((tok0 + t) * H + h) * L + c] = c < 7 ? s.dlam[c][t] : c < 7 + nlev ? pl[q] : 0.f;
       }
     }
   }
@@ -1220,13 +916,6 @@ __global__ __launch_bounds__(256, 1) void gdn_bwd_chunk_kernel(
 // ---------------------------------------------------------------------------
 // host launcher
 // ---------------------------------------------------------------------------
-struct GdnBwdWs {
-  __bf16 *qn, *kn, *knT, *wn, *un, *hs;
-  __bf16 *dq_p, *dw_p, *dk_p;   // per-V-slice partials, bf16 (summed in fp32 by the chunk kernel)
-  float *du, *dl_p, *del_p;
-  size_t bytes;
-};
-
 inline size_t balign(size_t x) { return (x + 255) & ~(size_t)255; }
 
 // recompute = false: no recompute regions (the caller brings q_new, K_new,
@@ -1237,7 +926,7 @@ inline GdnBwdWs gdn_bwd_ws_layout(void* base, int B, int T, int H, int K, int V,
   char* p = (char*)base;
   size_t off = 0;
   const size_t n = (size_t)B * T * H;
-  const size_t NT = (size_t)T / kGC, nvs = (size_t)V / kBVs;
+  const size_t NT = (size_t)T / kGC;
   const size_t nl = nlev > 0 ? (size_t)nlev : 1;
   w.qn = w.kn = w.knT = w.wn = w.un = w.hs = nullptr;
   if (recompute) {
@@ -1246,14 +935,15 @@ inline GdnBwdWs gdn_bwd_ws_layout(void* base, int B, int T, int H, int K, int V,
     w.knT = (__bf16*)(p + off); off += balign(n * K * 2);
     w.wn = (__bf16*)(p + off); off += balign(n * K * 2);
     w.un = (__bf16*)(p + off); off += balign(n * V * 2);
-    w.hs = (__bf16*)(p + off); off += balign((size_t)B * H * NT * nl * V * K * 2);
+    w.hs = (__bf16*)(p + off); off += balign((size_t)B * H * gdn_set_before((int)NT) * V * K * 2);
   }
-  w.dq_p = (__bf16*)(p + off); off += balign(nvs * n * K * 2);
-  w.dw_p = (__bf16*)(p + off); off += balign(nvs * n * K * 2);
-  w.dk_p = (__bf16*)(p + off); off += balign(nvs * n * K * 2);
+  w.dhs = (__bf16*)(p + off); off += balign((size_t)B * H * NT * nl * V * K * 2);
+  w.dq_p = (__bf16*)(p + off); off += balign(n * K * 2);
+  w.dw_p = (__bf16*)(p + off); off += balign(n * K * 2);
+  w.dk_p = (__bf16*)(p + off); off += balign(n * K * 2);
   w.du = (float*)(p + off); off += balign(n * V * 4);
-  w.dl_p = (float*)(p + off); off += balign(nvs * n * nl * 4);
-  w.del_p = (float*)(p + off); off += balign(nvs * B * H * NT * 4);
+  w.dl_p = (float*)(p + off); off += balign(n * nl * 4);
+  w.del_p = (float*)(p + off); off += balign((size_t)B * H * NT * 4);
   w.bytes = off;
   return w;
 }
@@ -1262,22 +952,10 @@ template <int KD, int VD, typename TB, typename TL, bool STRONG, typename E = __
 static hipError_t gdn_bwd_t(const void* q, const void* k, const void* v, const void* beta,
                             const float* gcum, const void* l, const void* dO, void* dq, void* dk,
                             void* dv, void* db, float* dg, float* dl, const GdnBwdWs& w, int B,
-                            int T, int H, int L, int nlev, int norm_qk, float scale,
+                            int T, int H, int V, int L, int nlev, int norm_qk, float scale,
                             hipStream_t stream) {
   const int NT = T / kGC;
   hipError_t e;
-  {
-    auto ks = gdn_bwd_scan_kernel<KD, TL, E>;
-    const int smem = (int)sizeof(GdnBscanSmem<KD>);
-    if ((e = hipFuncSetAttribute((const void*)ks, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                 smem)) != hipSuccess)
-      return e;
-    hipLaunchKernelGGL(ks, dim3(B * H * (VD / kBVs)), dim3(64 * gdn_bscan_waves<KD>()), smem,
-                       stream, w.qn, w.wn, w.kn,
-                       w.un, (const __bf16*)dO, gcum, (const TL*)l, w.hs, w.dq_p, w.dw_p, w.dk_p,
-                       w.du, w.dl_p, w.del_p, B, T, H, VD, L, nlev, STRONG ? 1 : 0);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
-  }
   {
     auto kc = gdn_bwd_chunk_kernel<KD, VD, TB, TL, STRONG, E>;
     const int smem = (int)sizeof(GdnBchunkSmem<KD, VD>);
@@ -1288,7 +966,7 @@ static hipError_t gdn_bwd_t(const void* q, const void* k, const void* v, const v
                        (const __bf16*)k, (const __bf16*)v, (const TB*)beta, gcum, (const TL*)l,
                        (const __bf16*)dO, w.dq_p, w.dw_p, w.dk_p, w.du, w.dl_p, w.del_p,
                        (__bf16*)dq, (__bf16*)dk, (__bf16*)dv, (TB*)db, dg, dl, B, T,
-                       H, L, nlev, norm_qk, scale);
+                       H, V, L, nlev, norm_qk, scale);
     if ((e = hipGetLastError()) != hipSuccess) return e;
   }
   return hipSuccess;
@@ -1311,20 +989,25 @@ hipError_t gdn_bwd_dispatch(const void* q, const void* k, const void* v, const v
                             int norm_qk, float scale, int strong, int h16, hipStream_t stream,
                             int* unsupported) {
   using namespace hattn;
+  {
+    hipError_t e = hattn_gdn_bwd_levels_launch(w, dO, gcum, l, B, T, H, K, V, L, nlev, dt_l, strong, h16,
+                                               stream, unsupported);
+    if (e != hipSuccess || *unsupported) return e;
+  }
 #define HATTN_GDN_BT(KD_, VD_, TB_, TL_)                                                        \
   return strong ? gdn_bwd_t<KD_, VD_, TB_, TL_, true>(q, k, v, beta, gcum, l, dO, dq, dk, dv, db,  \
-                                                      dg, dl, w, B, T, H, L, nlev, norm_qk, scale, \
+                                                      dg, dl, w, B, T, H, V, L, nlev, norm_qk, scale, \
                                                       stream)                                      \
                 : gdn_bwd_t<KD_, VD_, TB_, TL_, false>(q, k, v, beta, gcum, l, dO, dq, dk, dv, db, \
-                                                       dg, dl, w, B, T, H, L, nlev, norm_qk,       \
+                                                       dg, dl, w, B, T, H, V, L, nlev, norm_qk,       \
                                                        scale, stream);
 // fp16 q/k/v: the weak hierarchy with fp32 beta / lambda only.
 #define HATTN_GDN_B(KD_, VD_)                                                                   \
-  if (K == KD_ && V == VD_) {                                                                   \
+  if (K == KD_ && (VD_ == 0 || V == VD_)) {                                                                   \
     if (h16) {                                                                                  \
       if (!strong && dt_b == 2 && dt_l == 2)                                                    \
         return gdn_bwd_t<KD_, VD_, float, float, false, _Float16>(                              \
-            q, k, v, beta, gcum, l, dO, dq, dk, dv, db, dg, dl, w, B, T, H, L, nlev, norm_qk,   \
+            q, k, v, beta, gcum, l, dO, dq, dk, dv, db, dg, dl, w, B, T, H, V, L, nlev, norm_qk,   \
             scale, stream);                                                                     \
       *unsupported = 1;                                                                         \
       return hipSuccess;                                                                        \
@@ -1335,13 +1018,13 @@ hipError_t gdn_bwd_dispatch(const void* q, const void* k, const void* v, const v
     if (dt_b == 2 && dt_l == 0) HATTN_GDN_BT(KD_, VD_, float, __bf16)                           \
   }
   HATTN_GDN_B(256, 128)
-  HATTN_GDN_B(256, 64)
+  HATTN_GDN_B(256, 0)
   HATTN_GDN_B(192, 128)
-  HATTN_GDN_B(192, 64)
+  HATTN_GDN_B(192, 0)
   HATTN_GDN_B(128, 128)
-  HATTN_GDN_B(128, 64)
+  HATTN_GDN_B(128, 0)
   HATTN_GDN_B(64, 128)
-  HATTN_GDN_B(64, 64)
+  HATTN_GDN_B(64, 0)
 #undef HATTN_GDN_B
 #undef HATTN_GDN_BT
   *unsupported = 1;

@@ -8,8 +8,25 @@ constexpr int kGC = 64;       // chunk length
 constexpr int kLd64 = 72;     // LDS row stride of 64-wide bf16 tiles
 constexpr int kGMaxLev = 8;   // inter-chunk levels of the forward scan (T <= 64 * 2^8)
 constexpr int kGBwdMaxLev = 8;   // inter-chunk levels of the backward scan (T <= 64 * 2^8)
-constexpr int kBVs = 32;      // V columns per backward-scan workgroup
 constexpr int kLM = 65;       // row stride of 64 x 64 fp32 LDS matrices
+
+constexpr int kGdnScanGroups = 256;   // scan workgroups (row, V slice) below which the chip idles
+
+// V columns per state-scan workgroup (K >= 192: 16, so that a level's whole state
+// and the operands fit the registers of two waves per SIMD).
+constexpr int gdn_scan_bv(int K) { return K >= 192 ? 16 : 32; }
+
+// The level states kept for the backward: of every chunk, those of the levels it
+// reads (bit e of the chunk index set), in increasing level.  gdn_set_before(n):
+// the states of the chunks before n.
+__host__ __device__ inline size_t gdn_set_before(int n) {
+  size_t x = 0;
+  for (int e = 0; e < kGMaxLev; ++e) {
+    const int half = 1 << e, full = n >> (e + 1), rest = n & (2 * half - 1);
+    x += (size_t)full * half + (rest > half ? rest - half : 0);
+  }
+  return x;
+}
 
 // HType.STRONG intra-chunk levels: the reference's chunkwise GDN path takes
 // lambda of a pair inside a chunk at its strong level (make_levels_matrix with
@@ -291,6 +308,17 @@ __device__ __forceinline__ void l2norm_rinv_global(const __bf16* X, size_t ld, f
   ss += __shfl_xor(ss, 1, 64);
   ss += __shfl_xor(ss, 2, 64);
   if (part == 0) rinv[r] = __builtin_amdgcn_rsqf(ss + 1e-6f);
+}
+
+// A-operand fragment whose contraction index runs in the row order of two
+// stacked D tiles: lane (lq, ln) receives row r's elements c .. c + 3 and
+// c + 16 .. c + 19 (c = 32 step + 4 lq).  Paired with a B fragment built from
+// two D-layout accumulator quads (cat8), so states and V_new feed the next
+// product straight from registers.
+__device__ __forceinline__ bf16x8 frag_k2(const __bf16* X, int ld, int r, int c) {
+  const bf16x4 lo = *(const bf16x4*)(X + r * ld + c);
+  const bf16x4 hi = *(const bf16x4*)(X + r * ld + c + 16);
+  return bf16x8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
 }
 
 }  // namespace hattn

@@ -406,17 +406,6 @@ struct GdnScanSmem {
   float part[kGMaxLev + 1][kGC * C::LP]; // lambda_e o (q_new h_e) per level, o_intra last; [t][v]
 };
 
-// A-operand fragment whose contraction index runs in the row order of two
-// stacked D tiles: lane (lq, ln) receives row r's elements c .. c + 3 and
-// c + 16 .. c + 19 (c = 32 step + 4 lq).  Paired with a B fragment built from
-// two D-layout accumulator quads (cat8), so states and V_new feed the next
-// product straight from registers.
-__device__ __forceinline__ bf16x8 frag_k2(const __bf16* X, int ld, int r, int c) {
-  const bf16x4 lo = *(const bf16x4*)(X + r * ld + c);
-  const bf16x4 hi = *(const bf16x4*)(X + r * ld + c + 16);
-  return bf16x8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-}
-
 // One wave per inter-chunk level: wave e holds level e's whole [K x BV] state
 // in fp32 registers (tile (kt, nt) holds rows 16 kt + 4 lq + i, columns
 // 16 nt + ln) and runs its recurrence on its own,
@@ -429,10 +418,10 @@ __device__ __forceinline__ bf16x8 frag_k2(const __bf16* X, int ld, int r, int c)
 // barrier publishes the chunk's operands (staged in LDS from registers loaded
 // during the previous chunk), the second the level reads, which every thread
 // then sums for four outputs and stores.
-// SMODE kScanOut: the forward (o).  kScanSave (the backward's recompute): every
-// level's state at every chunk start is written to hsave, bf16
-// [row][chunk][level][v][k]; no output (o, q_new, P and the V slice are not
-// read).  kScanOutSave: both, for a forward whose backward takes the states
+// SMODE kScanOut: the forward (o).  kScanSave (the backward's recompute): the
+// states of the levels that a chunk reads, at the chunk's start, are written to
+// hsave, bf16 (the others are sums of them); no output (o, q_new, P and the V slice
+// are not read).  kScanOutSave: both, for a forward whose backward takes the states
 // from it.  Separate instantiations, so the plain forward carries no
 // registers for the states' stores.
 enum { kScanOut = 0, kScanSave = 1, kScanOutSave = 2 };
@@ -554,11 +543,8 @@ __global__ __launch_bounds__(512) void gdn_scan_kernel(
   const rsrc_t ro = make_rsrc(o_ok ? (const void*)(o + rowtok * V + v0) : (const void*)gcum,
                               o_ok ? (size_t)T * H * V * sizeof(TO) : 0);
   const unsigned o_voff = ((o_ok ? ot : 0) * HV + ov) * sizeof(TO);
-  // hsave: this level's planes (an empty range for the waves without a level)
-  const rsrc_t rh = make_rsrc(kSave ? (const void*)(hsave + (size_t)row * NT * nlev * V * KD +
-                                                    (size_t)(act ? e : 0) * V * KD + (size_t)v0 * KD)
-                                    : (const void*)gcum,
-                              kSave && act ? (size_t)NT * nlev * V * KD * 2 : 0);
+  // hsave: [row][states of the set levels, chunk by chunk][v][k]
+  __bf16* hrow = kSave ? hsave + ((size_t)row * gdn_set_before(NT) * V + v0) * KD : nullptr;
 
   stage_load(0);
   stage_store();
@@ -579,14 +565,17 @@ __global__ __launch_bounds__(512) void gdn_scan_kernel(
     const bool needy = act && !first && !reset;
 
     if constexpr (kSave) {
-      // level e's state at the chunk start -> hsave[row][ic][e][v][k]
+      // the state of a level that this chunk reads, at the chunk start
+      if (act && bit) {
+        const size_t slot = gdn_set_before(ic) + __builtin_popcount(ic & ((1 << e) - 1));
+        const rsrc_t rh = make_rsrc(hrow + slot * V * KD, (size_t)BV * KD * 2);
 #pragma unroll
-      for (int kt = 0; kt < NKT; ++kt)
+        for (int kt = 0; kt < NKT; ++kt)
 #pragma unroll
-        for (int nt = 0; nt < NVT; ++nt)
-          buf_store8(__builtin_bit_cast(uint2, cvt4e<E>(st[kt][nt])), rh,
-                     (unsigned)(((16 * nt + ln) * KD + 16 * kt + 4 * lq) * 2),
-                     (unsigned)((size_t)ic * nlev * V * KD * 2));
+          for (int nt = 0; nt < NVT; ++nt)
+            buf_store8(__builtin_bit_cast(uint2, cvt4e<E>(st[kt][nt])), rh,
+                       (unsigned)(((16 * nt + ln) * KD + 16 * kt + 4 * lq) * 2), 0);
+      }
     }
     if constexpr (kOut) {
       if (rd) {
@@ -768,16 +757,13 @@ inline GdnKeepWs gdn_keep_ws_layout(void* base, int B, int T, int H, int K, int 
   w.f = gdn_ws_layout(base, B, T, H, K, V);
   char* p = (char*)base;
   size_t off = w.f.bytes;
-  const size_t n = (size_t)B * T * H, NT = (size_t)T / kGC, nl = nlev > 0 ? (size_t)nlev : 1;
+  const size_t n = (size_t)B * T * H, NT = (size_t)T / kGC;
+  (void)nlev;
   w.kn = (__bf16*)(p + off); off += galign(n * K * 2);
-  w.hs = (__bf16*)(p + off); off += galign((size_t)B * H * NT * nl * V * K * 2);
+  w.hs = (__bf16*)(p + off); off += galign((size_t)B * H * gdn_set_before((int)NT) * V * K * 2);
   w.bytes = off;
   return w;
 }
-
-// V columns per scan workgroup (K >= 192: 16, so that the states of four levels of a
-// k-quarter and the A operands fit the registers of two waves per SIMD).
-template <int KD> struct ScanBV { static constexpr int value = KD >= 192 ? 16 : 32; };
 
 inline int device_cus() {
   static int cus[64] = {0};
@@ -819,7 +805,7 @@ static hipError_t gdn_scan_launch_t(const GdnWs& w, const void* v, const float* 
                                     const void* l, void* o, float* ht, __bf16* hsave, int B,
                                     int T, int H, int V, int L, int nlev, int final_state,
                                     int strong, hipStream_t stream) {
-  constexpr int BV = ScanBV<KD>::value;
+  constexpr int BV = gdn_scan_bv(KD);
   // hsave without o: the recompute; both: a forward that keeps the states
   auto ks = !hsave ? gdn_scan_kernel<KD, BV, TL, TO, kScanOut, E>
             : o ? gdn_scan_kernel<KD, BV, TL, TO, kScanOutSave, E>

@@ -528,7 +528,7 @@ static int gdn_fwd_impl(const void* q, const void* k, const void* v, const void*
                         void* Au, float* ht, int B, int T, int H, int K, int V, int L,
                         int dtype_qkv, int dtype_beta, int dtype_l, int dtype_o, int level_base,
                         int htype, int chunk_size, int l2norm_qk, float qk_scale,
-                        void* workspace, size_t workspace_bytes, bool keep, void* stream) {
+                        void* workspace, size_t workspace_bytes, bool keep, void* stream, bool any_v = false) {
   if (chunk_size != 64)
     return fail(HATTN_ERR_NOT_IMPLEMENTED, "chunk_size=%d (only 64 is supported)", chunk_size);
   if (level_base != 2)
@@ -557,7 +557,7 @@ static int gdn_fwd_impl(const void* q, const void* k, const void* v, const void*
   // fp16 q/k/v (fp16 MFMA): HType.WEAK with fp32 beta / lambda and an fp16 o
   if (dtype_qkv != HATTN_BF16 && dtype_qkv != HATTN_FP16)
     return fail(HATTN_ERR_NOT_IMPLEMENTED, "q/k/v dtype code %d (bf16 or fp16 required)", dtype_qkv);
-  if (keep && !(V == 64 || V == 128))
+  if (keep && !any_v && !(V == 64 || V == 128))
     return fail(HATTN_ERR_NOT_IMPLEMENTED,
                 "V=%d: the kept buffers serve a backward in one V block (V in {64, 128})", V);
   if (keep && nlev > hattn_gdn_bwd_max_levels())
@@ -598,6 +598,18 @@ int hattn_gdn_chunkwise_fwd(const void* q, const void* k, const void* v, const v
                       qk_scale, workspace, workspace_bytes, false, stream);
 }
 
+int hattn_gdn_chunkwise_fwd_keep_any_v(const void* q, const void* k, const void* v,
+                                       const void* beta, const float* g, const void* l, void* o,
+                                       float* g_cumsum, void* Aw, void* Au, float* ht, int B,
+                                       int T, int H, int K, int V, int L, int dtype_qkv,
+                                       int dtype_beta, int dtype_l, int dtype_o, int level_base,
+                                       int htype, int chunk_size, int l2norm_qk, float qk_scale,
+                                       void* workspace, size_t workspace_bytes, void* stream) {
+  return gdn_fwd_impl(q, k, v, beta, g, l, o, g_cumsum, Aw, Au, ht, B, T, H, K, V, L, dtype_qkv,
+                      dtype_beta, dtype_l, dtype_o, level_base, htype, chunk_size, l2norm_qk,
+                      qk_scale, workspace, workspace_bytes, true, stream, true);
+}
+
 size_t hattn_gdn_chunkwise_fwd_keep_workspace(int B, int T, int H, int K, int V, int L) {
   (void)L;
   if (B <= 0 || T < 64 || T % 64 != 0 || H <= 0 || K <= 0 || V <= 0) return 0;
@@ -630,7 +642,8 @@ static int gdn_bwd_impl(const void* q, const void* k, const void* v, const void*
                         int V, int L, int dtype_qkv, int dtype_beta, int dtype_l, int dtype_do,
                         int level_base, int htype, int chunk_size, int l2norm_qk,
                         float qk_scale, void* workspace, size_t workspace_bytes,
-                        const void* fwd_ws, size_t fwd_ws_bytes, bool kept, void* stream) {
+                        const void* fwd_ws, size_t fwd_ws_bytes, bool kept, void* stream,
+                        bool any_v = false) {
   // chunkwise_hgdn.py:818-858; HType.STRONG: the gradient of the strong forward
   // (level reads at every chunk for levels >= 1)
   if (chunk_size != 64)
@@ -645,10 +658,10 @@ static int gdn_bwd_impl(const void* q, const void* k, const void* v, const void*
   if (K > 256) return fail(HATTN_ERR_NOT_IMPLEMENTED, "K=%d > 256", K);
   if (K % 64 != 0 || V % 64 != 0)
     return fail(HATTN_ERR_VALUE, "K=%d, V=%d and BK, BV could be 64", K, V);
-  if (!((K == 64 || K == 128 || K == 192 || K == 256) && (V == 64 || V == 128)))
+  if (!((K == 64 || K == 128 || K == 192 || K == 256) && (any_v || V == 64 || V == 128)))
     return fail(HATTN_ERR_NOT_IMPLEMENTED,
                 "K=%d V=%d (the MI355X GDN backward supports K in {64, 128, 192, 256} and V in "
-                "{64, 128}; the host driver splits larger V into blocks)", K, V);
+                "{64, 128}; hattn_gdn_chunkwise_bwd_any_v takes any multiple of 64)", K, V);
   const int nlev = ceil_log2(T / 64);
   if (7 + nlev > L)
     return fail(HATTN_ERR_VALUE, "L=%d levels < 7 + ceil(log2(T/64))=%d", L, 7 + nlev);
@@ -732,6 +745,20 @@ int hattn_gdn_chunkwise_bwd_fwd_ws(const void* q, const void* k, const void* v, 
                       dtype_qkv, dtype_beta, dtype_l, dtype_do, level_base, htype, chunk_size,
                       l2norm_qk, qk_scale, workspace, workspace_bytes, fwd_workspace,
                       fwd_workspace_bytes, true, stream);
+}
+
+int hattn_gdn_chunkwise_bwd_any_v(const void* q, const void* k, const void* v, const void* beta,
+                                  const float* g_cumsum, const void* l, const void* do_, void* dq,
+                                  void* dk, void* dv, void* db, float* dg, float* dl, int B, int T,
+                                  int H, int K, int V, int L, int dtype_qkv, int dtype_beta,
+                                  int dtype_l, int dtype_do, int level_base, int htype,
+                                  int chunk_size, int l2norm_qk, float qk_scale, void* workspace,
+                                  size_t workspace_bytes, const void* fwd_workspace,
+                                  size_t fwd_workspace_bytes, void* stream) {
+  return gdn_bwd_impl(q, k, v, beta, g_cumsum, l, do_, dq, dk, dv, db, dg, dl, B, T, H, K, V, L,
+                      dtype_qkv, dtype_beta, dtype_l, dtype_do, level_base, htype, chunk_size,
+                      l2norm_qk, qk_scale, workspace, workspace_bytes, fwd_workspace,
+                      fwd_workspace_bytes, fwd_workspace != nullptr, stream, true);
 }
 
 namespace {

@@ -52,6 +52,12 @@ SIGNATURES = [
      [_P, _P, _P, _P, _F, _P, _P, _P, _P, _P, _P, _P, _P, _F, _F] + [_I] * 6 + [_I] * 4
      + [_I] * 3 + [_I, ctypes.c_float] + [_P, _S, _P, _S, _P]),
     ("hattn_gdn_chunkwise_bwd_fwd_ws_workspace", _S, [_I] * 6),
+    ("hattn_gdn_chunkwise_fwd_keep_any_v", _I,
+     [_P, _P, _P, _P, _F, _P, _P, _F, _P, _P, _F] + [_I] * 6 + [_I] * 4 + [_I] * 3
+     + [_I, ctypes.c_float] + [_P, _S, _P]),
+    ("hattn_gdn_chunkwise_bwd_any_v", _I,
+     [_P, _P, _P, _P, _F, _P, _P, _P, _P, _P, _P, _F, _F] + [_I] * 6 + [_I] * 4
+     + [_I] * 3 + [_I, ctypes.c_float] + [_P, _S, _P, _S, _P]),
     ("hattn_hstate_step", _I,
      [_P] * 9 + [_I] * 12 + [ctypes.c_float] + [_I] * 4 + [_P]),
     ("hattn_hstate_plan", _I, [_P, _I, _I, _I, _P]),

@@ -32,7 +32,7 @@ from hattention import _lib
 from hattention.base import HType, get_num_levels, ceil_log
 
 CHUNK = 64
-VB = 128   # V columns per backward launch
+VB = 128   # V columns that chunkwise_fwd_keep keeps a workspace for by itself
 
 
 def _validate(q, k, v, l, head_first, level_base, htype, chunk_size, **tensors):
@@ -131,12 +131,13 @@ def chunkwise_fwd_keep(
     *,
     qk_l2norm_scale: Optional[float] = None,
     keep: bool = True,
+    keep_any_v: bool = False,
 ):
     """:func:`chunkwise_fwd` that also returns the forward's workspace, holding
     what the backward would recompute (q_new, W_new, K_new, U and every level's
-    state at every chunk start, bit for bit), when the backward can take it
-    (V in {64, 128}; else None): pass it to :func:`chunkwise_bwd` as ``fwd_ws``
-    with the same inputs, and the backward skips its recompute
+    state that a chunk reads, bit for bit), for V in {64, 128} or, with
+    ``keep_any_v``, any V (else None): pass it to :func:`chunkwise_bwd` as
+    ``fwd_ws`` with the same inputs, and the backward skips its recompute
     (HAttentionFunction keeps it between its forward and backward).  Returns
     (g_cumsum, o, Aw, Au, ht, fwd_ws)."""
     B, T, G, H, K, V, L = _validate(q, k, v, l, head_first, level_base, htype, chunk_size,
@@ -155,11 +156,11 @@ def chunkwise_fwd_keep(
     Au = torch.empty(B, T, H, CHUNK, dtype=k.dtype, device=dev)
     ht = torch.zeros(B, H, K, V, L, dtype=torch.float32, device=dev) if output_final_state else None
     lib = _lib.load()
-    keep = keep and V in (64, VB)
+    keep = keep and (keep_any_v or V in (64, VB))
     ws, ws_ptr, ws_bytes = _lib.workspace(
         (lib.hattn_gdn_chunkwise_fwd_keep_workspace if keep
          else lib.hattn_gdn_chunkwise_fwd_workspace)(B, T, H, K, V, L), dev)
-    st = (lib.hattn_gdn_chunkwise_fwd_keep if keep else lib.hattn_gdn_chunkwise_fwd)(
+    st = (lib.hattn_gdn_chunkwise_fwd_keep_any_v if keep else lib.hattn_gdn_chunkwise_fwd)(
         _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.ptr(b), _lib.ptr(g), _lib.ptr(l),
         _lib.ptr(o), _lib.ptr(g_cumsum), _lib.ptr(Aw), _lib.ptr(Au), _lib.ptr(ht),
         B, T, H, K, V, L, _lib.dtype_code(q), _lib.dtype_code(b), _lib.dtype_code(l),
@@ -216,55 +217,30 @@ def chunkwise_bwd(
     dev = _lib.require_device(q, k, v, b, g, l, do)
     dtypes = (q.dtype, k.dtype, v.dtype, b.dtype)
     q, k, v, b, l = _narrow_half(q, k, v, b, l, htype)
-    Aw, Au = Aw.to(k.dtype), Au.to(k.dtype)
     if G != H:
         q = q.repeat_interleave(H // G, dim=2).contiguous()
         k = k.repeat_interleave(H // G, dim=2).contiguous()
     do = do.to(v.dtype).contiguous()
     lib = _lib.load()
-    # The gradients are sums over independent column blocks of V (each column of
-    # o depends on its column of v only): the kernels take V in {64, 128}, so a
-    # larger V runs block by block, dq / dk / db / dg / dl summed in fp32.
-    blocks = [(v0, min(v0 + VB, V)) for v0 in range(0, V, VB)]
+    dq = torch.empty(B, T, H, K, dtype=q.dtype, device=dev)
+    dk = torch.empty(B, T, H, K, dtype=k.dtype, device=dev)
     dv = torch.empty_like(v)
-    acc = None
-    for v0, v1 in blocks:
-        vb = v if len(blocks) == 1 else v[..., v0:v1].contiguous()
-        dob = do if len(blocks) == 1 else do[..., v0:v1].contiguous()
-        Vb = v1 - v0
-        dq_b = torch.empty(B, T, H, K, dtype=q.dtype, device=dev)
-        dk_b = torch.empty(B, T, H, K, dtype=k.dtype, device=dev)
-        dv_b = dv if len(blocks) == 1 else torch.empty_like(vb)
-        db_b = torch.empty_like(b)
-        dg_b = torch.empty(B, T, H, dtype=torch.float32, device=dev)
-        dl_b = torch.empty(B, T, H, L, dtype=torch.float32, device=dev)
-        kept = fwd_ws is not None and len(blocks) == 1
-        ws, ws_ptr, ws_bytes = _lib.workspace(
-            (lib.hattn_gdn_chunkwise_bwd_fwd_ws_workspace if kept
-             else lib.hattn_gdn_chunkwise_bwd_workspace)(B, T, H, K, Vb, L), dev)
-        args = (
-            _lib.ptr(q), _lib.ptr(k), _lib.ptr(vb), _lib.ptr(b), _lib.ptr(g), _lib.ptr(l),
-            _lib.ptr(Aw), _lib.ptr(Au), _lib.ptr(dob), _lib.ptr(dq_b), _lib.ptr(dk_b),
-            _lib.ptr(dv_b), _lib.ptr(db_b), _lib.ptr(dg_b), _lib.ptr(dl_b), B, T, H, K, Vb, L,
-            _lib.dtype_code(q), _lib.dtype_code(b), _lib.dtype_code(l), _lib.dtype_code(dob),
-            level_base, htype.value, chunk_size, 1 if qk_l2norm_scale is not None else 0,
-            float(qk_l2norm_scale) if qk_l2norm_scale is not None else 1.0, ws_ptr, ws_bytes)
-        if kept:
-            st = lib.hattn_gdn_chunkwise_bwd_fwd_ws(*args, _lib.ptr(fwd_ws), fwd_ws.numel(),
-                                                    _lib.stream_handle(dev))
-        else:
-            st = lib.hattn_gdn_chunkwise_bwd(*args, _lib.stream_handle(dev))
-        _lib.check(st)
-        del ws
-        if len(blocks) == 1:
-            dq, dk, db, dg, dl = dq_b, dk_b, db_b, dg_b, dl_b
-            break
-        dv[..., v0:v1] = dv_b
-        parts = (dq_b.float(), dk_b.float(), db_b.float(), dg_b, dl_b)
-        acc = parts if acc is None else tuple(a + p for a, p in zip(acc, parts))
-    if acc is not None:
-        dq, dk = acc[0].to(q.dtype), acc[1].to(k.dtype)
-        db, dg, dl = acc[2].to(b.dtype), acc[3], acc[4]
+    db = torch.empty_like(b)
+    dg = torch.empty(B, T, H, dtype=torch.float32, device=dev)
+    dl = torch.empty(B, T, H, L, dtype=torch.float32, device=dev)
+    ws, ws_ptr, ws_bytes = _lib.workspace(
+        (lib.hattn_gdn_chunkwise_bwd_fwd_ws_workspace if fwd_ws is not None
+         else lib.hattn_gdn_chunkwise_bwd_workspace)(B, T, H, K, V, L), dev)
+    _lib.check(lib.hattn_gdn_chunkwise_bwd_any_v(
+        _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.ptr(b), _lib.ptr(g), _lib.ptr(l),
+        _lib.ptr(do), _lib.ptr(dq), _lib.ptr(dk), _lib.ptr(dv), _lib.ptr(db), _lib.ptr(dg),
+        _lib.ptr(dl), B, T, H, K, V, L, _lib.dtype_code(q), _lib.dtype_code(b),
+        _lib.dtype_code(l), _lib.dtype_code(do), level_base, htype.value, chunk_size,
+        1 if qk_l2norm_scale is not None else 0,
+        float(qk_l2norm_scale) if qk_l2norm_scale is not None else 1.0, ws_ptr, ws_bytes,
+        _lib.ptr(fwd_ws), fwd_ws.numel() if fwd_ws is not None else 0,
+        _lib.stream_handle(dev)))
+    del ws
     if G != H:
         dq = dq.view(B, T, G, H // G, K).sum(3, dtype=torch.float32).to(q.dtype)
         dk = dk.view(B, T, G, H // G, K).sum(3, dtype=torch.float32).to(k.dtype)

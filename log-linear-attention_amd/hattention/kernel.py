@@ -83,7 +83,7 @@ class HAttentionFunction(torch.autograd.Function):
             g, o, Aw, Au, _, ctx.fwd_ws = _hg.chunkwise_fwd_keep(
                 q=q, k=k, v=v, b=b, g=g, l=l, head_first=head_first, level_base=level_base,
                 htype=htype, chunk_size=chunk_sizes[0], output_final_state=False,
-                qk_l2norm_scale=scale)
+                qk_l2norm_scale=scale, keep_any_v=True)
         else:
             # MAMBA2 with chunkwise=False is the reference's parallel.py path.
             raise NotImplementedError("only the chunkwise path is implemented on MI355X")
