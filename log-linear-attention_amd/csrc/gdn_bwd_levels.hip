@@ -7,6 +7,12 @@ namespace hattn {
 // ---------------------------------------------------------------------------
 // Kernel 3: reverse state scan
 // ---------------------------------------------------------------------------
+// V columns per workgroup: 32 where the state and its operands fit the registers (four
+// waves: one per SIMD), so that an A operand serves two products; two LDS buffers where
+// they fit.
+constexpr int gdn_dh_bv(int K, int NW) { return K <= 128 || (K <= 192 && NW == 4) ? 32 : 16; }
+constexpr bool gdn_dh_two_buffers(int K, int BV) { return K <= 128 || (K <= 192 && BV == 16); }
+
 template <int KD, int BV, bool DB>
 struct GdnDhSmem {
   static constexpr int LK = KD + 8, LVS = BV + 8, NB = DB ? 2 : 1;
@@ -23,7 +29,7 @@ struct GdnDhSmem {
 // contraction index: frag_k2, tr_frag_d).  NW waves per workgroup: with few (row,
 // V slice) pairs the levels are spread over two workgroups of four, which halves
 // the LDS reads of each (they bound a chunk: a wave reads every A operand itself).
-// Two LDS buffers where they fit (K <= 192): one barrier a chunk.
+// Two LDS buffers where they fit: one barrier a chunk.
 // (The previous reverse scan kept all levels in one workgroup, three barriers a
 // level, and formed the sums of kernel 4 on the way: 2.46 ms at B 4, T 8192, H 16, K
 // = V = 128; 10.1 ms for 128 of the 384 columns of V at B 1, T 16384, H 6, K = 192,
@@ -34,7 +40,7 @@ __global__ __launch_bounds__(64 * NW) void gdn_dh_scan_kernel(
     const __bf16* __restrict__ dO, const float* __restrict__ gcum, const TL* __restrict__ l,
     __bf16* __restrict__ dhs, int nrows, int T, int H, int V, int L, int nlev, int nparts,
     int strong) {
-  constexpr bool DB = KD <= 192;
+  constexpr bool DB = gdn_dh_two_buffers(KD, BV);
   using Sm = GdnDhSmem<KD, BV, DB>;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
   Sm& s = *(Sm*)smem_raw;
@@ -123,15 +129,8 @@ __global__ __launch_bounds__(64 * NW) void gdn_dh_scan_kernel(
     const __bf16* Wt = s.kwq[buf][1];
     const __bf16* Qt = s.kwq[buf][2];
     if (live) {
-      // dh_{c+1} -> dhs[row][chunk][level][v][k]
-      const rsrc_t rh = make_rsrc(dhs + ((((size_t)row * NT + ic) * nlev + e) * V + v0) * KD,
-                                  (size_t)BV * KD * 2);
-#pragma unroll
-      for (int kt = 0; kt < NKT; ++kt)
-#pragma unroll
-        for (int nt = 0; nt < NVT; ++nt)
-          buf_store8(__builtin_bit_cast(uint2, cvt4e<E>(st[kt][nt])), rh,
-                     (unsigned)(((16 * nt + ln) * KD + 16 * kt + 4 * lq) * 2), 0);
+      // dh_{c+1} -> dhs[row][chunk][level]
+      store_state_frags<KD, BV, E>(st, dhs + (((size_t)row * NT + ic) * nlev + e) * V * KD, v0);
     }
     // the next chunk's operands, into registers while this one is computed
     stage_load(max(ic - 1, 0));
@@ -207,93 +206,46 @@ __global__ __launch_bounds__(64 * NW) void gdn_dh_scan_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// Kernel 4: the sums over the levels, per chunk
+// Kernels 4: the sums over the levels, per chunk
 // ---------------------------------------------------------------------------
-template <int KD>
-struct GdnLevelSmem {
-  static constexpr int NW = KD <= 128 ? 4 : 8;   // waves
-  static constexpr int NP = NW / 4;              // parts of K of dq_new
-  static constexpr int LK = KD + 8;
-  union {
-    __bf16 tile[2][2][32 * LK];   // [buffer][h, dh][v][k]: 32 columns of V of one level
-    __bf16 z[2][kGC * LK];        // 64 rows of Z [k of h][k of dh], 16-bit hi and lo
-  };
-  __bf16 kn[kGC * LK];            // K_new [t][k]
-  float lam[kGBwdMaxLev][kGC];    // weight of each set level's read
-  float y[NP][kGBwdMaxLev][kGC];  // rowdot(q_new, dO h_j^T), by part of K
-  float red[NW];
-};
+// 8 values of a 16-bit row in the order of the stored fragments: 4 lq, 16 + 4 lq, + 0..3
+__device__ __forceinline__ bf16x8 row_frag(const __bf16* p) {
+  const int lq = (threadIdx.x & 63) >> 4;
+  const bf16x4 lo = *(const bf16x4*)(p + 4 * lq), hi = *(const bf16x4*)(p + 16 + 4 * lq);
+  return bf16x8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+}
 
-// Four waves, or eight where four would hold more than the registers take (K > 128).
-// Wave (wr, wc) = (w >> 1, w & 1) owns column half wc of its share wr of the rows of Z,
-// and, of the [64 x K] results, token tile w & 3 and part w >> 2 of K of dq_new, token
-// tiles 8 / NW wr + x and column half wc of dK_new.  The V columns go by in blocks of
-// 32, the levels of a block from the top: a clear level's dh joins the running sum R
-// (fp32, in the order of a B operand) and gives its part of dU; a set level's h gives
-// its part of Z with R + dh, and of dq_new and dlambda.  A level's [32 x K] pieces of h
-// and dh go through two LDS buffers, loaded one step ahead.  Z, whose products with
-// W_new and K_new contract over either index, then passes through LDS 64 rows at a time
-// as a 16-bit hi and lo part, so it loses nothing to rounding.
+// dq_new = sum over the read levels e of lambda_e o X_e, X_e = dO h_e^T, and dlambda_e =
+// rowdot(q_new, X_e).  Four waves, wave w the K columns K/4 w .. of every token; the
+// chunk's dO is staged in LDS, kReadCols columns of V at a time, and each wave loads its
+// part of the states' fragments PF blocks ahead.  No barrier between levels and few
+// registers: several workgroups per CU hide the loads.
+// (With dO's fragments loaded from memory by every wave, 8 bytes from each of 16 rows an
+// instruction, the L1 lookups bound the kernel: 976 us at B 4, T 8192, H 16, K = V = 128.)
+constexpr int kReadCols = 128;
 template <int KD, typename TL, typename E>
-__global__ __launch_bounds__(64 * GdnLevelSmem<KD>::NW) void gdn_bwd_level_kernel(
-    const __bf16* __restrict__ qn, const __bf16* __restrict__ wn, const __bf16* __restrict__ kn,
-    const __bf16* __restrict__ un, const __bf16* __restrict__ dO, const TL* __restrict__ l,
-    const __bf16* __restrict__ hs, const __bf16* __restrict__ dhs, __bf16* __restrict__ dqn,
-    __bf16* __restrict__ dwn, __bf16* __restrict__ dkn, float* __restrict__ du,
-    float* __restrict__ dl_p, float* __restrict__ del_p, int T, int H, int V, int L, int nlev,
-    int strong) {
-  using Sm = GdnLevelSmem<KD>;
-  extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
-  Sm& s = *(Sm*)smem_raw;
-  constexpr int NW = Sm::NW, NTH = 64 * NW, LK = Sm::LK, NKT = KD / 16, NH = KD / 32;
-  constexpr int ZR = 2 * NKT / NW, NX = NKT / Sm::NP, TT = 8 / NW;   // row tiles of Z, K tiles of dq_new, token tiles of dK_new
-  constexpr int UPR = KD / 8, HU = (32 * UPR + NTH - 1) / NTH;       // 16-byte units per row / per thread
+__global__ __launch_bounds__(256, KD <= 64 ? 3 : 2) void gdn_bwd_read_kernel(
+    const __bf16* __restrict__ qn, const __bf16* __restrict__ dO, const TL* __restrict__ l,
+    const __bf16* __restrict__ hs, __bf16* __restrict__ dqn, float* __restrict__ dl_p, int T,
+    int H, int V, int L, int nlev, int strong) {
+  constexpr int NKT = KD / 16, NQ = NKT / 4, PF = 4, LD = kReadCols + 8;
+  __shared__ __attribute__((aligned(16))) __bf16 so[kGC * LD];   // dO [t][v] of the column group
+  __shared__ float lam[kGBwdMaxLev][kGC];      // weight of each stored level's read
+  __shared__ float ysum[4][kGBwdMaxLev][kGC];  // rowdot(q_new, dO h_j^T), by wave
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int lq = lane >> 4, ln = lane & 15, wr = w >> 1, wc = w & 1;
-  const int tw = w & 3, kp = w >> 2;
+  const int lq = lane >> 4, ln = lane & 15;
   const int NT = T / kGC;
   const int ic = blockIdx.x % NT, row = blockIdx.x / NT;
   const int b = row / H, h = row % H;
   const size_t tok0 = (size_t)b * T + (size_t)ic * kGC;
   const size_t hk = (size_t)H * KD, hv = (size_t)H * V;
   const size_t rowk = (tok0 * H + h) * KD, rowv = (tok0 * H + h) * V;
-  const bool have_dh = ic + 1 < NT;
-  const __bf16* hrow = hs + ((size_t)row * gdn_set_before(NT) + gdn_set_before(ic)) * V * KD;
-  const __bf16* drow = dhs + ((size_t)row * NT + ic) * nlev * V * KD;
-  auto is_set = [&](int e) { return (ic >> e) & 1; };
-  // dh_{c+1} of level e reaches this chunk (a level with bit e clear never ends its block)
-  auto has_dh = [&](int e) { return have_dh && (ic & ((2 << e) - 1)) != (2 << e) - 1; };
-  // the next level at or below e with something to do in this chunk, or -1
-  auto work_at = [&](int e) {
-    while (e >= 0 && !is_set(e) && !have_dh) --e;
-    return e;
-  };
+  const int nset = __builtin_popcount(ic);
+  const __bf16* hrow = hs + ((size_t)row * gdn_set_before(NT) + gdn_set_before(ic)) * V * KD +
+                       (NQ * w * 64 + lane) * 8;
+  auto is_set = [&](int e) { return ((ic >> e) & 1) != 0; };
 
-  u32x4 ph[HU], pd[HU];
-  auto fetch = [&](int vb, int e) __attribute__((always_inline)) {
-    const __bf16* ps = hrow + ((size_t)__builtin_popcount(ic & ((1 << e) - 1)) * V + 32 * vb) * KD;
-    const __bf16* pt = drow + ((size_t)e * V + 32 * vb) * KD;
-    if (is_set(e))
-#pragma unroll
-      for (int i = 0; i < HU; ++i) ph[i] = *(const u32x4*)(ps + 8 * min(tid + NTH * i, 32 * UPR - 1));
-    if (has_dh(e))
-#pragma unroll
-      for (int i = 0; i < HU; ++i) pd[i] = *(const u32x4*)(pt + 8 * min(tid + NTH * i, 32 * UPR - 1));
-  };
-  auto put = [&](int buf, int e) __attribute__((always_inline)) {
-#pragma unroll
-    for (int i = 0; i < HU; ++i) {
-      const int u = tid + NTH * i, at = (u / UPR) * LK + 8 * (u % UPR);
-      if (32 * UPR % NTH != 0 && u >= 32 * UPR) break;
-      if (is_set(e)) *(u32x4*)(s.tile[buf][0] + at) = ph[i];
-      if (has_dh(e)) *(u32x4*)(s.tile[buf][1] + at) = pd[i];
-    }
-  };
-  const int top = work_at(nlev - 1);
-  if (top >= 0) fetch(0, top);
-
-  if (tid < 256) g2s_tile<KD>(kn + rowk, hk, s.kn, LK);
-  for (int u = tid; u < nlev * kGC; u += NTH) {
+  for (int u = tid; u < nlev * kGC; u += 256) {
     const int t = u / nlev, e = u % nlev;
     // what level e's stored state (bit e set) weighs in the output of token t: its
     // lambda, and with strong also that of every clear level e' >= 1 above, whose state
@@ -303,143 +255,342 @@ __global__ __launch_bounds__(64 * GdnLevelSmem<KD>::NW) void gdn_bwd_level_kerne
     if (strong)
       for (int e2 = e + 1; e2 < nlev; ++e2)
         if (!is_set(e2)) x += to_f32<TL>(lt[e2]);
-    s.lam[e][t] = x;
+    lam[e][t] = x;
 #pragma unroll
-    for (int x2 = 0; x2 < Sm::NP; ++x2) s.y[x2][e][t] = 0.f;
+    for (int i = 0; i < 4; ++i) ysum[i][e][t] = 0.f;
   }
-  // q_new of this wave's tokens in the layout of the products' results
-  bf16x4 qd[NX];
+  bf16x4 qd[4][NQ];   // q_new in the layout of the products' results
 #pragma unroll
-  for (int kt = 0; kt < NX; ++kt)
+  for (int tt = 0; tt < 4; ++tt)
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      qd[kt][i] = qn[rowk + (size_t)(16 * tw + 4 * lq + i) * hk + 16 * (NX * kp + kt) + ln];
-  if (top >= 0) put(0, top);
-  __syncthreads();
+    for (int x = 0; x < NQ; ++x)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        qd[tt][x][j] = qn[rowk + (size_t)(16 * tt + 4 * lq + j) * hk + 16 * (NQ * w + x) + ln];
 
-  floatx4 z[ZR][NH], adq[NX], adk[TT][NH];
+  floatx4 adq[4][NQ], xa[4][NQ];
+#pragma unroll
+  for (int tt = 0; tt < 4; ++tt)
+#pragma unroll
+    for (int x = 0; x < NQ; ++x) adq[tt][x] = xa[tt][x] = zero4();
+
+  for (int c0 = 0; c0 < V && nset > 0; c0 += kReadCols) {
+    const int nvb = min(kReadCols, V - c0) / 32, nsteps = nset * nvb;
+    bf16x8 fr[PF][NQ];
+    // step = (rank of the level) nvb + block of 32 columns; past the end the last one
+    // again: a load under a condition would be waited for at the branch
+    auto fetch = [&](int i, int step) __attribute__((always_inline)) {
+      const int st = min(step, nsteps - 1);
+      const __bf16* p = hrow + ((size_t)(st / nvb) * V + c0 + 32 * (st % nvb)) * KD;
+#pragma unroll
+      for (int x = 0; x < NQ; ++x) fr[i][x] = *(const bf16x8*)(p + x * 512);
+    };
+#pragma unroll
+    for (int i = 0; i < PF; ++i) fetch(i, i);
+    if (c0 > 0) __syncthreads();   // the last group's dO is read
+    for (int u = tid; u < kGC * nvb * 4; u += 256) {
+      const int t = u / (4 * nvb), c = 8 * (u % (4 * nvb));
+      *(u32x4*)(so + t * LD + c) = *(const u32x4*)(dO + rowv + (size_t)t * hv + c0 + c);
+    }
+    __syncthreads();
+    int e = -1, left = 0;   // the current level, its blocks to come
+    for (int s0 = 0; s0 < nsteps; s0 += PF) {
+#pragma unroll
+      for (int i = 0; i < PF; ++i) {
+        if (s0 + i < nsteps) {
+          if (left == 0) {
+            do ++e;
+            while (!is_set(e));
+            left = nvb;
+          }
+          const int vb = nvb - left;
+#pragma unroll
+          for (int tt = 0; tt < 4; ++tt) {
+            const bf16x8 a = row_frag(so + (16 * tt + ln) * LD + 32 * vb);
+#pragma unroll
+            for (int x = 0; x < NQ; ++x) xa[tt][x] = mfma16<E>(a, fr[i][x], xa[tt][x]);
+          }
+          fetch(i, s0 + i + PF);
+          if (--left == 0) {
+#pragma unroll
+            for (int tt = 0; tt < 4; ++tt) {
+              const floatx4 lam4 = *(const floatx4*)(&lam[e][16 * tt + 4 * lq]);
+              float y[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+              for (int x = 0; x < NQ; ++x) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                  adq[tt][x][j] += lam4[j] * xa[tt][x][j];
+                  y[j] += xa[tt][x][j] * from16<E>(qd[tt][x][j]);
+                }
+                xa[tt][x] = zero4();
+              }
+#pragma unroll
+              for (int j = 0; j < 4; ++j) {
+                const float ys = row_sum16(y[j]);
+                if (ln == 0) ysum[w][e][16 * tt + 4 * lq + j] += ys;
+              }
+            }
+          }
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int tt = 0; tt < 4; ++tt)
+#pragma unroll
+    for (int x = 0; x < NQ; ++x)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        dqn[rowk + (size_t)(16 * tt + 4 * lq + j) * hk + 16 * (NQ * w + x) + ln] = (__bf16)adq[tt][x][j];
+  __syncthreads();
+  for (int u = tid; u < nlev * kGC; u += 256) {
+    const int t = u / nlev, ee = u % nlev;
+    auto read = [&](int j) { return ysum[0][j][t] + ysum[1][j][t] + ysum[2][j][t] + ysum[3][j][t]; };
+    float x = 0.f;
+    if (strong ? ee >= 1 : is_set(ee)) {
+      if (is_set(ee)) {
+        x = read(ee);
+      } else {
+        for (int j = 0; j < ee; ++j)
+          if (is_set(j)) x += read(j);
+      }
+    }
+    dl_p[((tok0 + t) * H + h) * nlev + ee] = x;
+  }
+}
+
+template <int KD>
+struct GdnLevelSmem {
+  static constexpr int LK = KD + 8;
+  static constexpr int NWC = KD <= 128 ? 2 : 4, NW = 2 * NWC;   // column parts of Z, waves
+  union {
+    __bf16 z[2][kGC * LK];     // 64 rows of Z [k of h][k of dh], 16-bit hi and lo
+    float du[NW][4][4][64];    // each wave's share of dU: [token, column tile][row][lane]
+  };
+  float red[NW];
+};
+
+// dU, Z, dW_new, dK_new and trace Z.  Four waves (eight for K > 128, where four would
+// hold more than the registers take); wave (wr, wc) owns row half wr and column half
+// (quarter) wc of Z, and token tiles 2 wr, 2 wr + 1 and column part wc of dK_new.  The V columns go by in blocks of 32, the levels of a block from
+// the top: a clear level's dh joins the running sum R (fp32, in the order of a B
+// operand), a set level gives its part of Z with R + dh.  Every wave loads the fragments
+// of h and dh that it needs, PF levels ahead: no LDS and no barrier between levels.  A
+// block's sum of all clear levels' dh then gives its dU (turned around by a selector
+// product, as 16-bit hi and lo, like every fp32 operand here) and its part of dK_new.  Z,
+// whose products with W_new and K_new contract over either index, passes through LDS 64
+// rows at a time.
+// (One kernel with the reads as well took 2.6 ms at B 4, T 8192, H 16, K = V = 128: 250
+// registers with spills, one workgroup per CU, two thirds of its cycles waiting.)
+template <int KD, typename E>
+__global__ __launch_bounds__(64 * GdnLevelSmem<KD>::NW, KD <= 128 ? 2 : 1) void gdn_bwd_level_kernel(
+    const __bf16* __restrict__ wn, const __bf16* __restrict__ kn, const __bf16* __restrict__ un,
+    const __bf16* __restrict__ hs, const __bf16* __restrict__ dhs, __bf16* __restrict__ dwn,
+    __bf16* __restrict__ dkn, float* __restrict__ du, float* __restrict__ del_p, int T, int H,
+    int V, int nlev) {
+  using Sm = GdnLevelSmem<KD>;
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
+  Sm& s = *(Sm*)smem_raw;
+  constexpr int NW = Sm::NW, NWC = Sm::NWC, NTH = 64 * NW, LK = Sm::LK;
+  constexpr int NKT = KD / 16, NC = NKT / NWC, ZR = NKT / 2, NP = (NC + 1) / 2;
+  constexpr int PF = KD <= 64 ? 2 : 1;   // levels loaded ahead (registers)
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lq = lane >> 4, ln = lane & 15, wr = w / NWC, wc = w % NWC;
+  const int NT = T / kGC;
+  const int ic = blockIdx.x % NT, row = blockIdx.x / NT;
+  const int b = row / H, h = row % H;
+  const size_t tok0 = (size_t)b * T + (size_t)ic * kGC;
+  const size_t hk = (size_t)H * KD, hv = (size_t)H * V;
+  const size_t rowk = (tok0 * H + h) * KD, rowv = (tok0 * H + h) * V;
+  if (ic + 1 == NT) {
+    // no later chunk: every dh is zero
+    for (int u = tid; u < kGC * KD; u += NTH) {
+      const size_t at = rowk + (size_t)(u / KD) * hk + u % KD;
+      dwn[at] = dkn[at] = (__bf16)0.f;
+    }
+    for (int u = tid; u < kGC * V; u += NTH) du[rowv + (size_t)(u / V) * hv + u % V] = 0.f;
+    if (tid == 0) del_p[(size_t)row * NT + ic] = 0.f;
+    return;
+  }
+  const int nvb = V / 32;
+  const __bf16* hrow = hs + ((size_t)row * gdn_set_before(NT) + gdn_set_before(ic)) * V * KD +
+                       (ZR * wr * 64 + lane) * 8;
+  const __bf16* drow = dhs + ((size_t)row * NT + ic) * nlev * V * KD + (NC * wc * 64 + lane) * 8;
+  auto is_set = [&](int e) { return ((ic >> e) & 1) != 0; };
+  // dh_{c+1} of level e reaches this chunk (a level with bit e clear never ends its block)
+  auto has_dh = [&](int e) { return (ic & ((2 << e) - 1)) != (2 << e) - 1; };
+  struct Step {
+    int vb, e;
+  };
+  auto after = [&](Step x) {
+    if (--x.e < 0) {
+      x.e = nlev - 1;
+      ++x.vb;
+    }
+    return x;
+  };
+  struct Frags {
+    bf16x8 hf[ZR], df[NC];
+  };
+  auto fetch = [&](Frags& f, Step x) __attribute__((always_inline)) {
+    if (x.vb >= nvb) return;
+    const __bf16* ph = hrow + ((size_t)__builtin_popcount(ic & ((1 << x.e) - 1)) * V + 32 * x.vb) * KD;
+    const __bf16* pd = drow + ((size_t)x.e * V + 32 * x.vb) * KD;
+    if (is_set(x.e))
+#pragma unroll
+      for (int i = 0; i < ZR; ++i) f.hf[i] = *(const bf16x8*)(ph + i * 512);
+    if (has_dh(x.e))
+#pragma unroll
+      for (int i = 0; i < NC; ++i) f.df[i] = *(const bf16x8*)(pd + i * 512);
+  };
+  Step at{0, nlev - 1}, ahead = at;
+  Frags fr[PF];
+#pragma unroll
+  for (int i = 0; i < PF; ++i) {
+    fetch(fr[i], ahead);
+    ahead = after(ahead);
+  }
+  // K_new of this wave's tokens and columns, two K tiles a fragment (an odd last one
+  // alone), for the blocks' dU
+  bf16x8 kf[2][NP];
+#pragma unroll
+  for (int x = 0; x < 2; ++x)
+#pragma unroll
+    for (int y = 0; y < NP; ++y) {
+      const __bf16* p = kn + rowk + (size_t)(16 * (2 * wr + x) + ln) * hk + 16 * (NC * wc + 2 * y);
+      if (2 * y + 1 < NC) {
+        kf[x][y] = row_frag(p);
+      } else {
+        const bf16x4 k4 = *(const bf16x4*)(p + 4 * lq);
+        const __bf16 zero = to16<E>(0.f);
+        kf[x][y] = bf16x8{k4[0], k4[1], k4[2], k4[3], zero, zero, zero, zero};
+      }
+    }
+
+  floatx4 z[ZR][NC], adk[2][NC];
 #pragma unroll
   for (int x = 0; x < ZR; ++x)
 #pragma unroll
-    for (int y = 0; y < NH; ++y) z[x][y] = zero4();
+    for (int y = 0; y < NC; ++y) z[x][y] = zero4();
 #pragma unroll
-  for (int x = 0; x < NX; ++x) adq[x] = zero4();
+  for (int x = 0; x < 2; ++x)
 #pragma unroll
-  for (int x = 0; x < TT; ++x)
-#pragma unroll
-    for (int y = 0; y < NH; ++y) adk[x][y] = zero4();
+    for (int y = 0; y < NC; ++y) adk[x][y] = zero4();
+  float R[NC][8];
+  bf16x8 au[2];   // U of this wave's tokens, the block's columns
 
-  int buf = 0;
-  for (int vb = 0; vb < V / 32; ++vb) {
-    const bf16x8 ao = *(const bf16x8*)(dO + rowv + (size_t)(16 * tw + ln) * hv + 32 * vb + 8 * lq);
-    bf16x8 au[TT];
+  auto begin_block = [&](int vb) __attribute__((always_inline)) {
 #pragma unroll
-    for (int x = 0; x < TT; ++x)
-      au[x] = *(const bf16x8*)(un + rowv + (size_t)(16 * (TT * wr + x) + ln) * hv + 32 * vb + 8 * lq);
-    float R[NH][8];
+    for (int x = 0; x < 2; ++x)
+      au[x] = row_frag(un + rowv + (size_t)(16 * (2 * wr + x) + ln) * hv + 32 * vb);
 #pragma unroll
-    for (int y = 0; y < NH; ++y)
+    for (int y = 0; y < NC; ++y)
 #pragma unroll
       for (int j = 0; j < 8; ++j) R[y][j] = 0.f;
-    floatx4 adu[TT];   // token tile tw, column tiles TT kp + x
+  };
+  auto end_block = [&](int vb) __attribute__((always_inline)) {
+    bf16x8 sel[2];   // selectors of the first and second 16 of 32 contraction indices
 #pragma unroll
-    for (int x = 0; x < TT; ++x) adu[x] = zero4();
-
-    for (int e = top; e >= 0;) {
-      int ne = work_at(e - 1), nvb = vb;
-      if (ne < 0) {
-        ne = top;
-        nvb = vb + 1;
-      }
-      const bool more = nvb < V / 32;
-      if (more) fetch(nvb, ne);
-      const __bf16* Ht = s.tile[buf][0];
-      const __bf16* Dt = s.tile[buf][1];
-      if (!is_set(e)) {
-#pragma unroll
-        for (int y = 0; y < NH; ++y) {
-          const bf16x8 d = tr_frag(Dt, LK, 0, 16 * (NH * wc + y));
-#pragma unroll
-          for (int j = 0; j < 8; ++j) R[y][j] += from16<E>(d[j]);
-        }
-#pragma unroll
-        for (int c = 0; c < NH; ++c) {
-          const bf16x8 a = *(const bf16x8*)(s.kn + (16 * tw + ln) * LK + 32 * c + 8 * lq);
-#pragma unroll
-          for (int x = 0; x < TT; ++x)
-            adu[x] = mfma16<E>(a, *(const bf16x8*)(Dt + (16 * (TT * kp + x) + ln) * LK + 32 * c + 8 * lq), adu[x]);
-        }
-      } else {
-        // dq_new and dlambda: X = dO h^T, this wave's tokens and part of K
-        const floatx4 lam4 = *(const floatx4*)(&s.lam[e][16 * tw + 4 * lq]);
-        float yv[4] = {0.f, 0.f, 0.f, 0.f};
-        bf16x8 ah[ZR];
-#pragma unroll
-        for (int kt = 0; kt < NX; ++kt) {
-          const bf16x8 bh = tr_frag(Ht, LK, 0, 16 * (NX * kp + kt));
-          if constexpr (NW == 4) {   // the fragments are also those of its rows of Z
-            if (kt / ZR == wr) ah[kt % ZR] = bh;
-          }
-          const floatx4 x = mfma16<E>(ao, bh, zero4());
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            adq[kt][i] += lam4[i] * x[i];
-            yv[i] += from16<E>(qd[kt][i]) * x[i];
-          }
-        }
-        if constexpr (NW != 4)
-#pragma unroll
-          for (int x = 0; x < ZR; ++x) ah[x] = tr_frag(Ht, LK, 0, 16 * (ZR * wr + x));
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const float ys = row_sum16(yv[i]);
-          if (ln == 0) s.y[kp][e][16 * tw + 4 * lq + i] += ys;
-        }
-        if (have_dh) {
-          const bool own = has_dh(e);
-#pragma unroll
-          for (int y = 0; y < NH; ++y) {
-            bf16x8 g;
-            if (own) {
-              const bf16x8 d = tr_frag(Dt, LK, 0, 16 * (NH * wc + y));
-#pragma unroll
-              for (int j = 0; j < 8; ++j) g[j] = to16<E>(R[y][j] + from16<E>(d[j]));
-            } else {
-#pragma unroll
-              for (int j = 0; j < 8; ++j) g[j] = to16<E>(R[y][j]);
-            }
-#pragma unroll
-            for (int x = 0; x < ZR; ++x) z[x][y] = mfma16<E>(ah[x], g, z[x][y]);
-          }
-        }
-      }
-      buf ^= 1;
-      if (more) put(buf, ne);
-      __syncthreads();
-      e = nvb == vb ? ne : -1;
+    for (int j = 0; j < 4; ++j) {
+      const __bf16 one = to16<E>(4 * lq + j == ln ? 1.f : 0.f), zero = to16<E>(0.f);
+      sel[0][j] = one;
+      sel[0][4 + j] = zero;
+      sel[1][j] = zero;
+      sel[1][4 + j] = one;
     }
-
-    // U (sum_e wr dh)^T, the sum as hi + lo
-    if (have_dh)
+    floatx4 adu[2][2];
 #pragma unroll
-      for (int y = 0; y < NH; ++y) {
-        bf16x8 hi, lo;
+    for (int x = 0; x < 2; ++x) adu[x][0] = adu[x][1] = zero4();
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          hi[j] = to16<E>(R[y][j]);
-          lo[j] = to16<E>(R[y][j] - from16<E>(hi[j]));
+    for (int y = 0; y < NP; ++y) {
+      bf16x8 part[2][2];   // [K tile of the pair][hi, lo]
+#pragma unroll
+      for (int m = 0; m < 2; ++m)
+        if (2 * y + m < NC) {
+#pragma unroll
+          for (int j = 0; j < 8; ++j) {
+            part[m][0][j] = to16<E>(R[2 * y + m][j]);
+            part[m][1][j] = to16<E>(R[2 * y + m][j] - from16<E>(part[m][0][j]));
+          }
+#pragma unroll
+          for (int x = 0; x < 2; ++x)
+#pragma unroll
+            for (int p = 0; p < 2; ++p)
+              adk[x][2 * y + m] = mfma16<E>(au[x], part[m][p], adk[x][2 * y + m]);
         }
 #pragma unroll
-        for (int x = 0; x < TT; ++x) {
-          adk[x][y] = mfma16<E>(au[x], hi, adk[x][y]);
-          adk[x][y] = mfma16<E>(au[x], lo, adk[x][y]);
+      for (int p = 0; p < 2; ++p)
+#pragma unroll
+        for (int vt = 0; vt < 2; ++vt) {
+          // rows k, columns v of the pair (an odd last tile alone: zero beside it)
+          const floatx4 d0 = mfma16<E>(part[0][p], sel[vt], zero4());
+          const floatx4 d1 = 2 * y + 1 < NC ? mfma16<E>(part[1][p], sel[vt], zero4()) : zero4();
+          const bf16x8 bd = cat8e<E>(d0, d1);
+#pragma unroll
+          for (int x = 0; x < 2; ++x) adu[x][vt] = mfma16<E>(kf[x][y], bd, adu[x][vt]);
         }
+    }
+    // the column parts' shares: wave wc sums tiles (x, vt) = (m >> 1, m & 1), m = wc, ..
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+      for (int vt = 0; vt < 2; ++vt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) s.du[w][2 * x + vt][i][lane] = adu[x][vt][i];
+    __syncthreads();
+#pragma unroll
+    for (int m0 = 0; m0 < 4; m0 += NWC) {
+      const int m = m0 + wc;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        float x = 0.f;
+#pragma unroll
+        for (int c = 0; c < NWC; ++c) x += s.du[NWC * wr + c][m][i][lane];
+        du[rowv + (size_t)(16 * (2 * wr + (m >> 1)) + 4 * lq + i) * hv + 32 * vb + 16 * (m & 1) + ln] = x;
+      }
+    }
+    __syncthreads();
+  };
+  auto level = [&](Frags& f, int e) __attribute__((always_inline)) {
+    if (!is_set(e)) {
+#pragma unroll
+      for (int y = 0; y < NC; ++y)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) R[y][j] += from16<E>(f.df[y][j]);
+      return;
+    }
+    const bool own = has_dh(e);
+#pragma unroll
+    for (int y = 0; y < NC; ++y) {
+      bf16x8 g;
+      if (own) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) g[j] = to16<E>(R[y][j] + from16<E>(f.df[y][j]));
+      } else {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) g[j] = to16<E>(R[y][j]);
       }
 #pragma unroll
-    for (int x = 0; x < TT; ++x)
+      for (int x = 0; x < ZR; ++x) z[x][y] = mfma16<E>(f.hf[x], g, z[x][y]);
+    }
+  };
+  begin_block(0);
+  while (at.vb < nvb) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-        du[rowv + (size_t)(16 * tw + 4 * lq + i) * hv + 32 * vb + 16 * (TT * kp + x) + ln] = adu[x][i];
+    for (int i = 0; i < PF; ++i) {
+      if (at.vb < nvb) {
+        level(fr[i], at.e);
+        fetch(fr[i], ahead);
+        ahead = after(ahead);
+        const Step nx = after(at);
+        if (nx.vb != at.vb) {
+          end_block(at.vb);
+          if (nx.vb < nvb) begin_block(nx.vb);
+        }
+        at = nx;
+      }
+    }
   }
 
   // ---- d exp(Gc_last) = trace Z -------------------------------------------------------
@@ -447,75 +598,66 @@ __global__ __launch_bounds__(64 * GdnLevelSmem<KD>::NW) void gdn_bwd_level_kerne
 #pragma unroll
   for (int x = 0; x < ZR; ++x)
 #pragma unroll
-    for (int y = 0; y < NH; ++y)
-      if (ZR * wr + x == NH * wc + y)
+    for (int y = 0; y < NC; ++y)
+      if (ZR * wr + x == NC * wc + y)
 #pragma unroll
         for (int i = 0; i < 4; ++i) tr += 4 * lq + i == ln ? z[x][y][i] : 0.f;
 #pragma unroll
   for (int off = 32; off >= 1; off >>= 1) tr += __shfl_xor(tr, off, 64);
   if (lane == 0) s.red[w] = tr;
-  __syncthreads();
-  if (tid == 0) {
-    float x = 0.f;
-#pragma unroll
-    for (int i = 0; i < NW; ++i) x += s.red[i];
-    del_p[(size_t)row * NT + ic] = x;
-  }
 
   // ---- dW_new = -K_new Z^T, dK_new -= W_new Z, 64 rows of Z at a time ------------------
+  // of dW_new: token tile tw, column tiles NY kp + y of the 64
+  constexpr int NY = 16 / NW;
+  const int tw = w & 3, kp = w >> 2;
 #pragma unroll
   for (int rb = 0; rb < KD / 64; ++rb) {
-    if (have_dh) {
 #pragma unroll
-      for (int x = 0; x < ZR; ++x) {
-        const int r = 16 * (ZR * wr + x);   // this tile's first row of Z
-        if (r / 64 == rb) {
+    for (int x = 0; x < ZR; ++x) {
+      const int r = 16 * (ZR * wr + x);   // this tile's first row of Z
+      if (r / 64 == rb) {
 #pragma unroll
-          for (int y = 0; y < NH; ++y)
+        for (int y = 0; y < NC; ++y)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-              const int at = (r - 64 * rb + 4 * lq + i) * LK + 16 * (NH * wc + y) + ln;
-              const float v = z[x][y][i];
-              const __bf16 hi = to16<E>(v);
-              s.z[0][at] = hi;
-              s.z[1][at] = to16<E>(v - from16<E>(hi));
-            }
-        }
+          for (int i = 0; i < 4; ++i) {
+            const int to = (r - 64 * rb + 4 * lq + i) * LK + 16 * (NC * wc + y) + ln;
+            const float v = z[x][y][i];
+            const __bf16 hi = to16<E>(v);
+            s.z[0][to] = hi;
+            s.z[1][to] = to16<E>(v - from16<E>(hi));
+          }
       }
-      __syncthreads();
     }
-    constexpr int NY = 4 / Sm::NP;   // column tiles of the block per wave
+    __syncthreads();
     floatx4 adw[NY];
 #pragma unroll
     for (int y = 0; y < NY; ++y) adw[y] = zero4();
-    if (have_dh) {
 #pragma unroll
-      for (int c = 0; c < NH; ++c) {
-        const bf16x8 a = *(const bf16x8*)(s.kn + (16 * tw + ln) * LK + 32 * c + 8 * lq);
+    for (int c = 0; c < KD / 32; ++c) {
+      const bf16x8 a = *(const bf16x8*)(kn + rowk + (size_t)(16 * tw + ln) * hk + 32 * c + 8 * lq);
 #pragma unroll
-        for (int y = 0; y < NY; ++y)
+      for (int y = 0; y < NY; ++y)
 #pragma unroll
-          for (int p = 0; p < 2; ++p)
-            adw[y] = mfma16<E>(a, *(const bf16x8*)(s.z[p] + (16 * (NY * kp + y) + ln) * LK + 32 * c + 8 * lq), adw[y]);
+        for (int p = 0; p < 2; ++p)
+          adw[y] = mfma16<E>(a, *(const bf16x8*)(s.z[p] + (16 * (NY * kp + y) + ln) * LK + 32 * c + 8 * lq), adw[y]);
+    }
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      bf16x8 aw[2];
+#pragma unroll
+      for (int x = 0; x < 2; ++x) {
+        aw[x] = *(const bf16x8*)(wn + rowk + (size_t)(16 * (2 * wr + x) + ln) * hk + 64 * rb + 32 * c + 8 * lq);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) aw[x][j] = to16<E>(-from16<E>(aw[x][j]));
       }
 #pragma unroll
-      for (int c = 0; c < 2; ++c) {
-        bf16x8 aw[TT];
+      for (int y = 0; y < NC; ++y)
 #pragma unroll
-        for (int x = 0; x < TT; ++x) {
-          aw[x] = *(const bf16x8*)(wn + rowk + (size_t)(16 * (TT * wr + x) + ln) * hk + 64 * rb + 32 * c + 8 * lq);
+        for (int p = 0; p < 2; ++p) {
+          const bf16x8 bz = tr_frag(s.z[p], LK, 32 * c, 16 * (NC * wc + y));
 #pragma unroll
-          for (int j = 0; j < 8; ++j) aw[x][j] = to16<E>(-from16<E>(aw[x][j]));
+          for (int x = 0; x < 2; ++x) adk[x][y] = mfma16<E>(aw[x], bz, adk[x][y]);
         }
-#pragma unroll
-        for (int y = 0; y < NH; ++y)
-#pragma unroll
-          for (int p = 0; p < 2; ++p) {
-            const bf16x8 bz = tr_frag(s.z[p], LK, 32 * c, 16 * (NH * wc + y));
-#pragma unroll
-            for (int x = 0; x < TT; ++x) adk[x][y] = mfma16<E>(aw[x], bz, adk[x][y]);
-          }
-      }
     }
 #pragma unroll
     for (int y = 0; y < NY; ++y)
@@ -525,32 +667,17 @@ __global__ __launch_bounds__(64 * GdnLevelSmem<KD>::NW) void gdn_bwd_level_kerne
     __syncthreads();
   }
 #pragma unroll
-  for (int kt = 0; kt < NX; ++kt)
+  for (int x = 0; x < 2; ++x)
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      dqn[rowk + (size_t)(16 * tw + 4 * lq + i) * hk + 16 * (NX * kp + kt) + ln] = (__bf16)adq[kt][i];
-#pragma unroll
-  for (int x = 0; x < TT; ++x)
-#pragma unroll
-    for (int y = 0; y < NH; ++y)
+    for (int y = 0; y < NC; ++y)
 #pragma unroll
       for (int i = 0; i < 4; ++i)
-        dkn[rowk + (size_t)(16 * (TT * wr + x) + 4 * lq + i) * hk + 16 * (NH * wc + y) + ln] = (__bf16)adk[x][y][i];
-
-  // ---- dlambda ------------------------------------------------------------------------
-  for (int u = tid; u < nlev * kGC; u += NTH) {
-    const int t = u / nlev, e = u % nlev;
-    auto read = [&](int j) { return Sm::NP == 1 ? s.y[0][j][t] : s.y[0][j][t] + s.y[Sm::NP - 1][j][t]; };
+        dkn[rowk + (size_t)(16 * (2 * wr + x) + 4 * lq + i) * hk + 16 * (NC * wc + y) + ln] = (__bf16)adk[x][y][i];
+  if (tid == 0) {
     float x = 0.f;
-    if (strong ? e >= 1 : is_set(e)) {
-      if (is_set(e)) {
-        x = read(e);
-      } else {
-        for (int j = 0; j < e; ++j)
-          if (is_set(j)) x += read(j);
-      }
-    }
-    dl_p[((tok0 + t) * H + h) * nlev + e] = x;
+#pragma unroll
+    for (int i = 0; i < NW; ++i) x += s.red[i];
+    del_p[(size_t)row * NT + ic] = x;
   }
 }
 
@@ -561,9 +688,9 @@ template <int KD, int NW, typename TL, typename E>
 static hipError_t gdn_dh_scan_launch(const GdnBwdWs& w, const void* dO, const float* gcum,
                                      const void* l, int rows, int T, int H, int V, int L, int nlev,
                                      int strong, hipStream_t stream) {
-  constexpr int BV = gdn_scan_bv(KD);
+  constexpr int BV = gdn_dh_bv(KD, NW);
   auto ks = gdn_dh_scan_kernel<KD, BV, NW, TL, E>;
-  const int smem = (int)sizeof(GdnDhSmem<KD, BV, KD <= 192>);
+  const int smem = (int)sizeof(GdnDhSmem<KD, BV, gdn_dh_two_buffers(KD, BV)>);
   const int nparts = (nlev + NW - 1) / NW;
   hipError_t e = hipFuncSetAttribute((const void*)ks, hipFuncAttributeMaxDynamicSharedMemorySize, smem);
   if (e != hipSuccess) return e;
@@ -579,21 +706,23 @@ static hipError_t gdn_levels_launch(const GdnBwdWs& w, const void* dO, const flo
                                     int strong, hipStream_t stream) {
   hipError_t e;
   if (nlev > 0) {
-    // four levels per workgroup where one workgroup per (row, V slice) would leave
-    // CUs idle
-    const bool narrow = nlev <= 4 || (long)B * H * (V / gdn_scan_bv(KD)) < kGdnScanGroups;
+    // four levels per workgroup where their workgroups still run all at once, one per CU
+    const bool narrow = nlev <= 4 || 2L * B * H * (V / gdn_dh_bv(KD, 4)) <= kGdnScanGroups;
     e = narrow ? gdn_dh_scan_launch<KD, 4, TL, E>(w, dO, gcum, l, B * H, T, H, V, L, nlev, strong, stream)
                : gdn_dh_scan_launch<KD, 8, TL, E>(w, dO, gcum, l, B * H, T, H, V, L, nlev, strong, stream);
     if (e != hipSuccess) return e;
   }
-  auto ks = gdn_bwd_level_kernel<KD, TL, E>;
+  const int nchunks = B * H * (T / kGC);
+  hipLaunchKernelGGL((gdn_bwd_read_kernel<KD, TL, E>), dim3(nchunks), dim3(256), 0, stream, w.qn,
+                     (const __bf16*)dO, (const TL*)l, w.hs, w.dq_p, w.dl_p, T, H, V, L, nlev, strong);
+  if ((e = hipGetLastError()) != hipSuccess) return e;
+  auto ks = gdn_bwd_level_kernel<KD, E>;
   const int smem = (int)sizeof(GdnLevelSmem<KD>);
   if ((e = hipFuncSetAttribute((const void*)ks, hipFuncAttributeMaxDynamicSharedMemorySize, smem)) !=
       hipSuccess)
     return e;
-  hipLaunchKernelGGL(ks, dim3(B * H * (T / kGC)), dim3(64 * GdnLevelSmem<KD>::NW), smem, stream, w.qn,
-                     w.wn, w.kn, w.un, (const __bf16*)dO, (const TL*)l, w.hs, w.dhs, w.dq_p, w.dw_p,
-                     w.dk_p, w.du, w.dl_p, w.del_p, T, H, V, L, nlev, strong);
+  hipLaunchKernelGGL(ks, dim3(nchunks), dim3(64 * GdnLevelSmem<KD>::NW), smem, stream, w.wn, w.kn, w.un, w.hs, w.dhs,
+                     w.dw_p, w.dk_p, w.du, w.del_p, T, H, V, nlev);
   return hipGetLastError();
 }
 

@@ -28,6 +28,50 @@ __host__ __device__ inline size_t gdn_set_before(int n) {
   return x;
 }
 
+// A kept state [K x V] (and the backward's dh) is stored as the operand fragments of
+// products that contract over V, so that their reader loads them straight from memory:
+// [V / 32][K / 16][lane][8] 16-bit values, lane (lq, ln) of k tile kt holding row k = 16
+// kt + ln and columns 32 vb + {4 lq + 0..3, 16 + 4 lq + 0..3}.
+// store_state_frags: one wave's columns v0 .. v0 + BV - 1 of a state in accumulator
+// layout (st[kt][nt]: rows 16 kt + 4 lq + i, columns 16 nt + ln).  The transposition is
+// a product with a 0 / 1 selector, exact in either 16-bit format: the accumulators as A
+// operand (lane = column, contraction over k) against the selector of 16 of the 32 k
+// give D[v][k].  (Stored [v][k] and transposed by the reader through LDS, with a barrier
+// per level, the level sums took 2.17 ms at B 4, T 8192, H 16, K = V = 128.)
+template <int KD, int BV, typename E>
+__device__ __forceinline__ void store_state_frags(const floatx4 (&st)[KD / 16][BV / 16],
+                                                  __bf16* slot, int v0) {
+  constexpr int NKT = KD / 16, NVT = BV / 16;
+  const int lane = threadIdx.x & 63, lq = lane >> 4, ln = lane & 15;
+  bf16x8 sel[2];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const __bf16 one = to16<E>(4 * lq + j == ln ? 1.f : 0.f), zero = to16<E>(0.f);
+    sel[0][j] = one;
+    sel[0][4 + j] = zero;
+    sel[1][j] = zero;
+    sel[1][4 + j] = one;
+  }
+  const rsrc_t r = make_rsrc(slot + (size_t)(v0 / 32) * 32 * KD, (size_t)32 * KD * 2);
+#pragma unroll
+  for (int c = 0; c < NKT / 2; ++c) {
+    bf16x8 a[NVT];
+#pragma unroll
+    for (int nt = 0; nt < NVT; ++nt) a[nt] = cat8e<E>(st[2 * c][nt], st[2 * c + 1][nt]);
+#pragma unroll
+    for (int hf = 0; hf < 2; ++hf) {
+      floatx4 d[NVT];
+#pragma unroll
+      for (int nt = 0; nt < NVT; ++nt) d[nt] = mfma16<E>(a[nt], sel[hf], zero4());
+      const unsigned off = (unsigned)(((2 * c + hf) * 64 + lane) * 16);
+      if constexpr (NVT == 2)
+        buf_store16(__builtin_bit_cast(uint4, cat8e<E>(d[0], d[1])), r, off, 0);
+      else
+        buf_store8(__builtin_bit_cast(uint2, cvt4e<E>(d[0])), r, off + ((v0 / 16) & 1) * 8, 0);
+    }
+  }
+}
+
 // HType.STRONG intra-chunk levels: the reference's chunkwise GDN path takes
 // lambda of a pair inside a chunk at its strong level (make_levels_matrix with
 // htype STRONG, chunkwise_hgdn.py:630), which on an aligned 64-token chunk is

@@ -543,8 +543,8 @@ __global__ __launch_bounds__(512) void gdn_scan_kernel(
   const rsrc_t ro = make_rsrc(o_ok ? (const void*)(o + rowtok * V + v0) : (const void*)gcum,
                               o_ok ? (size_t)T * H * V * sizeof(TO) : 0);
   const unsigned o_voff = ((o_ok ? ot : 0) * HV + ov) * sizeof(TO);
-  // hsave: [row][states of the set levels, chunk by chunk][v][k]
-  __bf16* hrow = kSave ? hsave + ((size_t)row * gdn_set_before(NT) * V + v0) * KD : nullptr;
+  // hsave: [row][states of the set levels, chunk by chunk]
+  __bf16* hrow = kSave ? hsave + (size_t)row * gdn_set_before(NT) * V * KD : nullptr;
 
   stage_load(0);
   stage_store();
@@ -568,13 +568,7 @@ __global__ __launch_bounds__(512) void gdn_scan_kernel(
       // the state of a level that this chunk reads, at the chunk start
       if (act && bit) {
         const size_t slot = gdn_set_before(ic) + __builtin_popcount(ic & ((1 << e) - 1));
-        const rsrc_t rh = make_rsrc(hrow + slot * V * KD, (size_t)BV * KD * 2);
-#pragma unroll
-        for (int kt = 0; kt < NKT; ++kt)
-#pragma unroll
-          for (int nt = 0; nt < NVT; ++nt)
-            buf_store8(__builtin_bit_cast(uint2, cvt4e<E>(st[kt][nt])), rh,
-                       (unsigned)(((16 * nt + ln) * KD + 16 * kt + 4 * lq) * 2), 0);
+        store_state_frags<KD, BV, E>(st, hrow + slot * V * KD, v0);
       }
     }
     if constexpr (kOut) {
@@ -744,8 +738,8 @@ inline GdnWs gdn_ws_layout(void* base, int B, int T, int H, int K, int V) {
 }
 
 // The forward that keeps, for the backward, what its recompute would produce:
-// the forward's buffers, then the token-major K_new and every level's state at
-// every chunk start (bf16 [row][chunk][level][v][k], the backward's layout).
+// the forward's buffers, then the token-major K_new and the state of every level
+// that a chunk reads, at the chunk's start (16-bit fragments, gdn_common.h).
 struct GdnKeepWs {
   GdnWs f;
   __bf16 *kn, *hs;
