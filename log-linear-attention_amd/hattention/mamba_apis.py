@@ -25,7 +25,8 @@ import torch
 from hattention.base import HType, HStruct
 from hattention.kernel import hattention_kernel, hattention_prefill
 from hattention.mamba_layer import (CausalConv1dSilu, GatedRMSNorm, HMambaScanFunction,
-                                     lambda_mode_code, layer_epilogue, layer_prologue)
+                                     HMambaSplitFunction, lambda_mode_code, layer_epilogue,
+                                     layer_prologue)
 
 
 def compute_lambda(L: torch.Tensor, dl: torch.Tensor, lambda_mode: Optional[str]) -> torch.Tensor:
@@ -194,6 +195,14 @@ def hmamba_split_conv1d_scan_combined(
 
     gn = ngroups * dstate
     Dc = dim + 2 * gn
+    if lambda_level_fixed:
+        # one autograd node from zxbcdtdl to the out-projection's input
+        _check_scan_args(lambda_level_max, lambda_level_base, lambda_htype, lambda_hstruct,
+                         lambda_level_fixed, lambda_mode, dlambda, dlambda)
+        y = HMambaSplitFunction.apply(zxbcdtdl, conv1d_weight, conv1d_bias, dt_bias, A, L, D,
+                                      rmsnorm_weight, rmsnorm_eps, headdim, ngroups, dstate,
+                                      lambda_mode, lambda_level_base, lambda_htype)
+        return torch.nn.functional.linear(y, outproj_weight, outproj_bias)
     x, Bm, Cm = CausalConv1dSilu.apply(zxbcdtdl, dim, Dc, dim, dim + gn, conv1d_weight,
                                        conv1d_bias)
     c_dt = dim + Dc
@@ -212,6 +221,21 @@ def hmamba_split_conv1d_scan_combined(
     y = GatedRMSNorm.apply(y.reshape(batch, seqlen, dim), zxbcdtdl, 0, rmsnorm_weight,
                            rmsnorm_eps)
     return torch.nn.functional.linear(y, outproj_weight, outproj_bias)
+
+
+def _check_scan_args(lambda_level_max, lambda_level_base, lambda_htype, lambda_hstruct,
+                     lambda_level_fixed, lambda_mode, levels_L, levels_dl):
+    """The lambda options every scan of the layer needs (mamba_apis.py:96-102, 329-345)."""
+    for arg in (lambda_level_max, lambda_level_base, lambda_htype, lambda_hstruct,
+                lambda_level_fixed):
+        if arg is None:
+            raise ValueError
+    if levels_L != lambda_level_max or levels_dl != lambda_level_max:
+        raise ValueError
+    lambda_mode_code(lambda_mode)
+    if lambda_hstruct != HStruct.MAMBA2:
+        # the reference calls hattention_kernel with b=None, which GDELTA rejects
+        raise ValueError
 
 
 def hmamba_chunk_scan_combined(
