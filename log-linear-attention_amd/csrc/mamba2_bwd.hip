@@ -16,7 +16,7 @@
 // (the last identity is what the reference's reverse chunk-local cumsum of its
 // dg accumulator computes, chunkwise.py:1596).
 //
-// Segments of S = 16 chunks as in the forward.  Inter-chunk level e is a
+// Segments of S = 16 chunks as in the forward, or fewer (bwd_seg_log2).  Inter-chunk level e is a
 // source for chunk j when bit e of j is clear and is read when it is set.
 //   * mamba2_seg_sum_kernel<.., GCUM, ..>: forward summaries Sum(q), D_q (shared with
 //     the forward).
@@ -1305,9 +1305,33 @@ struct BwdWs {
 
 inline size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
-inline BwdWs bwd_ws_layout(void* base, int B, int T, int H, int V, int nlev) {
+// log2 of the chunks per segment of the backward: the forward's segments, halved as long
+// as there is at most one workgroup (a row and segment) per CU and at most 16 segments.
+// A workgroup walks its chunks one after the other, so a small problem's time is the
+// length of that walk.  Forward and backward in us, before and with the finer segments
+// (H = G, K = V = 64): 32 rows T 2048 253 -> 149, 8 rows T 4096 271 -> 171, 8 rows
+// T 8192 297 -> 230; fp32 8 rows T 1024 348 -> 178, 4 rows T 2048 532 -> 312.
+// Past one workgroup per CU it only adds passes (240 rows T 1024 207 -> 228), and past 16
+// segments the scan over them takes what the walk saves (8 rows T 4096 171 -> 190 at 32).
+// A 16-bit sequence of one forward segment stays whole: the finer backward would add
+// four launches to its two, and its 8 rows T 1024 take 191 -> 98 on the device but
+// 198 -> 207 called one by one from a host that needs that long for a forward and
+// backward.
+constexpr int kBwdMaxGroups = 256, kBwdMaxSeg = 16;
+inline int bwd_seg_log2(int rows, int NT, bool fp32) {
+  int s = seg_log2(NT);
+  if (!fp32 && NT <= (1 << kMaxLoc)) return s;
+  while (s > 1) {
+    const int nseg = (NT + (1 << (s - 1)) - 1) >> (s - 1);
+    if (nseg > kBwdMaxSeg || (long)rows * nseg > kBwdMaxGroups) break;
+    --s;
+  }
+  return s;
+}
+
+inline BwdWs bwd_ws_layout(void* base, int B, int T, int H, int V, int nlev, bool fp32) {
   const int NT = T / kBT;
-  const int slog = seg_log2(NT);
+  const int slog = bwd_seg_log2(B * H, NT, fp32);
   const int NSEG = (NT + (1 << slog) - 1) >> slog;
   const int ntop = nlev - min(slog, nlev);
   const size_t rows = (size_t)B * H;
@@ -1326,8 +1350,8 @@ inline BwdWs bwd_ws_layout(void* base, int B, int T, int H, int V, int nlev) {
 }
 
 // fsums / fsegd (or null): the forward's segment summaries and log-decays of
-// these inputs (its workspace, same segmentation and layout), which then
-// replace the summary pass.
+// these inputs (its workspace, same layout), which replace the summary pass where
+// the backward takes the forward's segments.
 // E: the 16-bit MFMA format (NP = 1): bf16, or fp16 for fp16 q / k / v / dO.
 template <int NP, typename TK, typename TV, typename TL, typename E = __bf16>
 static hipError_t bwd_launch_t(const void* q, const void* k, const void* v, const float* gc,
@@ -1336,12 +1360,12 @@ static hipError_t bwd_launch_t(const void* q, const void* k, const void* v, cons
                                const float* fsegd, int B, int T, int H, int V, int L, int nlev,
                                hipStream_t stream) {
   const int NT = T / kBT;
-  const int slog = seg_log2(NT);
+  const int rows = B * H;
+  const int slog = bwd_seg_log2(rows, NT, NP == 2);
   const int NSEG = (NT + (1 << slog) - 1) >> slog;
   const int nloc = min(slog, nlev), ntop = nlev - nloc;
-  const int rows = B * H;
-  const BwdWs w = bwd_ws_layout(ws, B, T, H, V, nlev);
-  const bool reuse = fsums != nullptr && fsegd != nullptr;
+  const BwdWs w = bwd_ws_layout(ws, B, T, H, V, nlev, NP == 2);
+  const bool reuse = fsums != nullptr && fsegd != nullptr && slog == seg_log2(NT);
   const float* sums = reuse ? fsums : w.sums;
   const float* segd = reuse ? fsegd : w.segd;
   hipError_t e;
@@ -1392,7 +1416,8 @@ static hipError_t bwd_launch_t(const void* q, const void* k, const void* v, cons
 }  // namespace hattn
 
 size_t hattn_mamba2_bwd_ws_bytes(int B, int T, int H, int V, int nlev) {
-  return hattn::bwd_ws_layout(nullptr, B, T, H, V, nlev).bytes;
+  // the fp32 backward's segments are the same or finer
+  return hattn::bwd_ws_layout(nullptr, B, T, H, V, nlev, true).bytes;
 }
 
 // dt_qk (= the dtype of dO): bf16 selects the bf16 kernels (v and lambda bf16 or

@@ -147,6 +147,23 @@ def test_forward_summaries_reused(T):
         assert mx < 1e-2 and fro < 2e-3, (name, mx, fro)
 
 
+# The backward's segments against one workgroup per CU (256) and 16 segments:
+# (2048, 1): 16 segments, the most; (2112, 1): one chunk more, so 4-chunk segments;
+# (1088, 85): 255 workgroups with 8-chunk segments, the last of one chunk; (1088, 86):
+# 258, so the forward's segments and its summaries; fp32 (704, 1): 2-chunk segments in
+# a sequence of one forward segment.
+@pytest.mark.parametrize("T,H,dtype", [(2048, 1, torch.bfloat16), (2112, 1, torch.bfloat16),
+                                       (1088, 85, torch.bfloat16), (1088, 86, torch.bfloat16),
+                                       (704, 1, torch.float32), (2048, 1, torch.float32)])
+def test_backward_segments(T, H, dtype):
+    L = 7 + math.ceil(math.log2(T // 64))
+    if dtype == torch.float32:
+        _run_x3(1, T, H, 64, 64, L, seed=T + H)
+        return
+    _run(1, T, H, 64, 64, L, seed=T + H, rows=[(0, 0), (0, H - 1)] if H > 1 else None,
+         reuse=True)
+
+
 def test_forward_workspace_kept_only_where_reused():
     """chunkwise_fwd_keep returns its workspace only for the backward that can
     take the summaries (bf16 q / k, K = V = 64, WEAK, several segments); a
