@@ -338,8 +338,9 @@ int hattn_gdn_chunkwise_bwd(const void* q, const void* k, const void* v, const v
                             size_t workspace_bytes, void* stream);
 
 /* Workspace bytes of hattn_gdn_chunkwise_bwd: the recomputed q_new, k_new (token-major
- * and per-chunk transposed), w_new, u (bf16), every level's state at every chunk start (bf16), and the
- * per-V-slice partial gradients of the level scan.  No counterpart in the
+ * and per-chunk transposed), w_new, u (bf16), the states of
+ * the levels set in each chunk's index at its start (16-bit), the reverse states of the
+ * other levels, and the level sums (dq_new, dw_new, dk_new, dU).  No counterpart in the
  * reference, which allocates h / dh and its temporaries with torch inside
  * chunkwise_bwd (chunkwise_hgdn.py:894-913). */
 size_t hattn_gdn_chunkwise_bwd_workspace(int B, int T, int H, int K, int V, int L);

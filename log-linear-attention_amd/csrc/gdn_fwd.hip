@@ -752,9 +752,10 @@ inline GdnKeepWs gdn_keep_ws_layout(void* base, int B, int T, int H, int K, int 
   char* p = (char*)base;
   size_t off = w.f.bytes;
   const size_t n = (size_t)B * T * H, NT = (size_t)T / kGC;
-  (void)nlev;
   w.kn = (__bf16*)(p + off); off += galign(n * K * 2);
-  w.hs = (__bf16*)(p + off); off += galign((size_t)B * H * gdn_set_before((int)NT) * V * K * 2);
+  // sized for every level of every chunk, as callers of the query may count on; the set
+  // levels' states take the first half or so
+  w.hs = (__bf16*)(p + off); off += galign((size_t)B * H * NT * nlev * V * K * 2);
   w.bytes = off;
   return w;
 }
@@ -863,7 +864,7 @@ void hattn_gdn_fwd_keep_buffers(const void* ws, int B, int T, int H, int K, int 
 }
 
 // The forward plus, in the workspace, the backward's recompute results
-// (q_new, W_new, K_new, U, every level's state at every chunk start).
+// (q_new, W_new, K_new, U, the set levels' states at every chunk start).
 hipError_t hattn_gdn_fwd_keep_launch(const void* q, const void* k, const void* v,
                                      const void* beta, const float* g, const void* l, void* o,
                                      float* gcum, void* aw, void* au, float* ht, void* ws, int B,

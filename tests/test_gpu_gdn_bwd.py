@@ -219,3 +219,33 @@ def test_kept_forward_not_offered_for_wide_v():
     B, T, H, K, V, L = 1, 256, 2, 64, 192, 9
     xs = [x.to("cuda:0") for x in make_gdn_inputs(B, T, H, K, V, L, seed=1)]
     assert chunkwise_fwd_keep(*xs, False, 2, HType.WEAK, 64, False)[5] is None
+
+
+@pytest.mark.parametrize("T,K,V", [(128, 64, 192), (1088, 128, 384), (640, 192, 192)])
+def test_kept_forward_of_any_v_gives_the_same_gradients(T, K, V):
+    """keep_any_v: the workspace of a V outside {64, 128} holds what the backward would
+    recompute, so outputs and gradients are equal bit for bit."""
+    from hattention.chunkwise_hgdn import chunkwise_fwd, chunkwise_fwd_keep, chunkwise_bwd
+    from hattention.base import HType
+    L = 7 + math.ceil(math.log2(T // 64))
+    xs = [x.cuda() for x in make_gdn_inputs(1, T, 2, K, V, L, seed=T + V)]
+    do = torch.randn(1, T, 2, V, generator=torch.Generator().manual_seed(6)).bfloat16().cuda()
+    print(f"[gdn keep any v] T={T} K={K} V={V}", flush=True)
+    gc, o, Aw, Au, _ = chunkwise_fwd(*xs, False, 2, HType.WEAK, 64, False)
+    ref = chunkwise_bwd(*xs[:4], gc, xs[5], Aw, Au, do, False, 2, HType.WEAK, 64)
+    kept = chunkwise_fwd_keep(*xs, False, 2, HType.WEAK, 64, False, keep_any_v=True)
+    assert kept[5] is not None and torch.equal(kept[1], o)
+    got = chunkwise_bwd(*xs[:4], kept[0], xs[5], kept[2], kept[3], do, False, 2, HType.WEAK, 64,
+                        fwd_ws=kept[5])
+    for name, a, r in zip(NAMES, got, ref):
+        assert torch.equal(a, r), (name, (a.float() - r.float()).abs().max().item())
+
+
+# Both sides of the reverse scan's choice of four or eight waves: four up to four levels
+# (T 1024) or up to 256 workgroups (2 rows V / 32), eight beyond (T 1088 and 66 rows).
+@pytest.mark.parametrize("T,H,K,V", [(1024, 66, 64, 64), (1088, 64, 64, 64), (1088, 66, 64, 64),
+                                     (1088, 66, 128, 64), (1088, 66, 192, 64),
+                                     (1088, 34, 256, 64), (2048, 33, 192, 128)])
+def test_reverse_scan_four_and_eight_waves(T, H, K, V):
+    _run(1, T, H, K, V, 7 + math.ceil(math.log2(T // 64)), seed=T + H + K,
+         rows=[(0, 0), (0, H - 1)])
