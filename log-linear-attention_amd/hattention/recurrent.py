@@ -247,10 +247,14 @@ def launch_layer_step(S: HState, x, dt, A, dt_bias, Bm, Cm, dl, Lp, D, dt_softpl
             t = t.contiguous()
         ops.append(t)
     x, dt, A, dt_bias, Bm, Cm, dl, Lp, D = ops
-    if x.shape != (B, H, P) or Bm.shape[0] != B or Bm.shape[2] != N or dl.shape != (B, H, L):
-        raise ValueError(f"the state {tuple(S.shape)} does not fit the operands")
     out_dtype = v_dtype if D is None else \
         torch.promote_types(v_dtype, torch.promote_types(x.dtype, D.dtype))
+    # per-head parameters of any other dtype: as fp32, as the layer's prologue and
+    # epilogue take them
+    A, dt_bias, D = (t if t is None or t.dtype in (torch.bfloat16, torch.float32) else t.float()
+                     for t in (A, dt_bias, D))
+    if x.shape != (B, H, P) or Bm.shape[0] != B or Bm.shape[2] != N or dl.shape != (B, H, L):
+        raise ValueError(f"the state {tuple(S.shape)} does not fit the operands")
     out = torch.empty(B, H, P, dtype=out_dtype, device=st.device)
     dc = _lib.DTYPE_CODES
     try:

@@ -53,3 +53,30 @@ def test_layer_step_types(act, par, mode, bias, resid):
 def test_layer_step_sizes(B, H, P, N, G, L):
     _run(B, H, P, N, G, L, BF, BF, "positive", True, True)
     _run(B, H, P, N, G, L, BF, BF, "positive", True, True, strong=True)
+
+
+@pytest.mark.parametrize("which", ["A", "dt_bias", "D"])
+def test_layer_step_half_parameters(which):
+    """fp16 per-head parameters are taken as their fp32 values."""
+    from hattention.base import HStruct, HType
+    from hattention.mamba_apis import hselective_state_update
+    from hattention.recurrent import HState
+    print(f"[layer step] fp16 {which}", flush=True)
+    B, H, P, N, L = 2, 4, 64, 64, 9
+    gen = torch.Generator(DEV).manual_seed(3)
+    rn = lambda *s: torch.randn(*s, device=DEV, generator=gen)
+    x, dt, dl, Lp = rn(B, H, P), rn(B, H), rn(B, H, L), rn(H, L)
+    Bm, Cm = rn(B, 1, N), rn(B, 1, N)
+    par = dict(A=-rn(H).abs(), dt_bias=rn(H), D=rn(H))
+    half = dict(par, **{which: par[which].half()})
+    outs = []
+    for p in (half, {n: t.float() for n, t in half.items()}):
+        S = HState(2, HType.WEAK, HStruct.MAMBA2, (B, H, N, P, L), F32, DEV)
+        out, S = hselective_state_update(
+            S, x, dt, p["A"], Bm, Cm, dl, Lp, D=p["D"], dt_bias=p["dt_bias"], dt_softplus=True,
+            lambda_mode="positive", lambda_level_max=L, lambda_level_base=2,
+            lambda_htype=HType.WEAK, lambda_hstruct=HStruct.MAMBA2, lambda_level_fixed=True)
+        outs.append((out, S.states))
+    assert outs[0][0].dtype == F32
+    for a, b in zip(*outs):
+        assert torch.equal(a, b)
