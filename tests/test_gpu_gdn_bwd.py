@@ -249,3 +249,28 @@ def test_kept_forward_of_any_v_gives_the_same_gradients(T, K, V):
 def test_reverse_scan_four_and_eight_waves(T, H, K, V):
     _run(1, T, H, K, V, 7 + math.ceil(math.log2(T // 64)), seed=T + H + K,
          rows=[(0, 0), (0, H - 1)])
+
+
+@pytest.mark.parametrize("V", [64, 192])
+def test_forward_keeps_nothing_without_gradients(V, monkeypatch):
+    """Inputs without gradients: the forward keeps no workspace and gives the same bits
+    as the forward that keeps it."""
+    from hattention import chunkwise_hgdn as hg
+    from hattention.base import HStruct, HType
+    from hattention.kernel import hattention_kernel
+    kept, real = [], hg.chunkwise_fwd_keep
+
+    def record(*a, **kw):
+        res = real(*a, **kw)
+        kept.append(res[5] is not None)
+        return res
+    monkeypatch.setattr(hg, "chunkwise_fwd_keep", record)
+    T, K = 256, 64
+    xs = [x.cuda() for x in make_gdn_inputs(1, T, 2, K, V, 9, seed=V)]
+    print(f"[gdn keep] V={V}", flush=True)
+    call = lambda v: hattention_kernel(xs[0], xs[1], v, *xs[3:], 0.125, False, 2, HType.WEAK,
+                                       HStruct.GDELTA, use_qk_l2norm_in_kernel=True)
+    o = call(xs[2])
+    og = call(xs[2].clone().requires_grad_())
+    assert kept == [False, True] and torch.equal(o, og.detach())
+    assert og.grad_fn is not None
