@@ -369,6 +369,7 @@ struct GdnLevelSmem {
     float du[NW][4][4][64];    // each wave's share of dU: [token, column tile][row][lane]
   };
   float red[NW];
+  int bad[NW];
 };
 
 // dU, Z, dW_new, dK_new and trace Z.  Four waves (eight for K > 128, where four would
@@ -381,6 +382,13 @@ struct GdnLevelSmem {
 // product, as 16-bit hi and lo, like every fp32 operand here) and its part of dK_new.  Z,
 // whose products with W_new and K_new contract over either index, passes through LDS 64
 // rows at a time.
+// fp16: sums that are larger than any of their terms (dh over the levels, Z over all of
+// V) are kept in range: Z's planes are scaled by a power of two from its largest element,
+// and where a sum of dh overflows, all is done again on dh / 8.  (Unscaled, dK and dg were
+// NaN at gradients 16 times below those at which any dh leaves fp16.  The scaling takes
+// 140 of 6030 us of a training step at B 4, T 8192, H 16, K = V = 128, 53 of 2150 at B 1,
+// T 4096, H 8, K 256, V 128; at K 192, V 384 other registers spill and it is 140 of 1690
+// us faster.)
 // (One kernel with the reads as well took 2.6 ms at B 4, T 8192, H 16, K = V = 128: 250
 // registers with spills, one workgroup per CU, two thirds of its cycles waiting.)
 template <int KD, typename E>
@@ -395,6 +403,7 @@ __global__ __launch_bounds__(64 * GdnLevelSmem<KD>::NW, KD <= 128 ? 2 : 1) void 
   constexpr int NW = Sm::NW, NWC = Sm::NWC, NTH = 64 * NW, LK = Sm::LK;
   constexpr int NKT = KD / 16, NC = NKT / NWC, ZR = NKT / 2, NP = (NC + 1) / 2;
   constexpr int PF = KD <= 64 ? 2 : 1;   // levels loaded ahead (registers)
+  constexpr bool kHalf = __is_same(E, _Float16);
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lq = lane >> 4, ln = lane & 15, wr = w / NWC, wc = w % NWC;
   const int NT = T / kGC;
@@ -444,13 +453,17 @@ __global__ __launch_bounds__(64 * GdnLevelSmem<KD>::NW, KD <= 128 ? 2 : 1) void 
 #pragma unroll
       for (int i = 0; i < NC; ++i) f.df[i] = *(const bf16x8*)(pd + i * 512);
   };
-  Step at{0, nlev - 1}, ahead = at;
   Frags fr[PF];
+  auto fetch_first = [&]() __attribute__((always_inline)) {
+    Step x{0, nlev - 1};
 #pragma unroll
-  for (int i = 0; i < PF; ++i) {
-    fetch(fr[i], ahead);
-    ahead = after(ahead);
-  }
+    for (int i = 0; i < PF; ++i) {
+      fetch(fr[i], x);
+      x = after(x);
+    }
+    return x;
+  };
+  Step ahead = fetch_first();
   // K_new of this wave's tokens and columns, two K tiles a fragment (an odd last one
   // alone), for the blocks' dU
   bf16x8 kf[2][NP];
@@ -469,14 +482,9 @@ __global__ __launch_bounds__(64 * GdnLevelSmem<KD>::NW, KD <= 128 ? 2 : 1) void 
     }
 
   floatx4 z[ZR][NC], adk[2][NC];
-#pragma unroll
-  for (int x = 0; x < ZR; ++x)
-#pragma unroll
-    for (int y = 0; y < NC; ++y) z[x][y] = zero4();
-#pragma unroll
-  for (int x = 0; x < 2; ++x)
-#pragma unroll
-    for (int y = 0; y < NC; ++y) adk[x][y] = zero4();
+  // fp16: the sums of dh over levels are taken times hs1, so that they stay below the
+  // format's 65504 where every dh does (1, or 1/8 in a second pass)
+  float hs1 = 1.f, zmax = 0.f;
   float R[NC][8];
   bf16x8 au[2];   // U of this wave's tokens, the block's columns
 
@@ -547,17 +555,19 @@ __global__ __launch_bounds__(64 * GdnLevelSmem<KD>::NW, KD <= 128 ? 2 : 1) void 
         float x = 0.f;
 #pragma unroll
         for (int c = 0; c < NWC; ++c) x += s.du[NWC * wr + c][m][i][lane];
+        if (kHalf) x *= 1.f / hs1;
         du[rowv + (size_t)(16 * (2 * wr + (m >> 1)) + 4 * lq + i) * hv + 32 * vb + 16 * (m & 1) + ln] = x;
       }
     }
     __syncthreads();
   };
+  auto dh_of = [&](__bf16 x) { return kHalf ? from16<E>(x) * hs1 : from16<E>(x); };
   auto level = [&](Frags& f, int e) __attribute__((always_inline)) {
     if (!is_set(e)) {
 #pragma unroll
       for (int y = 0; y < NC; ++y)
 #pragma unroll
-        for (int j = 0; j < 8; ++j) R[y][j] += from16<E>(f.df[y][j]);
+        for (int j = 0; j < 8; ++j) R[y][j] += dh_of(f.df[y][j]);
       return;
     }
     const bool own = has_dh(e);
@@ -566,7 +576,7 @@ __global__ __launch_bounds__(64 * GdnLevelSmem<KD>::NW, KD <= 128 ? 2 : 1) void 
       bf16x8 g;
       if (own) {
 #pragma unroll
-        for (int j = 0; j < 8; ++j) g[j] = to16<E>(R[y][j] + from16<E>(f.df[y][j]));
+        for (int j = 0; j < 8; ++j) g[j] = to16<E>(R[y][j] + dh_of(f.df[y][j]));
       } else {
 #pragma unroll
         for (int j = 0; j < 8; ++j) g[j] = to16<E>(R[y][j]);
@@ -575,22 +585,92 @@ __global__ __launch_bounds__(64 * GdnLevelSmem<KD>::NW, KD <= 128 ? 2 : 1) void 
       for (int x = 0; x < ZR; ++x) z[x][y] = mfma16<E>(f.hf[x], g, z[x][y]);
     }
   };
-  begin_block(0);
-  while (at.vb < nvb) {
+  bool again = false;
+  do {
+    Step at{0, nlev - 1};
+    if (again) ahead = fetch_first();
 #pragma unroll
-    for (int i = 0; i < PF; ++i) {
-      if (at.vb < nvb) {
-        level(fr[i], at.e);
-        fetch(fr[i], ahead);
-        ahead = after(ahead);
-        const Step nx = after(at);
-        if (nx.vb != at.vb) {
-          end_block(at.vb);
-          if (nx.vb < nvb) begin_block(nx.vb);
+    for (int x = 0; x < ZR; ++x)
+#pragma unroll
+      for (int y = 0; y < NC; ++y) z[x][y] = zero4();
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+      for (int y = 0; y < NC; ++y) adk[x][y] = zero4();
+    begin_block(0);
+    while (at.vb < nvb) {
+#pragma unroll
+      for (int i = 0; i < PF; ++i) {
+        if (at.vb < nvb) {
+          level(fr[i], at.e);
+          fetch(fr[i], ahead);
+          ahead = after(ahead);
+          const Step nx = after(at);
+          if (nx.vb != at.vb) {
+            end_block(at.vb);
+            if (nx.vb < nvb) begin_block(nx.vb);
+          }
+          at = nx;
         }
-        at = nx;
       }
     }
+    if constexpr (kHalf) {
+      // the largest of this wave's Z (NaN: an infinite operand met a zero), and whether
+      // a sum overflowed: an infinity among dK_new's accumulators or Z
+      float big = 0.f, sum = 0.f;
+#pragma unroll
+      for (int x = 0; x < ZR; ++x)
+#pragma unroll
+        for (int y = 0; y < NC; ++y)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            big = fmaxf(big, fabsf(z[x][y][i]));
+            sum += 0.f * z[x][y][i];
+          }
+#pragma unroll
+      for (int x = 0; x < 2; ++x)
+#pragma unroll
+        for (int y = 0; y < NC; ++y)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) sum += 0.f * adk[x][y][i];
+#pragma unroll
+      for (int off = 32; off >= 1; off >>= 1) {
+        big = fmaxf(big, __shfl_xor(big, off, 64));
+        sum += __shfl_xor(sum, off, 64);
+      }
+      if (lane == 0) {
+        s.red[w] = big;
+        s.bad[w] = sum == 0.f ? 0 : 1;
+      }
+      __syncthreads();
+      int bad = 0;
+      zmax = 0.f;
+#pragma unroll
+      for (int i = 0; i < NW; ++i) {
+        bad |= s.bad[i];
+        zmax = fmaxf(zmax, s.red[i]);
+      }
+      __syncthreads();
+      again = bad && !again;
+      if (again) hs1 = 0.125f;
+    }
+  } while (again);
+  float zs = 1.f;
+  if constexpr (kHalf) {
+    // Z's planes hold Z 2^k with its largest element below 2^15: Z is a sum of h dh over
+    // V, far above the 65504 of an fp16 where h and dh are not
+    int ex = 0;
+    if (zmax > 0.f && zmax < INFINITY) (void)frexpf(zmax, &ex);
+    zs = ldexpf(1.f, min(max(15 - ex, -60), 20));
+#pragma unroll
+    for (int x = 0; x < ZR; ++x)
+#pragma unroll
+      for (int y = 0; y < NC; ++y) z[x][y] *= zs;
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+      for (int y = 0; y < NC; ++y) adk[x][y] *= zs;
+    zs = 1.f / (zs * hs1);
   }
 
   // ---- d exp(Gc_last) = trace Z -------------------------------------------------------
@@ -604,7 +684,7 @@ __global__ __launch_bounds__(64 * GdnLevelSmem<KD>::NW, KD <= 128 ? 2 : 1) void 
         for (int i = 0; i < 4; ++i) tr += 4 * lq + i == ln ? z[x][y][i] : 0.f;
 #pragma unroll
   for (int off = 32; off >= 1; off >>= 1) tr += __shfl_xor(tr, off, 64);
-  if (lane == 0) s.red[w] = tr;
+  if (lane == 0) s.red[w] = tr * zs;
 
   // ---- dW_new = -K_new Z^T, dK_new -= W_new Z, 64 rows of Z at a time ------------------
   // of dW_new: token tile tw, column tiles NY kp + y of the 64
@@ -663,7 +743,7 @@ __global__ __launch_bounds__(64 * GdnLevelSmem<KD>::NW, KD <= 128 ? 2 : 1) void 
     for (int y = 0; y < NY; ++y)
 #pragma unroll
       for (int i = 0; i < 4; ++i)
-        dwn[rowk + (size_t)(16 * tw + 4 * lq + i) * hk + 64 * rb + 16 * (NY * kp + y) + ln] = (__bf16)-adw[y][i];
+        dwn[rowk + (size_t)(16 * tw + 4 * lq + i) * hk + 64 * rb + 16 * (NY * kp + y) + ln] = (__bf16)(-adw[y][i] * zs);
     __syncthreads();
   }
 #pragma unroll
@@ -672,7 +752,7 @@ __global__ __launch_bounds__(64 * GdnLevelSmem<KD>::NW, KD <= 128 ? 2 : 1) void 
     for (int y = 0; y < NC; ++y)
 #pragma unroll
       for (int i = 0; i < 4; ++i)
-        dkn[rowk + (size_t)(16 * (2 * wr + x) + 4 * lq + i) * hk + 16 * (NC * wc + y) + ln] = (__bf16)adk[x][y][i];
+        dkn[rowk + (size_t)(16 * (2 * wr + x) + 4 * lq + i) * hk + 16 * (NC * wc + y) + ln] = (__bf16)(adk[x][y][i] * zs);
   if (tid == 0) {
     float x = 0.f;
 #pragma unroll
