@@ -1308,19 +1308,22 @@ inline size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 // log2 of the chunks per segment of the backward: the forward's segments, halved as long
 // as there is at most one workgroup (a row and segment) per CU and at most 16 segments.
 // A workgroup walks its chunks one after the other, so a small problem's time is the
-// length of that walk.  Forward and backward in us, before and with the finer segments
-// (H = G, K = V = 64): 32 rows T 2048 253 -> 149, 8 rows T 4096 271 -> 171, 8 rows
-// T 8192 297 -> 230; fp32 8 rows T 1024 348 -> 178, 4 rows T 2048 532 -> 312.
+// length of that walk.  Forward and backward as called, in us, before and with the finer
+// segments (H = G, K = V = 64): 4 rows T 2048 243 -> 212, 64 rows T 1088 244 -> 217, and
+// 253 -> 149 of device time at 32 rows T 2048, where the host is the longer side.
 // Past one workgroup per CU it only adds passes (240 rows T 1024 207 -> 228), and past 16
 // segments the scan over them takes what the walk saves (8 rows T 4096 171 -> 190 at 32).
-// A 16-bit sequence of one forward segment stays whole: the finer backward would add
-// four launches to its two, and its 8 rows T 1024 take 191 -> 98 on the device but
-// 198 -> 207 called one by one from a host that needs that long for a forward and
-// backward.
-constexpr int kBwdMaxGroups = 256, kBwdMaxSeg = 16;
+// A sequence of one forward segment needs two launches whole and six in finer segments,
+// 12 to 50 us of a host: it is split where the walk takes longer than a whole training
+// call on such a host, 240 us of the walk of dq and dkv and the forward's, which is 10 us
+// a chunk in 16 bits and 20 in fp32.  So 16 bits never (8 rows T 1024: 191 -> 98 on the
+// device, 198 -> 207 as called), fp32 from 12 chunks on: 8 rows T 768 258 -> 198, T 1024
+// 349 -> 199; but T 512 194 -> 199, 4 rows T 256 189 -> 199 (200 -> 250 on a slower
+// host), and at K = V = 128, four calls, 472 -> 544.
+constexpr int kBwdMaxGroups = 256, kBwdMaxSeg = 16, kBwdMinWalk = 240;   // the last in us
 inline int bwd_seg_log2(int rows, int NT, bool fp32) {
   int s = seg_log2(NT);
-  if (!fp32 && NT <= (1 << kMaxLoc)) return s;
+  if (NT <= (1 << kMaxLoc) && (fp32 ? 20 : 10) * NT < kBwdMinWalk) return s;
   while (s > 1) {
     const int nseg = (NT + (1 << (s - 1)) - 1) >> (s - 1);
     if (nseg > kBwdMaxSeg || (long)rows * nseg > kBwdMaxGroups) break;

@@ -150,11 +150,12 @@ def test_forward_summaries_reused(T):
 # The backward's segments against one workgroup per CU (256) and 16 segments:
 # (2048, 1): 16 segments, the most; (2112, 1): one chunk more, so 4-chunk segments;
 # (1088, 85): 255 workgroups with 8-chunk segments, the last of one chunk; (1088, 86):
-# 258, so the forward's segments and its summaries; fp32 (704, 1): 2-chunk segments in
-# a sequence of one forward segment.
+# 258, so the forward's segments and its summaries; fp32 (704, 1): one segment of 11
+# chunks, whole; (768, 1): 2-chunk segments in a sequence of one forward segment.
 @pytest.mark.parametrize("T,H,dtype", [(2048, 1, torch.bfloat16), (2112, 1, torch.bfloat16),
                                        (1088, 85, torch.bfloat16), (1088, 86, torch.bfloat16),
-                                       (704, 1, torch.float32), (2048, 1, torch.float32)])
+                                       (704, 1, torch.float32), (768, 1, torch.float32),
+                                       (2048, 1, torch.float32)])
 def test_backward_segments(T, H, dtype):
     L = 7 + math.ceil(math.log2(T // 64))
     if dtype == torch.float32:
