@@ -272,8 +272,8 @@ size_t hattn_gdn_chunkwise_fwd_workspace(int B, int T, int H, int K, int V, int 
 
 /*
  * hattn_gdn_chunkwise_fwd that also leaves, in its workspace, what the
- * backward's recompute would produce: q_new, W_new, K_new, U and every level's
- * state at every chunk start (bf16), the same values bit for bit.  No
+ * backward's recompute would produce: q_new, W_new, K_new, U and the states of the
+ * levels set in each chunk's index at its start (16-bit), the same values bit for bit.  No
  * counterpart in the reference (its backward recomputes them,
  * chunkwise_hgdn.py:860-893); for callers that keep the forward's workspace
  * until the backward, as HAttentionFunction does between its forward and
@@ -291,8 +291,8 @@ int hattn_gdn_chunkwise_fwd_keep(const void* q, const void* k, const void* v, co
                                  void* stream);
 
 /* Workspace bytes of hattn_gdn_chunkwise_fwd_keep (the forward's, plus the
- * token-major k_new and the per-chunk level states).  No counterpart in the
- * reference. */
+ * token-major k_new and room for every level's state of every chunk).  No
+ * counterpart in the reference. */
 size_t hattn_gdn_chunkwise_fwd_keep_workspace(int B, int T, int H, int K, int V, int L);
 
 /*
@@ -339,9 +339,9 @@ int hattn_gdn_chunkwise_bwd(const void* q, const void* k, const void* v, const v
 
 /* Workspace bytes of hattn_gdn_chunkwise_bwd: the recomputed q_new, k_new (token-major
  * and per-chunk transposed), w_new, u (bf16), the states of
- * the levels set in each chunk's index at its start (16-bit), the reverse states of the
- * other levels, and the level sums (dq_new, dw_new, dk_new, dU).  No counterpart in the
- * reference, which allocates h / dh and its temporaries with torch inside
+ * the levels set in each chunk's index at its start (16-bit), the reverse states of every
+ * level after every chunk (16-bit), and the level sums (dq_new, dw_new, dk_new in bf16,
+ * dU in fp32).  No counterpart in the reference, which allocates h / dh and its temporaries with torch inside
  * chunkwise_bwd (chunkwise_hgdn.py:894-913). */
 size_t hattn_gdn_chunkwise_bwd_workspace(int B, int T, int H, int K, int V, int L);
 
@@ -352,8 +352,8 @@ size_t hattn_gdn_chunkwise_bwd_workspace(int B, int T, int H, int K, int V, int 
  * K, V, L, l2norm_qk and qk_scale, unchanged since.  No counterpart in the
  * reference (see hattn_gdn_chunkwise_fwd_keep).  Same arguments, results and
  * status codes as hattn_gdn_chunkwise_bwd, with workspace >=
- * hattn_gdn_chunkwise_bwd_fwd_ws_workspace(...) bytes (the level scan's
- * partial gradients only), plus fwd_workspace null or fwd_workspace_bytes
+ * hattn_gdn_chunkwise_bwd_fwd_ws_workspace(...) bytes (the reverse states and the
+ * level sums only), plus fwd_workspace null or fwd_workspace_bytes
  * below hattn_gdn_chunkwise_fwd_keep_workspace(...) -> HATTN_ERR_VALUE.  The
  * results equal hattn_gdn_chunkwise_bwd's bit for bit; a workspace of another
  * call gives wrong gradients.
@@ -368,8 +368,8 @@ int hattn_gdn_chunkwise_bwd_fwd_ws(const void* q, const void* k, const void* v, 
                                    size_t workspace_bytes, const void* fwd_workspace,
                                    size_t fwd_workspace_bytes, void* stream);
 
-/* Workspace bytes of hattn_gdn_chunkwise_bwd_fwd_ws: the level scan's partial
- * gradients (no recompute regions).  No counterpart in the reference. */
+/* Workspace bytes of hattn_gdn_chunkwise_bwd_fwd_ws: the reverse states and the level
+ * sums (no recompute regions).  No counterpart in the reference. */
 size_t hattn_gdn_chunkwise_bwd_fwd_ws_workspace(int B, int T, int H, int K, int V, int L);
 
 /*
@@ -377,7 +377,9 @@ size_t hattn_gdn_chunkwise_bwd_fwd_ws_workspace(int B, int T, int H, int K, int 
  * (the level sums and the chunk-local products run over all of V).  With
  * fwd_workspace (from the keeping forward on the same inputs) the backward takes
  * q_new, W_new, K_new, U and the level states from it, with NULL it recomputes them.
- * Workspaces: hattn_gdn_chunkwise_fwd_keep_workspace;
+ * Workspaces: hattn_gdn_chunkwise_fwd_keep_any_v_workspace (the states that a chunk
+ * reads, those of the levels set in its index: about half of the room that
+ * hattn_gdn_chunkwise_fwd_keep_workspace counts, which is enough as well);
  * hattn_gdn_chunkwise_bwd_fwd_ws_workspace with a forward workspace, else
  * hattn_gdn_chunkwise_bwd_workspace.  No counterpart in the reference.
  */
@@ -388,6 +390,7 @@ int hattn_gdn_chunkwise_fwd_keep_any_v(const void* q, const void* k, const void*
                                        int dtype_beta, int dtype_l, int dtype_o, int level_base,
                                        int htype, int chunk_size, int l2norm_qk, float qk_scale,
                                        void* workspace, size_t workspace_bytes, void* stream);
+size_t hattn_gdn_chunkwise_fwd_keep_any_v_workspace(int B, int T, int H, int K, int V, int L);
 int hattn_gdn_chunkwise_bwd_any_v(const void* q, const void* k, const void* v, const void* beta,
                                   const float* g_cumsum, const void* l, const void* do_, void* dq,
                                   void* dk, void* dv, void* db, float* dg, float* dl, int B, int T,

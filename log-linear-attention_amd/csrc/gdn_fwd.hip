@@ -746,16 +746,14 @@ struct GdnKeepWs {
   size_t bytes;
 };
 
-inline GdnKeepWs gdn_keep_ws_layout(void* base, int B, int T, int H, int K, int V, int nlev) {
+inline GdnKeepWs gdn_keep_ws_layout(void* base, int B, int T, int H, int K, int V) {
   GdnKeepWs w;
   w.f = gdn_ws_layout(base, B, T, H, K, V);
   char* p = (char*)base;
   size_t off = w.f.bytes;
   const size_t n = (size_t)B * T * H, NT = (size_t)T / kGC;
   w.kn = (__bf16*)(p + off); off += galign(n * K * 2);
-  // sized for every level of every chunk, as callers of the query may count on; the set
-  // levels' states take the first half or so
-  w.hs = (__bf16*)(p + off); off += galign((size_t)B * H * NT * nlev * V * K * 2);
+  w.hs = (__bf16*)(p + off); off += galign((size_t)B * H * gdn_set_before((int)NT) * V * K * 2);
   w.bytes = off;
   return w;
 }
@@ -837,7 +835,7 @@ static hipError_t gdn_launch_keep_t(const void* q, const void* k, const void* v,
                                     const float* g, const void* l, void* o, float* gcum, void* aw,
                                     void* au, float* ht, void* ws, int B, int T, int H, int V,
                                     int L, int nlev, int norm_qk, float scale, hipStream_t stream) {
-  const GdnKeepWs w = gdn_keep_ws_layout(ws, B, T, H, KD, V, nlev);
+  const GdnKeepWs w = gdn_keep_ws_layout(ws, B, T, H, KD, V);
   hipError_t e = gdn_prep_launch_t<KD, TB, TL, kPrepFwdKeep, STRONG, E>(
       q, k, v, beta, g, l, gcum, aw, au, w.f.qn, w.f.wn, w.kn, w.f.knT, w.f.un, w.f.pm, B, T, H,
       V, L, norm_qk, scale, stream);
@@ -848,14 +846,21 @@ static hipError_t gdn_launch_keep_t(const void* q, const void* k, const void* v,
 
 }  // namespace hattn
 
-size_t hattn_gdn_fwd_keep_ws_bytes(int B, int T, int H, int K, int V, int nlev) {
-  return hattn::gdn_keep_ws_layout(nullptr, B, T, H, K, V, nlev).bytes;
+size_t hattn_gdn_fwd_keep_ws_bytes(int B, int T, int H, int K, int V) {
+  return hattn::gdn_keep_ws_layout(nullptr, B, T, H, K, V).bytes;
 }
 
-void hattn_gdn_fwd_keep_buffers(const void* ws, int B, int T, int H, int K, int V, int nlev,
+// The bytes by which a workspace with room for every level's state of every chunk is larger.
+size_t hattn_gdn_fwd_keep_ws_spare(int B, int T, int H, int K, int V, int nlev) {
+  const size_t NT = (size_t)T / hattn::kGC, set = hattn::gdn_set_before((int)NT);
+  const size_t state = (size_t)V * K * 2, rows = (size_t)B * H;
+  return hattn::galign(rows * NT * nlev * state) - hattn::galign(rows * set * state);
+}
+
+void hattn_gdn_fwd_keep_buffers(const void* ws, int B, int T, int H, int K, int V,
                                 const __bf16** qn, const __bf16** wn, const __bf16** kn,
                                 const __bf16** un, const __bf16** hs) {
-  const hattn::GdnKeepWs w = hattn::gdn_keep_ws_layout(const_cast<void*>(ws), B, T, H, K, V, nlev);
+  const hattn::GdnKeepWs w = hattn::gdn_keep_ws_layout(const_cast<void*>(ws), B, T, H, K, V);
   *qn = w.f.qn;
   *wn = w.f.wn;
   *kn = w.kn;

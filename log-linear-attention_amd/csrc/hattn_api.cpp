@@ -57,14 +57,15 @@ hipError_t hattn_gdn_fwd_launch(const void* q, const void* k, const void* v, con
                                 int L, int nlev, int dt_b, int dt_l, int dt_o, int norm_qk,
                                 float scale, int strong, int h16, hipStream_t stream,
                                 int* unsupported);
-size_t hattn_gdn_fwd_keep_ws_bytes(int B, int T, int H, int K, int V, int nlev);
+size_t hattn_gdn_fwd_keep_ws_bytes(int B, int T, int H, int K, int V);
+size_t hattn_gdn_fwd_keep_ws_spare(int B, int T, int H, int K, int V, int nlev);
 hipError_t hattn_gdn_fwd_keep_launch(const void* q, const void* k, const void* v,
                                      const void* beta, const float* g, const void* l, void* o,
                                      float* gcum, void* aw, void* au, float* ht, void* ws, int B,
                                      int T, int H, int K, int V, int L, int nlev, int dt_b,
                                      int dt_l, int dt_o, int norm_qk, float scale, int strong,
                                      int h16, hipStream_t stream, int* unsupported);
-void hattn_gdn_fwd_keep_buffers(const void* ws, int B, int T, int H, int K, int V, int nlev,
+void hattn_gdn_fwd_keep_buffers(const void* ws, int B, int T, int H, int K, int V,
                                 const __bf16** qn, const __bf16** wn, const __bf16** kn,
                                 const __bf16** un, const __bf16** hs);
 size_t hattn_gdn_bwd_kept_ws_bytes(int B, int T, int H, int K, int V, int nlev);
@@ -521,6 +522,14 @@ size_t hattn_gdn_chunkwise_fwd_workspace(int B, int T, int H, int K, int V, int 
   return hattn_gdn_fwd_ws_bytes(B, T, H, K, V);
 }
 
+// A keeping forward's workspace.  The entry points for V in {64, 128} ask for room for
+// every level's state of every chunk, which their callers may count on; the kernels store
+// the states that a chunk reads, about half of them.
+static size_t gdn_keep_bytes(int B, int T, int H, int K, int V, int nlev, bool any_v) {
+  return hattn_gdn_fwd_keep_ws_bytes(B, T, H, K, V) +
+         (any_v ? 0 : hattn_gdn_fwd_keep_ws_spare(B, T, H, K, V, nlev));
+}
+
 // keep: also leave, in the workspace, what the backward's recompute would
 // produce (hattn_gdn_chunkwise_fwd_keep)
 static int gdn_fwd_impl(const void* q, const void* k, const void* v, const void* beta,
@@ -528,7 +537,8 @@ static int gdn_fwd_impl(const void* q, const void* k, const void* v, const void*
                         void* Au, float* ht, int B, int T, int H, int K, int V, int L,
                         int dtype_qkv, int dtype_beta, int dtype_l, int dtype_o, int level_base,
                         int htype, int chunk_size, int l2norm_qk, float qk_scale,
-                        void* workspace, size_t workspace_bytes, bool keep, void* stream, bool any_v = false) {
+                        void* workspace, size_t workspace_bytes, bool keep, void* stream,
+                        bool any_v = false) {
   if (chunk_size != 64)
     return fail(HATTN_ERR_NOT_IMPLEMENTED, "chunk_size=%d (only 64 is supported)", chunk_size);
   if (level_base != 2)
@@ -565,7 +575,7 @@ static int gdn_fwd_impl(const void* q, const void* k, const void* v, const void*
                 hattn_gdn_bwd_max_levels());
   if (!q || !k || !v || !beta || !g || !l || !o || !g_cumsum || !Aw || !Au)
     return fail(HATTN_ERR_VALUE, "null tensor pointer");
-  const size_t need = keep ? hattn_gdn_fwd_keep_ws_bytes(B, T, H, K, V, nlev)
+  const size_t need = keep ? gdn_keep_bytes(B, T, H, K, V, nlev, any_v)
                            : hattn_gdn_fwd_ws_bytes(B, T, H, K, V);
   if (workspace_bytes < need || workspace == nullptr)
     return fail(HATTN_ERR_VALUE, "workspace of %zu bytes is smaller than the %zu required",
@@ -613,7 +623,13 @@ int hattn_gdn_chunkwise_fwd_keep_any_v(const void* q, const void* k, const void*
 size_t hattn_gdn_chunkwise_fwd_keep_workspace(int B, int T, int H, int K, int V, int L) {
   (void)L;
   if (B <= 0 || T < 64 || T % 64 != 0 || H <= 0 || K <= 0 || V <= 0) return 0;
-  return hattn_gdn_fwd_keep_ws_bytes(B, T, H, K, V, ceil_log2(T / 64));
+  return gdn_keep_bytes(B, T, H, K, V, ceil_log2(T / 64), false);
+}
+
+size_t hattn_gdn_chunkwise_fwd_keep_any_v_workspace(int B, int T, int H, int K, int V, int L) {
+  (void)L;
+  if (B <= 0 || T < 64 || T % 64 != 0 || H <= 0 || K <= 0 || V <= 0) return 0;
+  return gdn_keep_bytes(B, T, H, K, V, ceil_log2(T / 64), true);
 }
 
 int hattn_gdn_chunkwise_fwd_keep(const void* q, const void* k, const void* v, const void* beta,
@@ -674,7 +690,7 @@ static int gdn_bwd_impl(const void* q, const void* k, const void* v, const void*
   if (!q || !k || !v || !beta || !g_cumsum || !l || !do_ || !dq || !dk || !dv || !db || !dg || !dl)
     return fail(HATTN_ERR_VALUE, "null tensor pointer");
   if (kept) {
-    const size_t fneed = hattn_gdn_fwd_keep_ws_bytes(B, T, H, K, V, nlev);
+    const size_t fneed = gdn_keep_bytes(B, T, H, K, V, nlev, any_v);
     if (fwd_ws == nullptr || fwd_ws_bytes < fneed)
       return fail(HATTN_ERR_VALUE,
                   "forward workspace of %zu bytes is smaller than the %zu of the keeping forward",
@@ -689,7 +705,7 @@ static int gdn_bwd_impl(const void* q, const void* k, const void* v, const void*
   hipError_t e;
   if (kept) {
     const __bf16 *qn, *wn, *kn, *un, *hs;
-    hattn_gdn_fwd_keep_buffers(fwd_ws, B, T, H, K, V, nlev, &qn, &wn, &kn, &un, &hs);
+    hattn_gdn_fwd_keep_buffers(fwd_ws, B, T, H, K, V, &qn, &wn, &kn, &un, &hs);
     e = hattn_gdn_bwd_kept_launch(q, k, v, beta, g_cumsum, l, do_, dq, dk, dv, db, dg, dl, qn, wn,
                                   kn, un, hs, workspace, B, T, H, K, V, L, nlev, dtype_beta,
                                   dtype_l, l2norm_qk ? 1 : 0, qk_scale,

@@ -55,6 +55,7 @@ SIGNATURES = [
     ("hattn_gdn_chunkwise_fwd_keep_any_v", _I,
      [_P, _P, _P, _P, _F, _P, _P, _F, _P, _P, _F] + [_I] * 6 + [_I] * 4 + [_I] * 3
      + [_I, ctypes.c_float] + [_P, _S, _P]),
+    ("hattn_gdn_chunkwise_fwd_keep_any_v_workspace", _S, [_I] * 6),
     ("hattn_gdn_chunkwise_bwd_any_v", _I,
      [_P, _P, _P, _P, _F, _P, _P, _P, _P, _P, _P, _F, _F] + [_I] * 6 + [_I] * 4
      + [_I] * 3 + [_I, ctypes.c_float] + [_P, _S, _P, _S, _P]),

@@ -158,7 +158,7 @@ def chunkwise_fwd_keep(
     lib = _lib.load()
     keep = keep and (keep_any_v or V in (64, VB))
     ws, ws_ptr, ws_bytes = _lib.workspace(
-        (lib.hattn_gdn_chunkwise_fwd_keep_workspace if keep
+        (lib.hattn_gdn_chunkwise_fwd_keep_any_v_workspace if keep
          else lib.hattn_gdn_chunkwise_fwd_workspace)(B, T, H, K, V, L), dev)
     st = (lib.hattn_gdn_chunkwise_fwd_keep_any_v if keep else lib.hattn_gdn_chunkwise_fwd)(
         _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.ptr(b), _lib.ptr(g), _lib.ptr(l),

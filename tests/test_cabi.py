@@ -368,3 +368,27 @@ def test_status_query_checks():
                                                  None) == _lib.HATTN_ERR_VALUE
     assert lib.hattn_mamba2_chunkwise_fwd_status(None, 1, 100, 1, 64, ctypes.byref(out),
                                                  None) == _lib.HATTN_ERR_VALUE
+
+
+@pytest.mark.parametrize("T", [64, 128, 192, 2048, 16384])
+def test_gdn_keep_any_v_workspace_holds_the_read_states(T):
+    """What the keeping forward for any V holds beyond the forward: the token-major K_new
+    and one state per set bit of each chunk's index, no more; the backward takes a forward
+    workspace of that size and refuses a smaller one."""
+    lib = _lib.load()
+    B, H, K, V, L = 2, 4, 128, 192, 15
+    pad = lambda x: (x + 255) // 256 * 256
+    states = sum(bin(c).count("1") for c in range(T // 64))
+    need = lib.hattn_gdn_chunkwise_fwd_keep_any_v_workspace(B, T, H, K, V, L)
+    assert need == lib.hattn_gdn_chunkwise_fwd_workspace(B, T, H, K, V, L) + \
+        pad(B * T * H * K * 2) + pad(B * H * states * V * K * 2)
+    assert lib.hattn_gdn_chunkwise_fwd_keep_workspace(B, T, H, K, V, L) >= need
+    assert lib.hattn_gdn_chunkwise_fwd_keep_any_v_workspace(B, 100, H, K, V, L) == 0
+    x = ctypes.c_void_p(0x1000)
+    st = lib.hattn_gdn_chunkwise_bwd_any_v(x, x, x, x, x, x, x, x, x, x, x, x, x, B, T, H, K, V, L,
+                                           0, 0, 0, 0, 2, 0, 64, 0, 1.0, x, 0, x, need - 1, None)
+    assert st == _lib.HATTN_ERR_VALUE and str(need) in lib.hattn_last_error().decode()
+    st = lib.hattn_gdn_chunkwise_bwd_any_v(x, x, x, x, x, x, x, x, x, x, x, x, x, B, T, H, K, V, L,
+                                           0, 0, 0, 0, 2, 0, 64, 0, 1.0, x, 0, x, need, None)
+    assert st == _lib.HATTN_ERR_VALUE   # the backward's own workspace
+    assert "forward workspace" not in lib.hattn_last_error().decode()
