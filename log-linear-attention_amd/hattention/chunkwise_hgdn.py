@@ -33,6 +33,33 @@ from hattention.base import HType, get_num_levels, ceil_log
 
 CHUNK = 64
 VB = 128   # V columns that chunkwise_fwd_keep keeps a workspace for by itself
+# A backward over all of V at once holds the level states and their gradients of all its
+# columns: B 8, T 8192, H 16, K 256, V 512 would take 52 GB at a time, 13 GB in blocks of
+# 128 columns.  More than BWD_LIMIT bytes are taken in blocks (at K 192, V 384, T 16384, H 6,
+# 3.2 GB: 6.1 ms at once, 38.7 in blocks of 128).
+BWD_LIMIT = 4 << 30
+# What one training call may hold between its forward and backward where V is neither 64
+# nor 128 (KEPT_V, for which it always holds its workspace: 1.7 GB at B 4, T 8192, H 16,
+# K = V = 128).  Above it the backward computes it again.
+KEEP_LIMIT = 2 << 30
+KEPT_V = (64, VB)
+
+
+def bwd_columns(B, T, H, K, V, L):
+    """V columns per call of the backward's kernels without a forward workspace: V, or the
+    most blocks of VB whose workspace fits BWD_LIMIT, at least one."""
+    lib = _lib.load()
+    n = V
+    while n > VB and lib.hattn_gdn_chunkwise_bwd_workspace(B, T, H, K, n, L) > BWD_LIMIT:
+        n = (n - 1) // VB * VB
+    return n
+
+
+def keeps_workspace(B, T, H, K, V, L):
+    """Whether a training call with V not in KEPT_V holds its forward's workspace for
+    the backward."""
+    need = _lib.load().hattn_gdn_chunkwise_fwd_keep_any_v_workspace(B, T, H, K, V, L)
+    return need <= KEEP_LIMIT and bwd_columns(B, T, H, K, V, L) == V
 
 
 def _validate(q, k, v, l, head_first, level_base, htype, chunk_size, **tensors):
@@ -132,14 +159,15 @@ def chunkwise_fwd_keep(
     qk_l2norm_scale: Optional[float] = None,
     keep: bool = True,
     keep_any_v: bool = False,
+    keep_if_fits: bool = False,
 ):
     """:func:`chunkwise_fwd` that also returns the forward's workspace, holding
     what the backward would recompute (q_new, W_new, K_new, U and every level's
     state that a chunk reads, bit for bit), for V in {64, 128} or, with
-    ``keep_any_v``, any V (else None): pass it to :func:`chunkwise_bwd` as
-    ``fwd_ws`` with the same inputs, and the backward skips its recompute
-    (HAttentionFunction keeps it between its forward and backward).  Returns
-    (g_cumsum, o, Aw, Au, ht, fwd_ws)."""
+    ``keep_any_v``, any V, with ``keep_if_fits`` any V within KEEP_LIMIT (else
+    None): pass it to :func:`chunkwise_bwd` as ``fwd_ws`` with the same inputs,
+    and the backward skips its recompute (HAttentionFunction keeps it between
+    its forward and backward).  Returns (g_cumsum, o, Aw, Au, ht, fwd_ws)."""
     B, T, G, H, K, V, L = _validate(q, k, v, l, head_first, level_base, htype, chunk_size,
                                     b=b, g=g)
     if g.dtype != torch.float32:
@@ -156,7 +184,8 @@ def chunkwise_fwd_keep(
     Au = torch.empty(B, T, H, CHUNK, dtype=k.dtype, device=dev)
     ht = torch.zeros(B, H, K, V, L, dtype=torch.float32, device=dev) if output_final_state else None
     lib = _lib.load()
-    keep = keep and (keep_any_v or V in (64, VB))
+    keep = keep and (keep_any_v or V in KEPT_V or
+                     (keep_if_fits and keeps_workspace(B, T, H, K, V, L)))
     ws, ws_ptr, ws_bytes = _lib.workspace(
         (lib.hattn_gdn_chunkwise_fwd_keep_any_v_workspace if keep
          else lib.hattn_gdn_chunkwise_fwd_workspace)(B, T, H, K, V, L), dev)
@@ -222,25 +251,44 @@ def chunkwise_bwd(
         k = k.repeat_interleave(H // G, dim=2).contiguous()
     do = do.to(v.dtype).contiguous()
     lib = _lib.load()
-    dq = torch.empty(B, T, H, K, dtype=q.dtype, device=dev)
-    dk = torch.empty(B, T, H, K, dtype=k.dtype, device=dev)
-    dv = torch.empty_like(v)
-    db = torch.empty_like(b)
-    dg = torch.empty(B, T, H, dtype=torch.float32, device=dev)
-    dl = torch.empty(B, T, H, L, dtype=torch.float32, device=dev)
-    ws, ws_ptr, ws_bytes = _lib.workspace(
-        (lib.hattn_gdn_chunkwise_bwd_fwd_ws_workspace if fwd_ws is not None
-         else lib.hattn_gdn_chunkwise_bwd_workspace)(B, T, H, K, V, L), dev)
-    _lib.check(lib.hattn_gdn_chunkwise_bwd_any_v(
-        _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.ptr(b), _lib.ptr(g), _lib.ptr(l),
-        _lib.ptr(do), _lib.ptr(dq), _lib.ptr(dk), _lib.ptr(dv), _lib.ptr(db), _lib.ptr(dg),
-        _lib.ptr(dl), B, T, H, K, V, L, _lib.dtype_code(q), _lib.dtype_code(b),
-        _lib.dtype_code(l), _lib.dtype_code(do), level_base, htype.value, chunk_size,
-        1 if qk_l2norm_scale is not None else 0,
-        float(qk_l2norm_scale) if qk_l2norm_scale is not None else 1.0, ws_ptr, ws_bytes,
-        _lib.ptr(fwd_ws), fwd_ws.numel() if fwd_ws is not None else 0,
-        _lib.stream_handle(dev)))
-    del ws
+
+    def call(v, do, fwd_ws):
+        V = v.shape[3]
+        dq = torch.empty(B, T, H, K, dtype=q.dtype, device=dev)
+        dk = torch.empty(B, T, H, K, dtype=k.dtype, device=dev)
+        dv = torch.empty_like(v)
+        db = torch.empty_like(b)
+        dg = torch.empty(B, T, H, dtype=torch.float32, device=dev)
+        dl = torch.empty(B, T, H, L, dtype=torch.float32, device=dev)
+        ws, ws_ptr, ws_bytes = _lib.workspace(
+            (lib.hattn_gdn_chunkwise_bwd_fwd_ws_workspace if fwd_ws is not None
+             else lib.hattn_gdn_chunkwise_bwd_workspace)(B, T, H, K, V, L), dev)
+        _lib.check(lib.hattn_gdn_chunkwise_bwd_any_v(
+            _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.ptr(b), _lib.ptr(g), _lib.ptr(l),
+            _lib.ptr(do), _lib.ptr(dq), _lib.ptr(dk), _lib.ptr(dv), _lib.ptr(db), _lib.ptr(dg),
+            _lib.ptr(dl), B, T, H, K, V, L, _lib.dtype_code(q), _lib.dtype_code(b),
+            _lib.dtype_code(l), _lib.dtype_code(do), level_base, htype.value, chunk_size,
+            1 if qk_l2norm_scale is not None else 0,
+            float(qk_l2norm_scale) if qk_l2norm_scale is not None else 1.0, ws_ptr, ws_bytes,
+            _lib.ptr(fwd_ws), fwd_ws.numel() if fwd_ws is not None else 0,
+            _lib.stream_handle(dev)))
+        return dq, dk, dv, db, dg, dl
+
+    cols = V if fwd_ws is not None else bwd_columns(B, T, H, K, V, L)
+    if cols == V:
+        dq, dk, dv, db, dg, dl = call(v, do, fwd_ws)
+    else:
+        # each column of o depends on its column of v only: the gradients of the other
+        # inputs are sums over blocks of columns, taken in fp32
+        dv, acc = torch.empty_like(v), None
+        for v0 in range(0, V, cols):
+            c = slice(v0, min(v0 + cols, V))
+            r = call(v[..., c].contiguous(), do[..., c].contiguous(), None)
+            dv[..., c] = r[2]
+            r = [x.float() for x in r[:2] + r[3:]]
+            acc = r if acc is None else [x.add_(y) for x, y in zip(acc, r)]
+        dq, dk, db = acc[0].to(q.dtype), acc[1].to(k.dtype), acc[2].to(b.dtype)
+        dg, dl = acc[3:]
     if G != H:
         dq = dq.view(B, T, G, H // G, K).sum(3, dtype=torch.float32).to(q.dtype)
         dk = dk.view(B, T, G, H // G, K).sum(3, dtype=torch.float32).to(k.dtype)

@@ -81,12 +81,12 @@ class HAttentionFunction(torch.autograd.Function):
             # q * scale / ||q|| and k / ||k|| are formed inside the kernels; the
             # forward's workspace (what the backward would recompute) is kept where a
             # backward can follow: storing it took 1099 us instead of 898 without it at
-            # B 4, T 8192, H 16, K = V = 128, and 1636 instead of 1301 (2.2 GB instead of
-            # 0.3) at B 1, T 16384, H 6, K 192, V 384
+            # B 4, T 8192, H 16, K = V = 128, and 1636 instead of 1301 (1.1 GB instead of
+            # 0.2) at B 1, T 16384, H 6, K 192, V 384
             g, o, Aw, Au, _, ctx.fwd_ws = _hg.chunkwise_fwd_keep(
                 q=q, k=k, v=v, b=b, g=g, l=l, head_first=head_first, level_base=level_base,
                 htype=htype, chunk_size=chunk_sizes[0], output_final_state=False,
-                qk_l2norm_scale=scale, keep=any(ctx.needs_input_grad), keep_any_v=True)
+                qk_l2norm_scale=scale, keep=any(ctx.needs_input_grad), keep_if_fits=True)
         else:
             # MAMBA2 with chunkwise=False is the reference's parallel.py path.
             raise NotImplementedError("only the chunkwise path is implemented on MI355X")

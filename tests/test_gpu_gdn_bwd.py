@@ -251,6 +251,62 @@ def test_reverse_scan_four_and_eight_waves(T, H, K, V):
          rows=[(0, 0), (0, H - 1)])
 
 
+@pytest.mark.parametrize("G,K,V,cols", [(2, 64, 192, 128), (1, 128, 384, 256), (2, 192, 320, 128)])
+def test_backward_in_blocks_of_columns(G, K, V, cols, monkeypatch):
+    """A backward whose workspace is above BWD_LIMIT goes by blocks of V columns: the same
+    dv, the other gradients as sums over the blocks (each rounded to bf16: 2^-8 of a term,
+    5e-3), the forward keeps nothing, and less memory is taken."""
+    from hattention import _lib, chunkwise_hgdn as hg
+    from hattention.base import HStruct, HType
+    from hattention.kernel import hattention_kernel
+    B, T, H, L = 2, 1024, 2, 11
+    query = _lib.load().hattn_gdn_chunkwise_bwd_workspace
+    xs = [x.cuda() for x in make_gdn_inputs(B, T, H, K, V, L, seed=V)]
+    xs[:2] = [x[:, :, :G].contiguous() for x in xs[:2]]
+    do = torch.randn(B, T, H, V, generator=torch.Generator().manual_seed(2)).bfloat16().cuda()
+    print(f"[gdn columns] G={G} K={K} V={V} cols={cols}", flush=True)
+    res = []
+    for limit in (hg.BWD_LIMIT, query(B, T, H, K, cols, L)):
+        monkeypatch.setattr(hg, "BWD_LIMIT", limit)
+        leaves = [x.clone().requires_grad_() for x in xs]
+        base = torch.cuda.memory_allocated()
+        o = hattention_kernel(*leaves, 0.125, False, 2, HType.WEAK, HStruct.GDELTA,
+                              use_qk_l2norm_in_kernel=True)
+        held = torch.cuda.memory_allocated() - base
+        torch.cuda.reset_peak_memory_stats()
+        grads = torch.autograd.grad(o, leaves, do)
+        res.append((grads, held, torch.cuda.max_memory_allocated() - base))
+        del o, grads
+    assert hg.bwd_columns(B, T, H, K, V, L) == cols
+    assert res[1][1] < res[0][1] and res[1][2] < res[0][2]
+    for name, a, r in zip(NAMES, res[1][0], res[0][0]):
+        if name == "dv":
+            assert torch.equal(a, r)
+        err = ((a.double() - r.double()).norm() / r.double().norm()).item()
+        assert err < 5e-3, (name, err)
+
+
+def test_wide_v_keeps_no_more_than_the_limit(monkeypatch):
+    """V outside {64, 128}: the forward's workspace is held up to KEEP_LIMIT bytes, and
+    without it the gradients are the same bit for bit."""
+    from hattention import _lib, chunkwise_hgdn as hg
+    from hattention.base import HType
+    B, T, H, K, V, L = 1, 640, 2, 64, 192, 11
+    need = _lib.load().hattn_gdn_chunkwise_fwd_keep_any_v_workspace(B, T, H, K, V, L)
+    xs = [x.cuda() for x in make_gdn_inputs(B, T, H, K, V, L, seed=3)]
+    do = torch.randn(B, T, H, V, generator=torch.Generator().manual_seed(4)).bfloat16().cuda()
+    res = []
+    for limit in (need, need - 1):
+        monkeypatch.setattr(hg, "KEEP_LIMIT", limit)
+        gc, _, Aw, Au, _, ws = hg.chunkwise_fwd_keep(*xs, False, 2, HType.WEAK, 64, False,
+                                                     keep_if_fits=True)
+        assert (ws is not None) == (limit == need)
+        res.append(hg.chunkwise_bwd(*xs[:4], gc, xs[5], Aw, Au, do, False, 2, HType.WEAK, 64,
+                                    fwd_ws=ws))
+    for a, r in zip(*res):
+        assert torch.equal(a, r)
+
+
 @pytest.mark.parametrize("V", [64, 192])
 def test_forward_keeps_nothing_without_gradients(V, monkeypatch):
     """Inputs without gradients: the forward keeps no workspace and gives the same bits
