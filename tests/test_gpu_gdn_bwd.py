@@ -330,3 +330,29 @@ def test_forward_keeps_nothing_without_gradients(V, monkeypatch):
     og = call(xs[2].clone().requires_grad_())
     assert kept == [False, True] and torch.equal(o, og.detach())
     assert og.grad_fn is not None
+
+
+@pytest.mark.parametrize("mode", [torch.no_grad, torch.inference_mode])
+@pytest.mark.parametrize("V", [64, 192])
+def test_forward_keeps_nothing_without_grad_mode(V, mode, monkeypatch):
+    """Inputs that require gradients (a model's parameters) under no_grad: nothing is kept
+    either, and the output has the same bits and no graph."""
+    from hattention import chunkwise_hgdn as hg
+    from hattention.base import HStruct, HType
+    from hattention.kernel import hattention_kernel
+    kept, real = [], hg.chunkwise_fwd_keep
+
+    def record(*a, **kw):
+        res = real(*a, **kw)
+        kept.append(res[5] is not None)
+        return res
+    monkeypatch.setattr(hg, "chunkwise_fwd_keep", record)
+    xs = [x.cuda().requires_grad_() for x in make_gdn_inputs(1, 256, 2, 64, V, 9, seed=V)]
+    print(f"[gdn keep] V={V} {mode.__name__}", flush=True)
+    call = lambda: hattention_kernel(*xs, 0.125, False, 2, HType.WEAK, HStruct.GDELTA,
+                                     use_qk_l2norm_in_kernel=True)
+    with mode():
+        o = call()
+    og = call()
+    assert kept == [False, True] and not o.requires_grad
+    assert torch.equal(o, og.detach())
