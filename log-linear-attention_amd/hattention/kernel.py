@@ -1,9 +1,9 @@
 """Autograd boundary of the chunkwise path (MI355X).
 
 Mirrors hattention/kernel.py:32-374: ``HAttentionFunction`` (same forward
-arguments, same saved tensors ``(q, k, v, b, g_cumsum, l, Aw, Au)``, same
-return ``o.to(q.dtype)``, backward returning grads cast to the input dtypes
-plus eight ``None``) and ``hattention_kernel`` (same signature and defaults).
+arguments, same saved tensors ``(q, k, v, b, g_cumsum, l, Aw, Au)`` and after
+them the GDELTA forward's workspace, same return ``o.to(q.dtype)``, backward
+returning grads cast to the input dtypes plus eight ``None``) and ``hattention_kernel`` (same signature and defaults).
 
 Dispatch (kernel.py:55-123):
 * MAMBA2 + chunkwise  -> ``chunkwise.chunkwise_fwd / chunkwise_bwd`` (HIP).
@@ -68,6 +68,7 @@ class HAttentionFunction(torch.autograd.Function):
                 q, k, v, g, l, head_first, level_base, htype, chunk_sizes[0], False)
             Aw = None
             Au = None
+            kept = None
         elif hstruct == HStruct.GDELTA and chunkwise:
             if b is None:
                 raise ValueError
@@ -83,7 +84,7 @@ class HAttentionFunction(torch.autograd.Function):
             # backward can follow: storing it took 1099 us instead of 898 without it at
             # B 4, T 8192, H 16, K = V = 128, and 1636 instead of 1301 (1.1 GB instead of
             # 0.2) at B 1, T 16384, H 6, K 192, V 384
-            g, o, Aw, Au, _, ctx.fwd_ws = _hg.chunkwise_fwd_keep(
+            g, o, Aw, Au, _, kept = _hg.chunkwise_fwd_keep(
                 q=q, k=k, v=v, b=b, g=g, l=l, head_first=head_first, level_base=level_base,
                 htype=htype, chunk_size=chunk_sizes[0], output_final_state=False,
                 qk_l2norm_scale=scale, keep=any(ctx.needs_input_grad), keep_if_fits=True)
@@ -91,7 +92,7 @@ class HAttentionFunction(torch.autograd.Function):
             # MAMBA2 with chunkwise=False is the reference's parallel.py path.
             raise NotImplementedError("only the chunkwise path is implemented on MI355X")
 
-        ctx.save_for_backward(q, k, v, b, g, l, Aw, Au)
+        ctx.save_for_backward(q, k, v, b, g, l, Aw, Au, kept)
         ctx.scale = scale
         ctx.dtype = g.dtype
         ctx.head_first = head_first
@@ -107,7 +108,7 @@ class HAttentionFunction(torch.autograd.Function):
     @input_guard
     @autocast_custom_bwd
     def backward(ctx, do):
-        q, k, v, b, g, l, Aw, Au = ctx.saved_tensors
+        q, k, v, b, g, l, Aw, Au, kept = ctx.saved_tensors
         if ctx.hstruct == HStruct.MAMBA2 and ctx.chunkwise:
             if b is not None or Aw is not None or Au is not None:
                 raise ValueError
@@ -130,7 +131,7 @@ class HAttentionFunction(torch.autograd.Function):
             dq, dk, dv, db, dg, dl = _hg.chunkwise_bwd(
                 q=q, k=k, v=v, b=b, g=g, l=l, Aw=Aw, Au=Au, do=do, head_first=ctx.head_first,
                 level_base=ctx.level_base, htype=ctx.htype, chunk_size=ctx.chunk_sizes[0],
-                qk_l2norm_scale=ctx.scale, fwd_ws=ctx.fwd_ws)
+                qk_l2norm_scale=ctx.scale, fwd_ws=kept)
         else:
             raise NotImplementedError
         return (dq.to(q), dk.to(k), dv.to(v), db.to(b) if b is not None else None,

@@ -234,13 +234,13 @@ class HMambaScanFunction(torch.autograd.Function):
                 htype):
         Cc, Bc = C.contiguous(), B.contiguous()
         ctx.cfg = (dt_softplus, lambda_mode, level_base, htype)
-        y, gcum, v, lam, ctx.fwd_ws = _scan_forward(x, dt, A, Bc, Cc, dl, L, D, dt_bias, *ctx.cfg)
-        ctx.save_for_backward(x, dt, A, Bc, Cc, dl, L, D, dt_bias, v, gcum, lam)
+        y, gcum, v, lam, ws = _scan_forward(x, dt, A, Bc, Cc, dl, L, D, dt_bias, *ctx.cfg)
+        ctx.save_for_backward(x, dt, A, Bc, Cc, dl, L, D, dt_bias, v, gcum, lam, ws)
         return y
 
     @staticmethod
     def backward(ctx, dy):
-        return _scan_backward(dy, *ctx.saved_tensors, ctx.fwd_ws, ctx.cfg) + (None,) * 4
+        return _scan_backward(dy, *ctx.saved_tensors, ctx.cfg) + (None,) * 4
 
 
 # --------------------------------------------------------------------------
@@ -338,12 +338,12 @@ class HMambaSplitFunction(torch.autograd.Function):
         dt = zx[..., c_dt:c_dt + H].contiguous()
         dl = zx[..., c_dt + H:].reshape(B_, S, H, Lv).contiguous()
         ctx.cfg = (True, lambda_mode, level_base, htype)
-        y, gcum, v, lam, ctx.fwd_ws = _scan_forward(x, dt, A, Bm, Cm, dl, L, D, dt_bias, *ctx.cfg)
+        y, gcum, v, lam, ws = _scan_forward(x, dt, A, Bm, Cm, dl, L, D, dt_bias, *ctx.cfg)
         y = y.reshape(B_, S, dim)
         w = rms_w.contiguous()
         out, rstd = gated_rmsnorm_forward(y, zx, 0, w, eps)
         ctx.save_for_backward(zx, wt, bs, y, w, rstd, x, dt, A, Bm, Cm, dl, L, D, dt_bias, v, gcum,
-                              lam)
+                              lam, ws)
         ctx.conv_shape = conv_w.shape
         return out
 
@@ -356,7 +356,7 @@ class HMambaSplitFunction(torch.autograd.Function):
         dzx = torch.empty_like(zx)
         dy, drms = gated_rmsnorm_backward(dout.contiguous(), y, zx, 0, w, rstd, dzx)
         dx, ddt, dA, dB, dC, ddl, dL, dD, dbias = _scan_backward(
-            dy.view(B_, S, H, P), x, dt, *scan, ctx.fwd_ws, ctx.cfg)
+            dy.view(B_, S, H, P), x, dt, *scan, ctx.cfg)
         dw, db = conv_silu_backward([g.contiguous() for g in (dx, dB, dC)], zx, dim, dim, dim + gn,
                                     wt, bs, dzx)
         c_dt = 2 * dim + 2 * gn
