@@ -575,10 +575,16 @@ template <int KIND, int NV, int R, bool STRONG = false, int KMAX = 256>
 hipError_t launch_steps(HsArgs a, int B, int nblk, hipStream_t stream) {
   const int nw = (a.K + R - 1) / R;
   // (a power of two; four tokens at K > 128, where eight would leave one workgroup
-  // per CU)
+  // per CU; fewer where a workgroup's 64 KB would not hold them beside the static
+  // arrays: 64640 bytes at K = 256, NV = 4 are the most that occurs)
   a.batch = a.T == 1 ? 1 : a.K > 128 ? 4 : hattn::kHsBatch;
-  const size_t smem =
-      (size_t)(a.batch * (2 * nw * R + (nw + 1) * 64 * NV) + 2 * nw * 64 * NV) * sizeof(float);
+  constexpr size_t kStatic = sizeof(float) * hattn::kHsBatch *
+                             (kHsMaxLevels + 64 + (KIND == kHsLayer ? 64 : 0) + 4) + 256;
+  auto bytes = [&](int batch) {
+    return (size_t)(batch * (2 * nw * R + (nw + 1) * 64 * NV) + 2 * nw * 64 * NV) * sizeof(float);
+  };
+  while (a.batch > 1 && bytes(a.batch) + kStatic > 65536) a.batch /= 2;
+  const size_t smem = bytes(a.batch);
   hipLaunchKernelGGL((hattn::hstate_steps_kernel<KIND, NV, R, STRONG, KMAX>), dim3(B * a.H, nblk), dim3(64 * nw),
                      smem, stream, a);
   return hipGetLastError();

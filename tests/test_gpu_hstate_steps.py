@@ -40,7 +40,9 @@ def _reference(S, depth, q, k, v, g, l, beta, strong):
 CASES = [  # B, H, K, V, L, T
     (1, 1, 64, 16, 5, 16), (1, 2, 17, 48, 7, 64), (2, 3, 100, 32, 18, 9), (1, 1, 256, 16, 32, 5),
     (24, 16, 64, 64, 18, 3), (40, 16, 33, 128, 14, 2), (8, 16, 128, 128, 19, 3), (1, 1, 64, 16, 1, 1),
-    (1, 2, 64, 16, 3, 4), (1, 1, 16, 16, 10, 300), (16, 16, 192, 48, 11, 6)]
+    (1, 2, 64, 16, 3, 4), (1, 1, 16, 16, 10, 300), (16, 16, 192, 48, 11, 6),
+    # the widest lanes at the most rows, where the operands nearly fill the LDS
+    (4, 16, 256, 64, 11, 6), (4, 16, 225, 64, 11, 5)]
 
 
 @pytest.mark.parametrize("strong", [False, True])
