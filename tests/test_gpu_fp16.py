@@ -117,7 +117,7 @@ def test_gdn_forward_fp16_native(T, K, V, final_state):
             assert mx < GDN16_MAX and fro < GDN16_FRO, (h, mx, fro)
 
 
-@pytest.mark.parametrize("T,K,V", [(512, 128, 128), (1024, 64, 64)])
+@pytest.mark.parametrize("T,K,V", [(512, 128, 128), (1024, 64, 64), (640, 64, 192), (1024, 192, 384)])
 def test_gdn_backward_fp16_native(T, K, V):
     from hattention.base import HType
     from hattention.chunkwise_hgdn import chunkwise_bwd, chunkwise_fwd

@@ -82,6 +82,28 @@ def test_fp32_beta_lambda():
     _run(1, 512, 2, 128, 128, 10, seed=31, fp32_beta_lambda=True)
 
 
+@pytest.mark.parametrize("K,V", [(64, 192), (128, 384)])
+def test_groups_wide_v(K, V):
+    # one key / query head for all four, V outside {64, 128}
+    from hattention.chunkwise_hgdn import chunkwise_fwd_keep, chunkwise_bwd
+    from hattention.base import HType
+    B, T, H, L = 1, 640, 4, 11
+    q, k, v, beta, g, l = make_gdn_inputs(B, T, H, K, V, L, seed=V)
+    q, k = q[:, :, :1].contiguous(), k[:, :, :1].contiguous()
+    do = torch.randn(B, T, H, V, generator=torch.Generator().manual_seed(43)).bfloat16()
+    xs = [x.cuda() for x in (q, k, v, beta, g, l)]
+    print(f"[gdn_bwd] G=1 H={H} K={K} V={V}", flush=True)
+    gc, _, Aw, Au, _, ws = chunkwise_fwd_keep(*xs, False, 2, HType.WEAK, 64, False, keep_any_v=True)
+    grads = chunkwise_bwd(*xs[:4], gc, xs[5], Aw, Au, do.cuda(), False, 2, HType.WEAK, 64, fwd_ws=ws)
+    ins = [x.double().requires_grad_() for x in (q, k, v, beta, g, l)]
+    rep = [x.expand(-1, -1, H, -1) for x in ins[:2]]
+    refs = [D.autograd_bwd(D.chunked_fwd, *(x[:, :, h:h + 1].detach() for x in rep + ins[2:]),
+                           do[:, :, h:h + 1].double(), chunk_size=64) for h in range(H)]
+    for i, (name, a) in enumerate(zip(NAMES, grads)):
+        r = torch.cat([x[i] for x in refs], 2)
+        _check(name, a, r.sum(2, keepdim=True) if i < 2 else r, "all")
+
+
 def test_groups():
     # G < H: dq / dk of a group are the sums over its heads (chunkwise_hgdn.py:1208-1215)
     from hattention.chunkwise_hgdn import chunkwise_fwd, chunkwise_bwd

@@ -122,7 +122,8 @@ def test_strong_bwd_small(T):
     _bwd(2, T, 2, 128, 128, 7 + math.ceil(math.log2(T // 64)), seed=40 + T)
 
 
-@pytest.mark.parametrize("K,V", [(64, 64), (192, 128), (256, 64)])
+# (V outside {64, 128}: column groups of 128 and blocks of 32 of the level kernels)
+@pytest.mark.parametrize("K,V", [(64, 64), (192, 128), (256, 64), (128, 192), (64, 384)])
 def test_strong_bwd_head_dims(K, V):
     _bwd(1, 1024, 2, K, V, 11, seed=50 + K)
 
