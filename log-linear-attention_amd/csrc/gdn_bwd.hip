@@ -22,12 +22,14 @@
 //   1. prep recompute (gdn_fwd.hip, from g_cumsum): q_new, K_new, W_new, U;
 //   2. forward scan recompute: the state of every level that a chunk reads, at the
 //      chunk's start, bf16 (both skipped where the forward kept their results);
-//   3. gdn_dh_scan_kernel walks the chunks backwards and stores dh_{c+1} of every level:
+//   3. gdn_dh_scan_kernel walks the chunks backwards and stores, in 16 bits, dh_{c+1} of
+//      every level whose block goes on past the chunk (nr):
 //        dV_new = K_new dh_{c+1},
 //        dh_c = nr (exp(Gc_last) dh_{c+1} - W_new^T dV_new) + rd q_new^T (lambda_e o dO);
-//   4. gdn_bwd_level_kernel, one workgroup per chunk, sums the rest over the levels:
-//        dU = sum_e wr K_new dh_{c+1},
+//   4. one workgroup per chunk each, the sums over the levels: gdn_bwd_read_kernel
 //        dq_new = sum_e rd lambda_e o (dO h_c^T),   dlambda_e = rd rowdot(q_new, dO h_c^T),
+//      and gdn_bwd_level_kernel
+//        dU = sum_e wr K_new dh_{c+1},
 //        Z = sum_e nr h_c dh_{c+1}^T  [K x K],      d exp(Gc_last) = trace Z,
 //        dW_new = -K_new Z^T,   dK_new = U (sum_e wr dh_{c+1})^T - W_new Z.
 //      A level with bit e clear (wr) is in the first half of its block, whose chunks
@@ -113,42 +115,28 @@ __device__ __forceinline__ floatx4 ld4f(const T* p) {
     return floatx4{(float)x[0], (float)x[1], (float)x[2], (float)x[3]};
   }
 }
-// An fp32 fragment of a 16 x 32 MFMA operand from global rows of stride rs,
-// sc * the sum over NP partials pstride apart (element j of lane (lq, ln): row
-// r0 + ln, column c0 + 8 lq + j), in two halves: frg_load issues the loads
-// (raw values in registers), frg_done sums and scales, so the loads can be
-// issued a step before the fragment is used.
-template <int NP, typename T>
+// An fp32 fragment of a 16 x 32 MFMA operand from global rows of stride rs, scaled by sc
+// (element j of lane (lq, ln): row r0 + ln, column c0 + 8 lq + j), in two halves:
+// frg_load issues the loads (raw values in registers), frg_done scales, so the loads
+// can be issued a step before the fragment is used.
+template <typename T>
 struct FrgPf {
   using V4 = typename std::conditional<sizeof(T) == 4, floatx4, bf16x4>::type;
-  V4 a[NP], b[NP];
+  V4 a, b;
 };
-template <int NP, typename T>
-__device__ __forceinline__ void frg_load(FrgPf<NP, T>& f, const T* X, size_t rs, size_t pstride,
-                                         int r0, int c0) {
+template <typename T>
+__device__ __forceinline__ void frg_load(FrgPf<T>& f, const T* X, size_t rs, int r0, int c0) {
   const int lane = threadIdx.x & 63;
   const T* p = X + (size_t)(r0 + (lane & 15)) * rs + c0 + 8 * (lane >> 4);
-#pragma unroll
-  for (int pp = 0; pp < NP; ++pp) {
-    f.a[pp] = *(const typename FrgPf<NP, T>::V4*)(p + pp * pstride);
-    f.b[pp] = *(const typename FrgPf<NP, T>::V4*)(p + pp * pstride + 4);
-  }
+  f.a = *(const typename FrgPf<T>::V4*)p;
+  f.b = *(const typename FrgPf<T>::V4*)(p + 4);
 }
-template <int NP, typename T>
-__device__ __forceinline__ void frg_done(const FrgPf<NP, T>& f, float sc, float* out) {
-  floatx4 a = zero4(), b = zero4();
-#pragma unroll
-  for (int pp = 0; pp < NP; ++pp) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      a[j] += (float)f.a[pp][j];
-      b[j] += (float)f.b[pp][j];
-    }
-  }
+template <typename T>
+__device__ __forceinline__ void frg_done(const FrgPf<T>& f, float sc, float* out) {
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
-    out[j] = sc * a[j];
-    out[4 + j] = sc * b[j];
+    out[j] = sc * (float)f.a[j];
+    out[4 + j] = sc * (float)f.b[j];
   }
 }
 // bf16x3 products: both operands fp32 (three MFMAs), or fp32 x bf16 (two).
@@ -176,64 +164,50 @@ __device__ __forceinline__ floatx4 mma_fb(const float* a, bf16x8 b, floatx4 c) {
     return mfma16x16x32(A[0], b, c);
   }
 }
-// ST[t][c] = (scale ? scale[t] : 1) * sum over NP partials of X[t][c], 64 rows of N.
-// Two units per step with all their partial loads issued together.
-template <int N, int LS, int NP, typename T>
-__device__ __forceinline__ void stage_rows(float* ST, const T* X, size_t rs, size_t pstride,
-                                           const float* scale) {
+// ST[t][c] = (scale ? scale[t] : 1) * X[t][c], 64 rows of N.  Two units per step with
+// their loads issued together.
+template <int N, int LS, typename T>
+__device__ __forceinline__ void stage_rows(float* ST, const T* X, size_t rs, const float* scale) {
   constexpr int IT = kGC * N / 4 / 256;
   static_assert(IT % 2 == 0, "units per thread");
 #pragma unroll 1
   for (int i0 = 0; i0 < IT; i0 += 2) {
-    floatx4 pv[2][NP];
+    floatx4 pv[2];
 #pragma unroll
     for (int d = 0; d < 2; ++d) {
       const int u = threadIdx.x + 256 * (i0 + d);
-      const int t = u / (N / 4), c = 4 * (u % (N / 4));
-#pragma unroll
-      for (int pp = 0; pp < NP; ++pp) pv[d][pp] = ld4f(X + (size_t)t * rs + c + pp * pstride);
+      pv[d] = ld4f(X + (size_t)(u / (N / 4)) * rs + 4 * (u % (N / 4)));
     }
 #pragma unroll
     for (int d = 0; d < 2; ++d) {
       const int u = threadIdx.x + 256 * (i0 + d);
       const int t = u / (N / 4), c = 4 * (u % (N / 4));
-      floatx4 a = pv[d][0];
-#pragma unroll
-      for (int pp = 1; pp < NP; ++pp) a += pv[d][pp];
+      floatx4 a = pv[d];
       if (scale) a *= scale[t];
       *(floatx4*)(ST + t * LS + c) = a;
     }
   }
 }
 
-// stage_rows of 64 bf16 partial rows of 64 columns in two halves: rows_load
-// issues every load of the block (4 units per thread, NP partials each) into
-// registers, rows_store sums, scales and writes them to ST later, so the loads
-// of a block fly while an earlier step computes.
-template <int NP>
+// stage_rows of 64 bf16 rows of 64 columns in two halves: rows_load issues every load of
+// the block (4 units per thread) into registers, rows_store scales and writes them to ST
+// later, so the loads of a block fly while an earlier step computes.
 struct RowsPf {
-  bf16x4 x[4][NP];
+  bf16x4 x[4];
 };
-template <int NP>
-__device__ __forceinline__ void rows_load(RowsPf<NP>& pf, const __bf16* X, size_t rs,
-                                          size_t pstride) {
+__device__ __forceinline__ void rows_load(RowsPf& pf, const __bf16* X, size_t rs) {
 #pragma unroll
   for (int d = 0; d < 4; ++d) {
     const int u = threadIdx.x + 256 * d, t = u >> 4, c = 4 * (u & 15);
-#pragma unroll
-    for (int pp = 0; pp < NP; ++pp) pf.x[d][pp] = *(const bf16x4*)(X + (size_t)t * rs + c + pp * pstride);
+    pf.x[d] = *(const bf16x4*)(X + (size_t)t * rs + c);
   }
 }
-template <int LS, int NP>
-__device__ __forceinline__ void rows_store(float* ST, const RowsPf<NP>& pf, const float* scale) {
+template <int LS>
+__device__ __forceinline__ void rows_store(float* ST, const RowsPf& pf, const float* scale) {
 #pragma unroll
   for (int d = 0; d < 4; ++d) {
     const int u = threadIdx.x + 256 * d, t = u >> 4, c = 4 * (u & 15);
-    floatx4 a = zero4();
-#pragma unroll
-    for (int pp = 0; pp < NP; ++pp)
-      a += floatx4{(float)pf.x[d][pp][0], (float)pf.x[d][pp][1], (float)pf.x[d][pp][2],
-                   (float)pf.x[d][pp][3]};
+    floatx4 a = {(float)pf.x[d][0], (float)pf.x[d][1], (float)pf.x[d][2], (float)pf.x[d][3]};
     if (scale) a *= scale[t];
     *(floatx4*)(ST + t * LS + c) = a;
   }
@@ -407,10 +381,10 @@ __global__ __launch_bounds__(256, 1) void gdn_bwd_chunk_kernel(
   }
   __syncthreads();
 
-  // step 5's fragments of X = e o dq_new (partials) are loaded while step 4 computes
-  FrgPf<1, __bf16> pfx[KD / 32];
+  // step 5's fragments of X = e o dq_new are loaded while step 4 computes
+  FrgPf<__bf16> pfx[KD / 32];
 #pragma unroll
-  for (int c = 0; c < KD / 32; ++c) frg_load(pfx[c], dq_p + rowk, hk, 0, t16, 32 * c);
+  for (int c = 0; c < KD / 32; ++c) frg_load(pfx[c], dq_p + rowk, hk, t16, 32 * c);
 
   // ---- 4: Z = dO V^T; Z o P o Gamma -> S0, dP = Z o Gamma o Lambda o beta_s -> S4 -----
   {
@@ -515,14 +489,14 @@ __global__ __launch_bounds__(256, 1) void gdn_bwd_chunk_kernel(
   }
   __syncthreads();
 
-  // step 7's fragments of e o dW_new (partials) and dU are loaded while step 6 computes
-  FrgPf<1, __bf16> pfw[KD / 32];
+  // step 7's fragments of e o dW_new and dU are loaded while step 6 computes
+  FrgPf<__bf16> pfw[KD / 32];
   constexpr int NFU = VD ? VD / 32 : 1;
-  FrgPf<1, float> pfu[NFU];
+  FrgPf<float> pfu[NFU];
 #pragma unroll
-  for (int c = 0; c < KD / 32; ++c) frg_load(pfw[c], dw_p + rowk, hk, 0, t16, 32 * c);
+  for (int c = 0; c < KD / 32; ++c) frg_load(pfw[c], dw_p + rowk, hk, t16, 32 * c);
 #pragma unroll
-  for (int c = 0; c < NFU; ++c) frg_load(pfu[c], du + rowv, hv, 0, t16, 32 * c);
+  for (int c = 0; c < NFU; ++c) frg_load(pfu[c], du + rowv, hv, t16, 32 * c);
 
   // ---- 6: H = (F1 beta) Aw^T, D = E Aw^T; dGc_t -= rowsum(M o H); dM = tril(D) -> S0 --
   {
@@ -578,7 +552,7 @@ __global__ __launch_bounds__(256, 1) void gdn_bwd_chunk_kernel(
       for (int c = 0; c < NFU; ++c) frg_done(pfu[c], 1.f, a3[c]);
       if (c0 + NFU < VN / 32)
 #pragma unroll
-        for (int c = 0; c < NFU; ++c) frg_load(pfu[c], du + rowv, hv, 0, t16, 32 * (c0 + NFU + c));
+        for (int c = 0; c < NFU; ++c) frg_load(pfu[c], du + rowv, hv, t16, 32 * (c0 + NFU + c));
 #pragma unroll
       for (int nt = 0; nt < 4; ++nt)
 #pragma unroll
@@ -631,10 +605,10 @@ __global__ __launch_bounds__(256, 1) void gdn_bwd_chunk_kernel(
   }
   __syncthreads();
 
-  // the kb loop's first partial block (X) is loaded while steps 9 compute
-  constexpr bool PF = KD <= 128;   // partial blocks prefetched into registers
-  RowsPf<1> pf;
-  if constexpr (PF) rows_load<1>(pf, dq_p + rowk, hk, 0);
+  // the kb loop's first block of 64 columns (X) is loaded while steps 9 compute
+  constexpr bool PF = KD <= 128;   // the blocks prefetched into registers
+  RowsPf pf;
+  if constexpr (PF) rows_load(pf, dq_p + rowk, hk);
 
   // ---- 9: Y = dAw Aw^T -> S1; dA = -strict-tril(Aw^T Y) -> S1 --------------------------
   {
@@ -705,12 +679,12 @@ __global__ __launch_bounds__(256, 1) void gdn_bwd_chunk_kernel(
       }
     }
     // ---- 10: X -> ST; dQ = X + dM K; U2 = -P^T X; dGc += rowdot(X, Q) ----------------
-    // (PF: each block's partial loads are issued one step before it is staged)
+    // (PF: each block's loads are issued one step before it is staged)
     if constexpr (PF) {
-      rows_store<LS, 1>(ST, pf, s.e);
-      rows_load<1>(pf, dw_p + rowk + k0, hk, 0);
+      rows_store<LS>(ST, pf, s.e);
+      rows_load(pf, dw_p + rowk + k0, hk);
     } else {
-      stage_rows<64, LS, 1>(ST, dq_p + rowk + k0, hk, 0, s.e);
+      stage_rows<64, LS>(ST, dq_p + rowk + k0, hk, s.e);
     }
     __syncthreads();
     floatx4 u2[4];
@@ -740,10 +714,10 @@ __global__ __launch_bounds__(256, 1) void gdn_bwd_chunk_kernel(
 
     // ---- 11: e o dW_new -> ST; U2 += Aw^T ST ---------------------------------------------
     if constexpr (PF) {
-      rows_store<LS, 1>(ST, pf, s.e);
-      rows_load<1>(pf, dk_p + rowk + k0, hk, 0);
+      rows_store<LS>(ST, pf, s.e);
+      rows_load(pf, dk_p + rowk + k0, hk);
     } else {
-      stage_rows<64, LS, 1>(ST, dw_p + rowk + k0, hk, 0, s.e);
+      stage_rows<64, LS>(ST, dw_p + rowk + k0, hk, s.e);
     }
     __syncthreads();
 #pragma unroll
@@ -781,10 +755,10 @@ __global__ __launch_bounds__(256, 1) void gdn_bwd_chunk_kernel(
 
     // ---- 13: dK_new -> ST; dK = U1 + beta o U2 + r o dK_new; dbeta, dGc of K_new -------
     if constexpr (PF) {
-      rows_store<LS, 1>(ST, pf, nullptr);
-      if (kb + 1 < KD / 64) rows_load<1>(pf, dq_p + rowk + k0 + 64, hk, 0);
+      rows_store<LS>(ST, pf, nullptr);
+      if (kb + 1 < KD / 64) rows_load(pf, dq_p + rowk + k0 + 64, hk);
     } else {
-      stage_rows<64, LS, 1>(ST, dk_p + rowk + k0, hk, 0, nullptr);
+      stage_rows<64, LS>(ST, dk_p + rowk + k0, hk, nullptr);
     }
     __syncthreads();
 #pragma unroll
@@ -843,7 +817,7 @@ __global__ __launch_bounds__(256, 1) void gdn_bwd_chunk_kernel(
     float rbv[4] = {0.f, 0.f, 0.f, 0.f};
     for (int vb = 0; vb < VN / 64; ++vb) {
       const int v0 = 64 * vb;
-      stage_rows<64, LS, 1>(ST, du + rowv + v0, hv, 0, nullptr);
+      stage_rows<64, LS>(ST, du + rowv + v0, hv, nullptr);
       g2s_tile<64>(dO + rowv + v0, hv, SD, LDB);
       __syncthreads();
 #pragma unroll

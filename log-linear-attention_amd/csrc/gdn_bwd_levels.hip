@@ -129,7 +129,7 @@ __global__ __launch_bounds__(64 * NW) void gdn_dh_scan_kernel(
     const __bf16* Wt = s.kwq[buf][1];
     const __bf16* Qt = s.kwq[buf][2];
     if (live) {
-      // dh_{c+1} -> dhs[row][chunk][level]
+      // dh_{c+1} -> dhs[row][chunk][level], as fragments
       store_state_frags<KD, BV, E>(st, dhs + (((size_t)row * NT + ic) * nlev + e) * V * KD, v0);
     }
     // the next chunk's operands, into registers while this one is computed

@@ -976,9 +976,9 @@ hipError_t hattn_gdn_fwd_launch(const void* q, const void* k, const void* v, con
 }
 
 // Forward recompute for the backward: q_new, K_new (token-major and per-chunk
-// transposed), W_new, U from the chunk-local cumsum (prep kernel) and every
-// level's per-chunk starting state, bf16 [row][chunk][level][v][k] (scan
-// kernel, no output).
+// transposed), W_new, U from the chunk-local cumsum (prep kernel) and the states of
+// the levels set in each chunk's index at its start, as 16-bit fragments
+// (gdn_common.h; scan kernel, no output).
 hipError_t hattn_gdn_recompute_launch(const void* q, const void* k, const void* v,
                                       const void* beta, const float* gcum, const void* l,
                                       __bf16* qn, __bf16* kn, __bf16* knT, __bf16* wn, __bf16* un,
