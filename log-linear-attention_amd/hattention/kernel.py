@@ -262,8 +262,11 @@ def postprocess_prefill_hstate_(hstate, q, k, v, b, g, l, scale, head_first, lev
         raise ValueError("shape mismatch between the HState and q, k, v, g, l")
     if L < level_chunk:
         raise ValueError(f"{L} levels, the prefill needs at least {level_chunk}")
-    if hstruct != HStruct.MAMBA2 and b is None:
-        raise ValueError
+    if hstruct != HStruct.MAMBA2:
+        if b is None:
+            raise ValueError
+        if b.shape != (B, T, H):
+            raise ValueError("b must be [B, T, H]")
     k, v, g = k.contiguous(), v.contiguous(), g.float().contiguous()
     b = b.contiguous() if hstruct != HStruct.MAMBA2 else None
     counts, _ = _prefill_counts(T, L, level_base)

@@ -383,6 +383,8 @@ def hselective_state_update(
         raise ValueError
     if D is not None and D.shape != (nheads,):
         raise ValueError
+    if dt_bias is not None and dt_bias.shape != (nheads,):
+        raise ValueError
     for arg in (lambda_level_max, lambda_level_base, lambda_htype, lambda_hstruct,
                 lambda_level_fixed):
         if arg is None:
