@@ -157,9 +157,10 @@ def hattention_kernel(
     """kernel.py:338-374."""
     if chunk_sizes is None:
         chunk_sizes = (64, 64)
-    if not torch.is_grad_enabled():
+    if hstruct == HStruct.GDELTA and not torch.is_grad_enabled():
         # no backward can follow (the function itself sees only the inputs' requires_grad)
-        q, k, v, b, g, l = (x.detach() if x is not None else None for x in (q, k, v, b, g, l))
+        q, k, v, b, g, l = (x.detach() if x is not None and x.requires_grad else x
+                            for x in (q, k, v, b, g, l))
     return HAttentionFunction.apply(q, k, v, b, g, l, scale, head_first, level_base, htype,
                                     hstruct, chunk_sizes, chunkwise, use_qk_l2norm_in_kernel)
 
