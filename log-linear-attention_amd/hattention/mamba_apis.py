@@ -365,12 +365,8 @@ def hselective_state_update(
         raise NotImplementedError
     if z is not None:
         raise NotImplementedError
-    dims = [(x, 3), (dt, 2), (A, 1), (B, 3), (C, 3), (dl, 3), (L, 2)]
-    if any(t.dim() != n for t, n in dims):
-        raise ValueError
-    if D is not None and D.dim() != 1:
-        raise ValueError
-    if dt_bias is not None and dt_bias.dim() != 1:
+    # (the other operands' dimensions with their shapes below)
+    if x.dim() != 3 or B.dim() != 3 or L.dim() != 2:
         raise ValueError
     batch, nheads, headdim = x.shape
     _, ngroups, dstate = B.shape
