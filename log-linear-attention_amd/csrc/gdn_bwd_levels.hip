@@ -389,8 +389,11 @@ struct GdnLevelSmem {
 // 140 of 6030 us of a training step at B 4, T 8192, H 16, K = V = 128, 53 of 2150 at B 1,
 // T 4096, H 8, K 256, V 128; at K 192, V 384 other registers spill and it is 140 of 1690
 // us faster.)
-// (One kernel with the reads as well took 2.6 ms at B 4, T 8192, H 16, K = V = 128: 250
-// registers with spills, one workgroup per CU, two thirds of its cycles waiting.)
+// Bound by waits for its loads (three quarters of a wave's cycles) at two workgroups a CU:
+// 1525 us at B 4, T 8192, H 16, K = V = 128.  Its 256 registers do not hold everything:
+// 46 spill at K = 128, 67 at 192, 364 at 256, none at 64.
+// (One kernel with the reads as well took 2.6 ms there: one workgroup per CU, two thirds
+// of its cycles waiting.)
 template <int KD, typename E>
 __global__ __launch_bounds__(64 * GdnLevelSmem<KD>::NW, KD <= 128 ? 2 : 1) void gdn_bwd_level_kernel(
     const __bf16* __restrict__ wn, const __bf16* __restrict__ kn, const __bf16* __restrict__ un,

@@ -114,7 +114,7 @@ __device__ __forceinline__ float lane_before(float x) { return dpp_f32<0x138, 0x
 // (STRONG is an instance of its own: the two cascades in one kernel cost 70 spilled
 // registers.)  NV (elements per lane) sets the number of workgroups: the host takes
 // the widest that still fills the chip.  Measured: one GDELTA step of B 4, H 16, K =
-// V = 128, L 18 in 39 us (3.9 TB/s of the 4.8 that a copy reaches), 40 tokens at B
+// V = 128, L 18 in 41 us (3.7 TB/s of the 4.8 that a copy reaches), 40 tokens at B
 // 1, H 16, K = V = 64 / 128 in 64 / 160 us: there the cascade's shifts and the
 // barrier of u bound a token.
 template <int NV>

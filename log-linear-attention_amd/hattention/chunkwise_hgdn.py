@@ -34,9 +34,9 @@ from hattention.base import HType, get_num_levels, ceil_log
 CHUNK = 64
 VB = 128   # V columns that chunkwise_fwd_keep keeps a workspace for by itself
 # A backward over all of V at once holds the level states and their gradients of all its
-# columns: B 8, T 8192, H 16, K 256, V 512 would take 52 GB at a time, 13 GB in blocks of
+# columns: B 8, T 8192, H 16, K 256, V 512 would take 52 GB at a time, 16 GB in blocks of
 # 128 columns.  More than BWD_LIMIT bytes are taken in blocks (at K 192, V 384, T 16384, H 6,
-# 3.2 GB: 6.1 ms at once, 38.7 in blocks of 128).
+# 3.2 GB: 5.8 ms at once, 12.0 in blocks of 128).
 BWD_LIMIT = 4 << 30
 # What one training call may hold between its forward and backward where V is neither 64
 # nor 128 (KEPT_V, for which it always holds its workspace: 1.7 GB at B 4, T 8192, H 16,

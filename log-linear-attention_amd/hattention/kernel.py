@@ -81,8 +81,8 @@ class HAttentionFunction(torch.autograd.Function):
             from hattention import chunkwise_hgdn as _hg
             # q * scale / ||q|| and k / ||k|| are formed inside the kernels; the
             # forward's workspace (what the backward would recompute) is kept where a
-            # backward can follow: storing it took 1099 us instead of 898 without it at
-            # B 4, T 8192, H 16, K = V = 128, and 1636 instead of 1301 (1.1 GB instead of
+            # backward can follow: storing it takes 1097 us instead of 945 without it at
+            # B 4, T 8192, H 16, K = V = 128, and 1637 instead of 1304 (1.1 GB instead of
             # 0.2) at B 1, T 16384, H 6, K 192, V 384
             g, o, Aw, Au, _, kept = _hg.chunkwise_fwd_keep(
                 q=q, k=k, v=v, b=b, g=g, l=l, head_first=head_first, level_base=level_base,

@@ -1,7 +1,9 @@
 """HMambaSplitFunction (the split-conv layer as one autograd node) against the chain of
 its parts, CausalConv1dSilu -> HMambaScanFunction -> GatedRMSNorm: the same bits in the
 output and in every gradient, for parameters in bf16 and fp32, grouped B / C, and where
-the folded scan does not apply (fp32 activations, headdim 128 without its summaries)."""
+the folded scan does not apply (fp32 activations, headdim 128 without its summaries).
+What both sides share, the kernels and the scan's forward and backward, is compared with
+the oracle in test_gpu_mamba_layer.py."""
 import pytest
 import torch
 
