@@ -241,25 +241,12 @@ def test_mamba2_backward_fp16_takes_fp16_kernels():
     assert call(H16) == _lib.HATTN_ERR_NOT_IMPLEMENTED
 
 
-@pytest.mark.parametrize("T,K,V", [(1024, 64, 64), (1024, 128, 128), (512, 192, 384), (512, 256, 64)])
-def test_gdn_backward_fp16_scaled_gradients(T, K, V):
-    """A loss scaled by 2^n scales the gradients by 2^n, up to where the gradients
-    themselves leave fp16: products of the states and their gradients over all of V, and
-    sums of the gradients over levels, may be far above 65504.  Values that share a sign
-    (v = 16 + noise, keys and dO with a mean) make these sums as large as they get.
-    Tolerance: the scale only moves roundings at the subnormal end, fewer than the two
-    of 2^-11 that an operand and a stored sum have, 1e-3."""
+def _scaled_gradients(q, k, v, b, g, l, do, exponents):
+    """Gradients of dO 2^n against 2^n times those of dO, where the gradients stay in
+    fp16.  Tolerance: the scale only moves roundings at the subnormal end, fewer than the
+    two of 2^-11 that an operand and a stored sum have, 1e-3."""
     from hattention.base import HType
     from hattention.chunkwise_hgdn import chunkwise_bwd, chunkwise_fwd
-    print(f"[gdn fp16 scaled] T={T} K={K} V={V}", flush=True)
-    H, L = 2, 7 + math.ceil(math.log2(T // 64))
-    gen = torch.Generator().manual_seed(T + V)
-    rn = lambda *s: torch.randn(*s, generator=gen)
-    q, k = ((0.5 + rn(1, T, H, K)).to(HALF) for _ in range(2))
-    v = (16 + 0.1 * rn(1, T, H, V)).to(HALF)
-    b, l = torch.sigmoid(rn(1, T, H)), torch.nn.functional.softplus(rn(1, T, H, L))
-    g = -0.002 * torch.rand(1, T, H, generator=gen)
-    do = ((1 + 0.1 * rn(1, T, H, V)) / 16).to(HALF)
     xs = [x.cuda() for x in (q, k, v, b, g, l)]
     gc, _, Aw, Au, _ = chunkwise_fwd(*xs, False, 2, HType.WEAK, 64, False, qk_l2norm_scale=1.0)
 
@@ -269,10 +256,46 @@ def test_gdn_backward_fp16_scaled_gradients(T, K, V):
         return dict(zip(("dq", "dk", "dv", "db", "dg", "dl"), r))
 
     ref = grads(0)
-    for n in (4, 6, 8, 10, 12):
+    for n in exponents:
         for name, x in grads(n).items():
             want = ref[name].double() * 2.0 ** n
             if x.dtype == HALF and want.abs().max() > 65000:
                 continue
             err = ((x.double() - want).norm() / want.norm()).item()
             assert err < 1e-3, (n, name, err)
+
+
+@pytest.mark.parametrize("T,K,V", [(1024, 64, 64), (1024, 128, 128), (512, 192, 384), (512, 256, 64)])
+def test_gdn_backward_fp16_scaled_gradients(T, K, V):
+    """A loss scaled by 2^n scales the gradients by 2^n, up to where the gradients
+    themselves leave fp16: products of the states and their gradients over all of V may be
+    far above 65504.  Values that share a sign (v = 16 + noise, keys and dO with a mean)
+    make these sums as large as they get."""
+    print(f"[gdn fp16 scaled] T={T} K={K} V={V}", flush=True)
+    H, L = 2, 7 + math.ceil(math.log2(T // 64))
+    gen = torch.Generator().manual_seed(T + V)
+    rn = lambda *s: torch.randn(*s, generator=gen)
+    q, k = ((0.5 + rn(1, T, H, K)).to(HALF) for _ in range(2))
+    v = (16 + 0.1 * rn(1, T, H, V)).to(HALF)
+    b, l = torch.sigmoid(rn(1, T, H)), torch.nn.functional.softplus(rn(1, T, H, L))
+    g = -0.002 * torch.rand(1, T, H, generator=gen)
+    do = ((1 + 0.1 * rn(1, T, H, V)) / 16).to(HALF)
+    _scaled_gradients(q, k, v, b, g, l, do, (4, 6, 8, 10, 12))
+
+
+@pytest.mark.parametrize("T,K", [(2048, 128), (4096, 192), (2048, 256)])
+def test_gdn_backward_fp16_sums_over_levels(T, K):
+    """State gradients in fp16's range whose sums over the levels are not: queries with a
+    mean and keys without, hardly any decay, and level weights of 2^-e, which make every
+    level's gradient as large as the others'.  At 2^17 the sums overflow, at 2^15 not."""
+    print(f"[gdn fp16 level sums] T={T} K={K}", flush=True)
+    H, V, L = 1, 64, 7 + math.ceil(math.log2(T // 64))
+    gen = torch.Generator().manual_seed(T + V)
+    rn = lambda *s: torch.randn(*s, generator=gen)
+    q, k = (0.5 + rn(1, T, H, K)).to(HALF), rn(1, T, H, K).to(HALF)
+    v = (16 + 0.1 * rn(1, T, H, V)).to(HALF)
+    b, l = 0.001 * torch.sigmoid(rn(1, T, H)), torch.nn.functional.softplus(rn(1, T, H, L))
+    l[..., 7:] *= 2.0 ** -torch.arange(L - 7)
+    g = -0.0002 * torch.rand(1, T, H, generator=gen)
+    do = ((1 + 0.1 * rn(1, T, H, V)) / 16).to(HALF)
+    _scaled_gradients(q, k, v, b, g, l, do, (15, 17))

@@ -11,6 +11,7 @@ a relative Frobenius error < 1e-2 (dg: 5e-2, see TOL_FRO_DG).  At the full
 BASELINE size every (batch, head) row is independent, so the oracle runs on a
 few rows at the full length.
 """
+import gc
 import math
 
 import pytest
@@ -291,6 +292,7 @@ def test_backward_in_blocks_of_columns(G, K, V, cols, monkeypatch):
     for limit in (hg.BWD_LIMIT, query(B, T, H, K, cols, L)):
         monkeypatch.setattr(hg, "BWD_LIMIT", limit)
         leaves = [x.clone().requires_grad_() for x in xs]
+        gc.collect()
         base = torch.cuda.memory_allocated()
         o = hattention_kernel(*leaves, 0.125, False, 2, HType.WEAK, HStruct.GDELTA,
                               use_qk_l2norm_in_kernel=True)

@@ -1,6 +1,8 @@
 """The forward workspace that a training call holds for its backward is one of the node's
 saved tensors: saved-tensor hooks (offloading, for instance) see it, and it goes when the
 backward has run, also while the output is still referred to."""
+import gc
+
 import pytest
 import torch
 
@@ -46,6 +48,7 @@ def _call(kind):
 def test_workspace_is_a_saved_tensor(kind):
     print(f"[saved workspace] {kind}", flush=True)
     fn, xs = _call(kind)
+    gc.collect()             # (nothing of earlier calls goes while memory is counted)
     torch.cuda.synchronize()
 
     def step(hooks):
